@@ -38,9 +38,9 @@ int sdt_debug_spme_interp(sdt_mob_t mob, const double* mesh, double alpha, doubl
 /* Launch forms of a mobility's kernels, for tests and measurements:
  * interp_form, meshes per LDS pass of the interp kernel: 0 the built-in
  * choice (1), else 1, 2 or 4 (4: FP32 only; an error at apply time
- * otherwise); z_form, threads and pencils per workgroup of the z transform:
- * 0 the built-in choice (FP32 (512, 16), FP64 (512, 8)), 1 .. 5 =
- * (1024, 16), (1024, 16), (512, 16), (512, 8), (256, 8), (256, 4);
+ * otherwise); z_form, the most threads and pencils per workgroup of the z
+ * transform: 0 the built-in choice, 1 .. 5 = (256, 16), (128, 16), (256, 8),
+ * (128, 8), (256, 4);
  * spread_form: the point-owner spread's sums in wide launches (0 the
  * built-in choice: FP32 3 + 8, FP64 1 + 8; 1 forces staged in LDS, 2 forces
  * read by scalar loads (FP32), 3 forces staged in LDS and summed by the

@@ -18,6 +18,8 @@ ARCH = os.environ.get("SDT_OFFLOAD_ARCH", "gfx950")
 
 HIP_SOURCES = [
     ("spme_kernels.hip", []),
+    ("fft_f32.hip", []),
+    ("fft_f64.hip", []),
     ("sort_kernels.hip", []),
     # exact FP64 pair decisions: no contraction into fused multiply-adds
     ("pair_kernels.hip", ["-ffp-contract=off"]),

@@ -1,4 +1,6 @@
-// Device-side radix-2/3/4/5/8 Stockham FFT on pencils held in LDS.
+// Device-side FFT pieces: r-point DFTs in registers (2 .. 20 points) and a
+// general radix-2/3/4/5/8 Stockham chain on pencils held in LDS, for the mesh
+// sides without a two-stage kernel (fft_kernels.hpp).
 //
 // Self-sorting decimation-in-frequency form: a stage of radix r on a
 // sub-sequence length `len` with stride `s` (m = len / r) reads
@@ -43,7 +45,12 @@ __device__ __forceinline__ int lpad(int e) { return e + (e >> 4); }
 
 template <typename T>
 __device__ __forceinline__ cplx<T> cmul(cplx<T> a, cplx<T> b) {
-    return cplx<T>{a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x};
+    // fused explicitly: the same rounding in every kernel
+    return cplx<T>{fma(a.x, b.x, -(a.y * b.y)), fma(a.x, b.y, a.y * b.x)};
+}
+template <typename T>
+__device__ __forceinline__ cplx<T> cmulc(cplx<T> a, cplx<T> b) {   // a conj(b)
+    return cplx<T>{fma(a.x, b.x, a.y * b.y), fma(a.y, b.x, -(a.x * b.y))};
 }
 template <typename T>
 __device__ __forceinline__ cplx<T> cadd(cplx<T> a, cplx<T> b) {
@@ -57,6 +64,13 @@ __device__ __forceinline__ cplx<T> csub(cplx<T> a, cplx<T> b) {
 template <typename T, int SIGN>
 __device__ __forceinline__ cplx<T> rot90(cplx<T> a) {
     return SIGN < 0 ? cplx<T>{a.y, -a.x} : cplx<T>{-a.y, a.x};
+}
+
+// the multiple of b that is 1 modulo a (a, b coprime)
+constexpr int crt_unit(int a, int b) {
+    int e = b;
+    while (e % a != 1) e += b;
+    return e;
 }
 
 // r-point DFT in registers, kernel e^{SIGN * 2 pi i j t / r}
@@ -78,7 +92,7 @@ __device__ __forceinline__ void small_dft(cplx<T>* a) {
         const T s1 = T(SIGN) * T(0.86602540378443864676372317075294);
         cplx<T> t1 = cadd(a[1], a[2]);
         cplx<T> t2 = csub(a[1], a[2]);
-        cplx<T> m = cplx<T>{a[0].x + c1 * t1.x, a[0].y + c1 * t1.y};
+        cplx<T> m = cplx<T>{fma(c1, t1.x, a[0].x), fma(c1, t1.y, a[0].y)};
         cplx<T> j = cplx<T>{-s1 * t2.y, s1 * t2.x};
         a[0] = cadd(a[0], t1);
         a[1] = cadd(m, j);
@@ -115,20 +129,18 @@ __device__ __forceinline__ void small_dft(cplx<T>* a) {
         const T s1 = T(0.38268343236508977172845998403040);   // sin(pi/8)
         const T h = T(0.70710678118654752440084436210485);
         const T sg = T(SIGN);
-        // w_16^e = cos(2 pi e / 16) + SIGN i sin(2 pi e / 16), e = n2 k1
+        // v w_16^e, w_16^e = cos(2 pi e / 16) + SIGN i sin(2 pi e / 16), e = n2 k1
         auto tw16 = [&](cplx<T> v, int e) -> cplx<T> {
             T cr, ci;
             switch (e) {
                 case 1: cr = c1; ci = s1; break;
-                case 2: cr = h; ci = h; break;
+                case 2: return cplx<T>{h * (v.x - sg * v.y), h * (v.y + sg * v.x)};
                 case 3: cr = s1; ci = c1; break;
-                case 4: cr = T(0); ci = T(1); break;
-                case 6: cr = -h; ci = h; break;
-                case 9: cr = -c1; ci = -s1; break;
-                default: return v;
+                case 4: return rot90<T, SIGN>(v);
+                case 6: return cplx<T>{h * (-v.x - sg * v.y), h * (-v.y + sg * v.x)};
+                default: cr = -c1; ci = -s1; break;   // 9
             }
-            ci *= sg;
-            return cplx<T>{v.x * cr - v.y * ci, v.x * ci + v.y * cr};
+            return cmul(v, cplx<T>{cr, sg * ci});
         };
 #pragma unroll
         for (int n2 = 1; n2 < 4; n2++)
@@ -148,15 +160,68 @@ __device__ __forceinline__ void small_dft(cplx<T>* a) {
         const T s2 = T(SIGN) * T(0.58778525229247312916870595463907);  // sin(4pi/5)
         cplx<T> t1 = cadd(a[1], a[4]), t2 = cadd(a[2], a[3]);
         cplx<T> d1 = csub(a[1], a[4]), d2 = csub(a[2], a[3]);
-        cplx<T> m1 = cplx<T>{a[0].x + c1 * t1.x + c2 * t2.x, a[0].y + c1 * t1.y + c2 * t2.y};
-        cplx<T> m2 = cplx<T>{a[0].x + c2 * t1.x + c1 * t2.x, a[0].y + c2 * t1.y + c1 * t2.y};
-        cplx<T> n1 = cplx<T>{-(s1 * d1.y + s2 * d2.y), s1 * d1.x + s2 * d2.x};
-        cplx<T> n2 = cplx<T>{-(s2 * d1.y - s1 * d2.y), s2 * d1.x - s1 * d2.x};
+        cplx<T> m1 = cplx<T>{fma(c2, t2.x, fma(c1, t1.x, a[0].x)),
+                             fma(c2, t2.y, fma(c1, t1.y, a[0].y))};
+        cplx<T> m2 = cplx<T>{fma(c1, t2.x, fma(c2, t1.x, a[0].x)),
+                             fma(c1, t2.y, fma(c2, t1.y, a[0].y))};
+        cplx<T> n1 = cplx<T>{-fma(s2, d2.y, s1 * d1.y), fma(s2, d2.x, s1 * d1.x)};
+        cplx<T> n2 = cplx<T>{-fma(-s1, d2.y, s2 * d1.y), fma(-s1, d2.x, s2 * d1.x)};
         a[0] = cplx<T>{a[0].x + t1.x + t2.x, a[0].y + t1.y + t2.y};
         a[1] = cadd(m1, n1);
         a[4] = csub(m1, n1);
         a[2] = cadd(m2, n2);
         a[3] = csub(m2, n2);
+    } else if constexpr (R == 9) {
+        // n = 3 n1 + n2: 3-point DFTs over n1, twiddles w_9^(n2 k1), 3-point
+        // DFTs over n2; X[k1 + 3 k2]
+        const T sg = T(SIGN);
+        const cplx<T> w1{T(0.76604444311897803520239265055542), sg * T(0.64278760968653932632264340990726)};
+        const cplx<T> w2{T(0.17364817766693034885171662676931), sg * T(0.98480775301220805936674302458952)};
+        const cplx<T> w4{T(-0.93969262078590838405410927732473), sg * T(0.34202014332566873304409961468226)};
+        cplx<T> b[3][3];
+#pragma unroll
+        for (int n2 = 0; n2 < 3; n2++) {
+            b[n2][0] = a[n2]; b[n2][1] = a[3 + n2]; b[n2][2] = a[6 + n2];
+            small_dft<T, 3, SIGN>(b[n2]);
+        }
+        b[1][1] = cmul(b[1][1], w1);
+        b[1][2] = cmul(b[1][2], w2);
+        b[2][1] = cmul(b[2][1], w2);
+        b[2][2] = cmul(b[2][2], w4);
+#pragma unroll
+        for (int k1 = 0; k1 < 3; k1++) {
+            cplx<T> c[3] = {b[0][k1], b[1][k1], b[2][k1]};
+            small_dft<T, 3, SIGN>(c);
+#pragma unroll
+            for (int k2 = 0; k2 < 3; k2++) a[k1 + 3 * k2] = c[k2];
+        }
+    } else {
+        // R = A B with A, B coprime (6 = 3 2, 10 = 5 2, 12 = 4 3, 15 = 5 3,
+        // 18 = 9 2, 20 = 5 4): the prime-factor form, input n = (B n1 + A n2)
+        // mod R and output k with k = k1 (mod A), k = k2 (mod B), needs no
+        // twiddles between its A- and B-point DFTs (Good 1958)
+        constexpr int A = R == 6 ? 3 : (R == 12 ? 4 : (R == 18 ? 9 : 5)), B = R / A;
+        // E1 = 1 (mod A), 0 (mod B); E2 = 0 (mod A), 1 (mod B)
+        constexpr int E1 = crt_unit(A, B), E2 = crt_unit(B, A);
+        static_assert(R == 6 || R == 10 || R == 12 || R == 15 || R == 18 || R == 20, "radix");
+        cplx<T> b[B][A];
+#pragma unroll
+        for (int n2 = 0; n2 < B; n2++) {
+#pragma unroll
+            for (int n1 = 0; n1 < A; n1++) b[n2][n1] = a[(B * n1 + A * n2) % R];
+            small_dft<T, A, SIGN>(b[n2]);
+        }
+#pragma unroll
+        for (int k1 = 0; k1 < A; k1++) {
+            cplx<T> c[B];
+#pragma unroll
+            for (int n2 = 0; n2 < B; n2++) c[n2] = b[n2][k1];
+            small_dft<T, B, SIGN>(c);
+#pragma unroll
+            for (int k2 = 0; k2 < B; k2++) {
+                a[(k1 * E1 + k2 * E2) % R] = c[k2];
+            }
+        }
     }
 }
 
@@ -256,62 +321,7 @@ __device__ __forceinline__ void fft_pencils_inplace(cplx<T>* buf, int npen, int 
     }
 }
 
-// Two-stage in-place transform for K = R1 R2 (R1, R2 powers of two <= 16):
-// stage 1 (radix R1, stride 1): butterfly j < R2 reads elements j + R2 u,
-// applies w_K^(j u) and writes R1 j + u; stage 2 (radix R2, stride R1, no
-// twiddles): butterfly j < R1 reads and writes elements j + R1 u. Index
-// arithmetic is shifts and masks; stage 2 is in place per thread. Requires
-// npen * R2 <= MAXB * blockDim.x.
-template <typename T, int R1, int R2, int SIGN, int MAXB = 1>
-__device__ __forceinline__ void fft2_pencils(cplx<T>* buf, int npen, int PS,
-                                             const cplx<T>* __restrict__ tw) {
-    static_assert((R1 & (R1 - 1)) == 0 && (R2 & (R2 - 1)) == 0, "powers of two");
-    {
-        cplx<T> a[MAXB][R1];
-#pragma unroll
-        for (int v = 0; v < MAXB; v++) {
-            const int it = threadIdx.x + v * blockDim.x;
-            if (it < npen * R2) {
-                const int pen = it / R2, j = it % R2;
-                const cplx<T>* base = buf + pen * PS;
-#pragma unroll
-                for (int u = 0; u < R1; u++) a[v][u] = base[lpad(j + R2 * u)];
-                small_dft<T, R1, SIGN>(a[v]);
-#pragma unroll
-                for (int u = 1; u < R1; u++) {
-                    cplx<T> w = tw[j * u];
-                    if (SIGN > 0) w.y = -w.y;
-                    a[v][u] = cmul(a[v][u], w);
-                }
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int v = 0; v < MAXB; v++) {
-            const int it = threadIdx.x + v * blockDim.x;
-            if (it < npen * R2) {
-                const int pen = it / R2, j = it % R2;
-                cplx<T>* base = buf + pen * PS;
-#pragma unroll
-                for (int u = 0; u < R1; u++) base[lpad(R1 * j + u)] = a[v][u];
-            }
-        }
-        __syncthreads();
-    }
-    for (int it = threadIdx.x; it < npen * R1; it += blockDim.x) {
-        const int pen = it / R1, j = it % R1;
-        cplx<T>* base = buf + pen * PS;
-        cplx<T> a[R2];
-#pragma unroll
-        for (int u = 0; u < R2; u++) a[u] = base[lpad(j + R1 * u)];
-        small_dft<T, R2, SIGN>(a);
-#pragma unroll
-        for (int u = 0; u < R2; u++) base[lpad(j + R1 * u)] = a[u];
-    }
-    __syncthreads();
-}
-
-// Runs all stages; returns the buffer holding the result (a or b).// Runs all stages; returns the buffer holding the result (a or b).
+// Runs all stages; returns the buffer holding the result (a or b).
 template <typename T, int SIGN>
 __device__ __forceinline__ cplx<T>* fft_pencils(cplx<T>* a, cplx<T>* b, int npen, int PS, const FFTArgs& fa,
                                 const cplx<T>* tw) {

@@ -51,9 +51,8 @@ struct SpmeGpu {
     // interp meshes per LDS pass: 0 the built-in choice (1), else 1, 2 or
     // (FP32) 4
     int interp_form = 0;
-    // z transform launch shape: 0 the built-in choice (FP32 2, FP64 3),
-    // 1 .. 5 (threads, pencils) = (1024, 16), (1024, 16), (512, 16),
-    // (512, 8), (256, 8), (256, 4)
+    // z transform launch shape: 0 the built-in choice, 1 .. 5 at most
+    // (threads, pencils) = (256, 16), (128, 16), (256, 8), (128, 8), (256, 4)
     int z_form = 0;
     // spread launch form: bits 0-1, force reads of wide FP32 launches (0
     // built-in = scalar loads, 1 staged in LDS, 2 scalar loads); bit 2, mesh
@@ -65,7 +64,7 @@ struct SpmeGpu {
     // replaces the launch choices of a width class (re-plans the FFT order)
     void set_tuning(const SpmeTuning& t, int width);
     DevBuf<double> d_tw;   // K roots of unity (cos, sin) of -2*pi*j/K
-    DevBuf<double> d_bsp2; // |b(m)|^2 per wavenumber index, K entries
+    DevBuf<double> d_fac;  // influence factor per wavenumber index, K entries
     DevBuf<double> d_frac; // 3N fractional offsets (sorted order)
     DevBuf<int> d_base;    // 3N B-spline base mesh indices (sorted order)
     DevBuf<double> d_a2;   // N radii squared (sorted order), poly only

@@ -14,6 +14,7 @@
 #include <map>
 #include <mutex>
 #include "fft_lds.hpp"
+#include "spme_fft.hpp"
 #include "real_gpu.hpp"
 #include "spme_gpu.hpp"
 
@@ -1055,213 +1056,27 @@ fft_y_kernel(FFTArgs fa, cplx<T>* __restrict__ spec, const double* __restrict__ 
     }
 }
 
-// K = R1 R2 (both powers of two): the two-stage transform; otherwise the
-// planned radix-8/4/2/3/5 stages
-template <typename T, int SIGN, int MAXI2, int R1, int R2>
-__device__ __forceinline__ void fft_any(cplx<T>* buf, int npen, int PS, const FFTArgs& fa,
-                                        const cplx<T>* tw) {
-    if constexpr (R1 > 0) fft2_pencils<T, R1, R2, SIGN, (R2 >= 16 ? 2 : 1)>(buf, npen, PS, tw);
-    else fft_pencils_inplace<T, SIGN, MAXI2>(buf, npen, PS, fa, tw);
-}
-
-// Mesh side and divisions by K and K/2+1: compile-time when the two-stage
-// transform fixes K = R1 R2, magic reciprocals otherwise
-template <int R1, int R2>
-struct KDiv {
-    static constexpr int KC = R1 * R2;
-    int K, Kh;
-    unsigned K_m, Kh_m;
-    __device__ __forceinline__ explicit KDiv(const FFTArgs& fa) {
-        if constexpr (KC > 0) {
-            K = KC;
-            Kh = KC / 2 + 1;
-        } else {
-            K = fa.K;
-            Kh = fa.K / 2 + 1;
-        }
-        K_m = fa.K_m;
-        Kh_m = fa.Kh_m;
-    }
-    __device__ __forceinline__ int div_k(int i) const {
-        if constexpr (KC > 0) return (int)((unsigned)i / (unsigned)KC);
-        else return (int)fdiv((unsigned)i, K_m);
-    }
-    __device__ __forceinline__ int div_kh(int i) const {
-        if constexpr (KC > 0) return (int)((unsigned)i / (unsigned)(KC / 2 + 1));
-        else return (int)fdiv((unsigned)i, Kh_m);
-    }
-};
-
-// ------------------------------------------------ fused x + y plane -------
-// One workgroup per z-plane of one mesh: the K x K real plane is read once,
-// transformed along x (two real rows per complex FFT) and along y in LDS
-// (in place, padded pencils), and the K x (K/2+1) half-spectrum plane is
-// written once. The inverse kernel mirrors it. Used when one plane fits LDS.
-// Register bounds are template parameters: MAXI2 radix-2 butterflies and
-// MAXP pack/unpack items per thread (K <= 128: 5 and 8; K <= 180: 8 and 16).
-constexpr int kPlaneThreads = 1024;
-
-template <typename T, int MAXI2, int MAXP, int R1, int R2>
-__global__ void __launch_bounds__(kPlaneThreads)
-fft_plane_fwd_kernel(FFTArgs fa, const T* __restrict__ real, cplx<T>* __restrict__ spec,
-                     const double* __restrict__ tw_g) {
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    const KDiv<R1, R2> kd(fa);
-    const int K = kd.K, Kh = kd.Kh, PS = pencil_stride(K), H = K / 2;
-    cplx<T>* tw = reinterpret_cast<cplx<T>*>(smem_raw);
-    cplx<T>* buf = tw + K;
-    load_twiddles(tw, tw_g, K);
-    const size_t plane = blockIdx.x;
-    const T* src = real + plane * K * K;
-    // row pairs (2j, 2j+1) -> pencil j; the loads of a thread (8 at a time)
-    // are in flight together
-    for (int i0 = threadIdx.x; i0 < H * K; i0 += 8 * kPlaneThreads) {
-        cplx<T> v[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const int i = min(i0 + u * kPlaneThreads, H * K - 1);
-            const int j = kd.div_k(i), x = i - j * K;
-            v[u] = cplx<T>{src[(size_t)(2 * j) * K + x], src[(size_t)(2 * j + 1) * K + x]};
-        }
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const int i = i0 + u * kPlaneThreads;
-            const int j = kd.div_k(i), x = i - j * K;
-            if (i < H * K) buf[j * PS + lpad(x)] = v[u];
-        }
-    }
-    __syncthreads();
-    fft_any<T, -1, MAXI2, R1, R2>(buf, H, PS, fa, tw);
-    // unpack Z_j = A + i B into the half spectra of rows 2j and 2j+1, stored
-    // as y-pencils (pencil kx, element y)
-    {
-        cplx<T> va[MAXP], vb[MAXP];
-        const int nit = H * Kh;
-#pragma unroll
-        for (int u = 0; u < MAXP; u++) {
-            const int i = threadIdx.x + u * blockDim.x;
-            if (i < nit) {
-                const int j = kd.div_kh(i), k = i - j * Kh;
-                const cplx<T> zk = buf[j * PS + lpad(k)];
-                const cplx<T> zm = buf[j * PS + lpad(k == 0 ? 0 : K - k)];
-                const T h = T(0.5);
-                va[u] = cplx<T>{h * (zk.x + zm.x), h * (zk.y - zm.y)};
-                vb[u] = cplx<T>{h * (zk.y + zm.y), h * (zm.x - zk.x)};
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < MAXP; u++) {
-            const int i = threadIdx.x + u * blockDim.x;
-            if (i < nit) {
-                const int j = kd.div_kh(i), k = i - j * Kh;
-                buf[k * PS + lpad(2 * j)] = va[u];
-                buf[k * PS + lpad(2 * j + 1)] = vb[u];
-            }
-        }
-        __syncthreads();
-    }
-    fft_any<T, -1, MAXI2, R1, R2>(buf, Kh, PS, fa, tw);
-    cplx<T>* dst = spec + plane * K * Kh;
-    for (int i = threadIdx.x; i < K * Kh; i += blockDim.x) {
-        const int y = kd.div_kh(i), kx = i - y * Kh;
-        dst[i] = buf[kx * PS + lpad(y)];
-    }
-}
-
-template <typename T, int MAXI2, int MAXP, int R1, int R2>
-__global__ void __launch_bounds__(kPlaneThreads)
-fft_plane_inv_kernel(FFTArgs fa, const cplx<T>* __restrict__ spec, T* __restrict__ real,
-                     const double* __restrict__ tw_g) {
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    const KDiv<R1, R2> kd(fa);
-    const int K = kd.K, Kh = kd.Kh, PS = pencil_stride(K), H = K / 2;
-    cplx<T>* tw = reinterpret_cast<cplx<T>*>(smem_raw);
-    cplx<T>* buf = tw + K;
-    load_twiddles(tw, tw_g, K);
-    const size_t plane = blockIdx.x;
-    const cplx<T>* src = spec + plane * K * Kh;
-    // the loads of a thread (8 at a time) are in flight together
-    for (int i0 = threadIdx.x; i0 < K * Kh; i0 += 8 * kPlaneThreads) {
-        cplx<T> v[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) v[u] = src[min(i0 + u * kPlaneThreads, K * Kh - 1)];
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const int i = i0 + u * kPlaneThreads;
-            const int y = kd.div_kh(i), kx = i - y * Kh;
-            if (i < K * Kh) buf[kx * PS + lpad(y)] = v[u];
-        }
-    }
-    __syncthreads();
-    fft_any<T, +1, MAXI2, R1, R2>(buf, Kh, PS, fa, tw);
-    // pack the half spectra of rows 2j, 2j+1 into Z_j = A + i B (full x):
-    // the pair A, B at kx = kk gives Z_j[kk] and Z_j[K - kk]
-    {
-        cplx<T> vz[MAXP], vw[MAXP];
-        const int nit = H * Kh;
-#pragma unroll
-        for (int u = 0; u < MAXP; u++) {
-            const int i = threadIdx.x + u * blockDim.x;
-            if (i < nit) {
-                const int j = kd.div_kh(i), kk = i - j * Kh;
-                cplx<T> A = buf[kk * PS + lpad(2 * j)];
-                cplx<T> B = buf[kk * PS + lpad(2 * j + 1)];
-                if (kk == 0 || 2 * kk == K) { A.y = T(0); B.y = T(0); }
-                vz[u] = cplx<T>{A.x - B.y, A.y + B.x};
-                vw[u] = cplx<T>{A.x + B.y, B.x - A.y};
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < MAXP; u++) {
-            const int i = threadIdx.x + u * blockDim.x;
-            if (i < nit) {
-                const int j = kd.div_kh(i), kk = i - j * Kh;
-                buf[j * PS + lpad(kk)] = vz[u];
-                if (kk > 0 && 2 * kk < K) buf[j * PS + lpad(K - kk)] = vw[u];
-            }
-        }
-        __syncthreads();
-    }
-    fft_any<T, +1, MAXI2, R1, R2>(buf, H, PS, fa, tw);
-    T* dst = real + plane * K * K;
-    for (int i = threadIdx.x; i < H * K; i += blockDim.x) {
-        const int j = kd.div_k(i), x = i - j * K;
-        const cplx<T> v = buf[j * PS + lpad(x)];
-        dst[(size_t)(2 * j) * K + x] = v.x;
-        dst[(size_t)(2 * j + 1) * K + x] = v.y;
-    }
-}
-
 // ------------------------------------------ z transform + influence -------
-// A workgroup takes NP = 2^lnp consecutive (y, kx) positions of the flat
-// K x (K/2+1) half-plane index j = y (K/2+1) + kx (contiguous in memory, so
-// every z-plane read is one NP-element run) for one right-hand side: forward
-// z-FFT of all components in place, the RPY influence tensor
-// (src/mob/spme.cc:201-310, spme.h:114-123), inverse z-FFT, store.
-// Mono (NC = 3): B = lm2 (1 - k^2/3)(I - k k^T / k^2) applied to the
-// 3-vector. Poly (NC = 6, spreads of f and a^2 f): the reference's three
-// mesh round trips (flags 1, 2, 2) reduce to two outputs
-//   U = G (F f - k^2/6 F[a^2 f]),  W = -k^2/6 G F f,  G = lm2 (I - k k^T / k^2)
-// interpolated as interp(U) + a_i^2 interp(W).
+// The mesh sides without a two-stage kernel (250 and those above 324): the
+// same work as fft_kernels.hpp's fft2_z_influence_kernel with the general
+// radix chain, in place in LDS.
 constexpr int kZMaxI2 = 8;
+constexpr int kZThreads = 512;
 
-template <typename T, int R1, int R2, int NT>
-__global__ void __launch_bounds__(NT)
+template <typename T, int NC>
+__global__ void __launch_bounds__(kZThreads)
 fft_z_influence_kernel(FFTArgs fa, cplx<T>* __restrict__ spec, const double* __restrict__ tw_g,
-                       const double* __restrict__ bsp2, int lnp, int NC, double box, double xi) {
+                       const double* __restrict__ fac_g, int lnp, double box, double xi) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    const KDiv<R1, R2> kd(fa);
-    const int K = kd.K, Kh = kd.Kh, PS = pencil_stride(K);
+    const int K = fa.K, Kh = K / 2 + 1, PS = pencil_stride(K);
     const int NP = 1 << lnp;
     const int nj = K * Kh;
     cplx<T>* tw = reinterpret_cast<cplx<T>*>(smem_raw);
     cplx<T>* buf = tw + K;
     load_twiddles(tw, tw_g, K);
-    // |b|^2 factors in arithmetic T, after the spectrum buffer
-    T* s_b2 = reinterpret_cast<T*>(buf + (size_t)NC * NP * PS);
-    for (int i = threadIdx.x; i < K; i += blockDim.x) s_b2[i] = (T)bsp2[i];
+    // influence factors in arithmetic T, after the spectrum buffer
+    T* s_fac = reinterpret_cast<T*>(buf + (size_t)NC * NP * PS);
+    for (int i = threadIdx.x; i < K; i += blockDim.x) s_fac[i] = (T)fac_g[i];
     const int nch = (nj + NP - 1) >> lnp;
     const int j0 = (int)(blockIdx.x % nch) * NP;
     const int rhs = (int)(blockIdx.x / nch);
@@ -1270,95 +1085,50 @@ fft_z_influence_kernel(FFTArgs fa, cplx<T>* __restrict__ spec, const double* __r
     const int nvalid = min(NP, nj - j0);
     // the loads of a thread (ZB at a time) are in flight together
     constexpr int ZB = 8;
-    for (int i0 = threadIdx.x; i0 < NC * NP * K; i0 += ZB * NT) {
+    for (int i0 = threadIdx.x; i0 < NC * NP * K; i0 += ZB * kZThreads) {
         cplx<T> v[ZB];
 #pragma unroll
         for (int u = 0; u < ZB; u++) {
-            const int i = i0 + u * NT;
+            const int i = i0 + u * kZThreads;
             const int jl = i & (NP - 1);
             const int cz = i >> lnp;
-            const int c = kd.div_k(cz), z = cz - c * K;
+            const int c = (int)fdiv(cz, fa.K_m), z = cz - c * K;
             v[u] = (i < NC * NP * K && jl < nvalid) ? base[c * mesh_sz + (size_t)z * nj + jl]
                                                     : cplx<T>{T(0), T(0)};
         }
 #pragma unroll
         for (int u = 0; u < ZB; u++) {
-            const int i = i0 + u * NT;
+            const int i = i0 + u * kZThreads;
             const int jl = i & (NP - 1);
             const int cz = i >> lnp;
-            const int c = kd.div_k(cz), z = cz - c * K;
+            const int c = (int)fdiv(cz, fa.K_m), z = cz - c * K;
             if (i < NC * NP * K) buf[(c * NP + jl) * PS + lpad(z)] = v[u];
         }
     }
     __syncthreads();
-    fft_any<T, -1, kZMaxI2, R1, R2>(buf, NC * NP, PS, fa, tw);
-    // influence
-    const T twopi_l = (T)(2.0 * M_PI / box);
-    const T inv_xi2 = (T)(1.0 / (xi * xi));
+    fft_pencils_inplace<T, -1, kZMaxI2>(buf, NC * NP, PS, fa, tw);
+    const Influence<T> inf(box, xi);
     const int cs = NP * PS;    // component stride in LDS
     for (int i = threadIdx.x; i < NP * K; i += blockDim.x) {
-        const int jl = kd.div_k(i), z = i - jl * K;
+        const int jl = (int)fdiv(i, fa.K_m), z = i - jl * K;
         if (jl >= nvalid) continue;
         const int j = j0 + jl;
-        const int y = kd.div_kh(j), kxi = j - y * Kh;
-        const int my = (y <= K / 2) ? y : y - K;
-        const int mz = (z <= K / 2) ? z : z - K;
-        const T kx = twopi_l * (T)kxi;
-        const T ky = twopi_l * (T)my;
-        const T kz = twopi_l * (T)mz;
-        const T kk = kx * kx + ky * ky + kz * kz;
-        T m2 = T(0), ex = T(0), ey = T(0), ez = T(0);
-        if (kk > T(0)) {
-            const T kx2 = kk * inv_xi2;
-            m2 = T(6.0 * M_PI) * exp(-kx2 * T(0.25)) / kk *
-                 (T(1) + kx2 * (T(0.25) + kx2 * T(0.125)));
-            m2 *= s_b2[kxi] * s_b2[y] * s_b2[z];
-            const T rk = T(1) / sqrt(kk);
-            ex = kx * rk; ey = ky * rk; ez = kz * rk;
-        }
-        const int o = jl * PS + lpad(z);
-        if (NC == 3) {
-            const T s = m2 * (T(1) - kk / T(3));
-            cplx<T> g0 = buf[o], g1 = buf[cs + o], g2 = buf[2 * cs + o];
-            // (I - e e^T) g, scaled
-            const T dr = ex * g0.x + ey * g1.x + ez * g2.x;
-            const T di = ex * g0.y + ey * g1.y + ez * g2.y;
-            buf[o] = cplx<T>{s * (g0.x - ex * dr), s * (g0.y - ex * di)};
-            buf[cs + o] = cplx<T>{s * (g1.x - ey * dr), s * (g1.y - ey * di)};
-            buf[2 * cs + o] = cplx<T>{s * (g2.x - ez * dr), s * (g2.y - ez * di)};
-        } else {
-            const T q = -kk / T(6);
-            cplx<T> f[3], a[3];
+        const int y = (int)fdiv(j, fa.Kh_m), kxi = j - y * Kh;
+        cplx<T>* o = buf + jl * PS + lpad(z);
+        cplx<T> g[NC];
 #pragma unroll
-            for (int c = 0; c < 3; c++) {
-                f[c] = buf[c * cs + o];
-                a[c] = buf[(3 + c) * cs + o];
-            }
-            cplx<T> u[3], w[3];
+        for (int c = 0; c < NC; c++) g[c] = o[c * cs];
+        inf.template apply<NC>(kxi, y <= K / 2 ? y : y - K, z <= K / 2 ? z : z - K,
+                               s_fac[kxi] * s_fac[y] * s_fac[z], g);
 #pragma unroll
-            for (int c = 0; c < 3; c++) {
-                u[c] = cplx<T>{f[c].x + q * a[c].x, f[c].y + q * a[c].y};
-                w[c] = cplx<T>{q * f[c].x, q * f[c].y};
-            }
-            const T ur = ex * u[0].x + ey * u[1].x + ez * u[2].x;
-            const T ui = ex * u[0].y + ey * u[1].y + ez * u[2].y;
-            const T wr = ex * w[0].x + ey * w[1].x + ez * w[2].x;
-            const T wi = ex * w[0].y + ey * w[1].y + ez * w[2].y;
-            const T e3[3] = {ex, ey, ez};
-#pragma unroll
-            for (int c = 0; c < 3; c++) {
-                buf[c * cs + o] = cplx<T>{m2 * (u[c].x - e3[c] * ur), m2 * (u[c].y - e3[c] * ui)};
-                buf[(3 + c) * cs + o] =
-                    cplx<T>{m2 * (w[c].x - e3[c] * wr), m2 * (w[c].y - e3[c] * wi)};
-            }
-        }
+        for (int c = 0; c < NC; c++) o[c * cs] = g[c];
     }
     __syncthreads();
-    fft_any<T, +1, kZMaxI2, R1, R2>(buf, NC * NP, PS, fa, tw);
+    fft_pencils_inplace<T, +1, kZMaxI2>(buf, NC * NP, PS, fa, tw);
     for (int i = threadIdx.x; i < NC * NP * K; i += blockDim.x) {
         const int jl = i & (NP - 1);
         const int cz = i >> lnp;
-        const int c = kd.div_k(cz), z = cz - c * K;
+        const int c = (int)fdiv(cz, fa.K_m), z = cz - c * K;
         if (jl < nvalid) base[c * mesh_sz + (size_t)z * nj + jl] = buf[(c * NP + jl) * PS + lpad(z)];
     }
 }
@@ -1651,8 +1421,13 @@ void SpmeGpu<T>::create(int npos_, double box_, double xi_, int K_, int porder_,
     SDT_HIP_CHECK(sync_memcpy(d_tw.get(), tw.data(), sizeof(double) * 2 * K, hipMemcpyHostToDevice));
     std::vector<double> bs;
     bspline_moduli(K, porder, bs);
-    d_bsp2.reserve(K);
-    SDT_HIP_CHECK(sync_memcpy(d_bsp2.get(), bs.data(), sizeof(double) * K, hipMemcpyHostToDevice));
+    // the influence factors |b(m)|^2 e^{-k_m^2 / 4 xi^2}, one per mesh index
+    for (int m = 0; m < K; m++) {
+        const double k = 2.0 * M_PI / box * (m <= K / 2 ? m : m - K);
+        bs[m] *= exp(-k * k / (4.0 * xi * xi));
+    }
+    d_fac.reserve(K);
+    SDT_HIP_CHECK(sync_memcpy(d_fac.get(), bs.data(), sizeof(double) * K, hipMemcpyHostToDevice));
     d_frac.reserve(3 * (size_t)npos);
     d_base.reserve(3 * (size_t)npos);
     d_frac_u.reserve(3 * (size_t)npos);
@@ -1858,28 +1633,8 @@ static size_t max_lds_bytes() {
     return v;
 }
 
-template <typename T>
-static size_t plane_lds_bytes(int K) {
-    return (K + (size_t)(K / 2 + 1) * pencil_stride(K)) * sizeof(cplx<T>);
-}
-
-// the fused x + y plane kernels apply when one half-spectrum plane fits the
-// LDS of a workgroup and the per-thread butterfly / pack bounds hold:
-// 0 = not applicable, 1 = the K <= 128 variant, 2 = the K <= 180 variant
-template <typename T>
-static int plane_path(int K) {
-    if (plane_lds_bytes<T>(K) > max_lds_bytes()) return 0;
-    const int Kh = K / 2 + 1, H = K / 2, nt = kPlaneThreads;
-    if (Kh * K <= 2 * 5 * nt && H * K <= 8 * nt && H * Kh <= 8 * nt) return 1;
-    if (sizeof(T) == 4 && Kh * K <= 2 * 8 * nt && H * K <= 16 * nt && H * Kh <= 16 * nt) return 2;
-    return 0;
-}
-
-template <typename T>
-static void allow_lds(const void* fn, size_t bytes) {
+void allow_lds(const void* fn, size_t bytes) {
     if (bytes <= 64 * 1024) return;
-    // raised once per kernel and size: later launches (and graph captures of
-    // them) make no attribute call
     static std::mutex mu;
     static std::map<const void*, size_t> raised;
     std::lock_guard<std::mutex> lk(mu);
@@ -1891,33 +1646,18 @@ static void allow_lds(const void* fn, size_t bytes) {
 
 template <typename T>
 void SpmeGpu<T>::fft_forward(int b, hipStream_t s) {
+    typedef Fft2Launch<T> F2;
+    if (fft_form != 1 && F2::plane_fits(K)) {
+        F2::plane(K, true, nmesh(b), d_real.get(), d_spec.get(), d_tw.get(), s);
+        return;
+    }
+    if (F2::has_xy(K)) {
+        F2::xy(K, true, nmesh(b), d_real.get(), d_spec.get(), d_tw.get(), s);
+        return;
+    }
     const FFTArgs fa = fft_args(plans[width_class(b)]);
     const int Kh = K / 2 + 1;
     const long long nrows = (long long)nmesh(b) * K * K;
-    if (const int pv = fft_form == 1 ? 0 : plane_path<T>(K)) {
-        const size_t lds = plane_lds_bytes<T>(K);
-        const dim3 grid((unsigned)(nmesh(b) * K));
-        if (sizeof(T) == 4 && K == 128) {
-            // two-stage 16 x 8 transforms (FP32: 16 complex registers)
-            allow_lds<T>((const void*)fft_plane_fwd_kernel<T, 5, 8, 16, 8>, lds);
-            hipLaunchKernelGGL((fft_plane_fwd_kernel<T, 5, 8, 16, 8>), grid, dim3(kPlaneThreads), lds, s,
-                               fa, d_real.get(), d_spec.get(), d_tw.get());
-        } else if (K == 64) {
-            allow_lds<T>((const void*)fft_plane_fwd_kernel<T, 5, 8, 8, 8>, lds);
-            hipLaunchKernelGGL((fft_plane_fwd_kernel<T, 5, 8, 8, 8>), grid, dim3(kPlaneThreads), lds, s,
-                               fa, d_real.get(), d_spec.get(), d_tw.get());
-        } else if (pv == 1) {
-            allow_lds<T>((const void*)fft_plane_fwd_kernel<T, 5, 8, 0, 0>, lds);
-            hipLaunchKernelGGL((fft_plane_fwd_kernel<T, 5, 8, 0, 0>), grid, dim3(kPlaneThreads), lds, s,
-                               fa, d_real.get(), d_spec.get(), d_tw.get());
-        } else if constexpr (sizeof(T) == 4) {
-            allow_lds<T>((const void*)fft_plane_fwd_kernel<T, 8, 16, 0, 0>, lds);
-            hipLaunchKernelGGL((fft_plane_fwd_kernel<T, 8, 16, 0, 0>), grid, dim3(kPlaneThreads), lds, s,
-                               fa, d_real.get(), d_spec.get(), d_tw.get());
-        }
-        SDT_HIP_CHECK(hipGetLastError());
-        return;
-    }
     const int NR = 2 << pick_lnp<T>(K, 1, 48 * 1024);
     hipLaunchKernelGGL((fft_x_r2c_kernel<T>), dim3(ceil_div(nrows, NR)), dim3(256),
                        fft_lds_bytes<T>(K, NR / 2), s, fa, nrows, d_real.get(), d_spec.get(),
@@ -1932,81 +1672,58 @@ void SpmeGpu<T>::fft_forward(int b, hipStream_t s) {
 
 template <typename T>
 void SpmeGpu<T>::influence(int b, hipStream_t s) {
+    const int NC = poly ? 6 : 3;
+    // at most this many threads and 2^lnp pencils per component in a
+    // workgroup; z_form > 0 picks smaller ones
+    static const int forms[][2] = {{512, 4}, {256, 4}, {128, 4}, {256, 3}, {128, 3}, {256, 2}};
+    SDT_REQUIRE(z_form >= 0 && z_form <= 5, SDT_EINVAL, "z transform: form must be in [0, 5]");
+    const int zf = z_form;
+    if (Fft2Launch<T>::has(K)) {
+        Fft2Launch<T>::z(K, NC, b, d_spec.get(), d_tw.get(), d_fac.get(), forms[zf][0],
+                         forms[zf][1], box, xi, s);
+        return;
+    }
     const FFTArgs fa = fft_args(plans[width_class(b)]);
     const int Kh = K / 2 + 1;
-    const int NC = poly ? 6 : 3;
     const int nj = K * Kh;
-    // threads per workgroup and at most 2^lnp pencils per component, one
-    // padded buffer of NC * 2^lnp pencils within ~110 KB and the butterfly
-    // bounds; z_form > 0 picks (threads, largest lnp) explicitly. Built-in
-    // (measured at K = 128, 100 columns): FP32 512 threads x 16 pencils,
-    // FP64 512 x 8 (three workgroups per CU instead of one)
-    static const int forms[][2] = {{1024, 4}, {1024, 4}, {512, 4}, {512, 3}, {256, 3}, {256, 2}};
-    SDT_REQUIRE(z_form >= 0 && z_form <= 5, SDT_EINVAL, "z transform: form must be in [0, 5]");
-    const int zf = z_form > 0 ? z_form : (sizeof(T) == 4 ? 2 : 3);
-    const int nt = forms[zf][0];
     int lnp = forms[zf][1];
     const size_t budget = std::min<size_t>(max_lds_bytes(), 112 * 1024);
     auto lds_of = [&](int l) {
         return (K + (size_t)NC * ((size_t)1 << l) * pencil_stride(K)) * sizeof(cplx<T>) +
                (size_t)K * sizeof(T);
     };
-    while (lnp > 0 && (lds_of(lnp) > budget || NC * (K << lnp) > 2 * kZMaxI2 * nt)) lnp--;
-    SDT_REQUIRE(lds_of(lnp) <= max_lds_bytes() && NC * K <= 2 * kZMaxI2 * nt, SDT_EINVAL,
+    while (lnp > 0 && (lds_of(lnp) > budget || NC * (K << lnp) > 2 * kZMaxI2 * kZThreads)) lnp--;
+    SDT_REQUIRE(lds_of(lnp) <= max_lds_bytes() && NC * K <= 2 * kZMaxI2 * kZThreads, SDT_EINVAL,
                 "z transform: mesh dimension too large");
     const size_t lds = lds_of(lnp);
     const unsigned nch = ceil_div(nj, (size_t)1 << lnp);
     const dim3 grid(nch * (unsigned)b);
-#define SDT_Z_LAUNCH(R1, R2, NT)                                                              \
-    do {                                                                                      \
-        allow_lds<T>((const void*)fft_z_influence_kernel<T, R1, R2, NT>, lds);                \
-        hipLaunchKernelGGL((fft_z_influence_kernel<T, R1, R2, NT>), grid, dim3(NT), lds, s, fa, \
-                           d_spec.get(), d_tw.get(), d_bsp2.get(), lnp, NC, box, xi);         \
-    } while (0)
-#define SDT_Z_SHAPES(NT)                                                                      \
-    do {                                                                                      \
-        /* two-stage transforms need one stage-1 butterfly per thread */                      \
-        if (sizeof(T) == 4 && K == 128 && (NC << lnp) * 8 <= NT) SDT_Z_LAUNCH(16, 8, NT);     \
-        else if (K == 64 && (NC << lnp) * 8 <= NT) SDT_Z_LAUNCH(8, 8, NT);                    \
-        else SDT_Z_LAUNCH(0, 0, NT);                                                          \
-    } while (0)
-    if (nt == 1024) SDT_Z_SHAPES(1024);
-    else if (nt == 512) SDT_Z_SHAPES(512);
-    else SDT_Z_SHAPES(256);
-#undef SDT_Z_SHAPES
-#undef SDT_Z_LAUNCH
+    if (poly) {
+        allow_lds((const void*)fft_z_influence_kernel<T, 6>, lds);
+        hipLaunchKernelGGL((fft_z_influence_kernel<T, 6>), grid, dim3(kZThreads), lds, s, fa,
+                           d_spec.get(), d_tw.get(), d_fac.get(), lnp, box, xi);
+    } else {
+        allow_lds((const void*)fft_z_influence_kernel<T, 3>, lds);
+        hipLaunchKernelGGL((fft_z_influence_kernel<T, 3>), grid, dim3(kZThreads), lds, s, fa,
+                           d_spec.get(), d_tw.get(), d_fac.get(), lnp, box, xi);
+    }
     SDT_HIP_CHECK(hipGetLastError());
 }
 
 template <typename T>
 void SpmeGpu<T>::fft_backward(int b, hipStream_t s) {
+    typedef Fft2Launch<T> F2;
+    if (fft_form != 1 && F2::plane_fits(K)) {
+        F2::plane(K, false, nmesh(b), d_real.get(), d_spec.get(), d_tw.get(), s);
+        return;
+    }
+    if (F2::has_xy(K)) {
+        F2::xy(K, false, nmesh(b), d_real.get(), d_spec.get(), d_tw.get(), s);
+        return;
+    }
     const FFTArgs fa = fft_args(plans[width_class(b)]);
     const int Kh = K / 2 + 1;
     const long long nrows = (long long)nmesh(b) * K * K;
-    if (const int pv = fft_form == 1 ? 0 : plane_path<T>(K)) {
-        const size_t lds = plane_lds_bytes<T>(K);
-        const dim3 grid((unsigned)(nmesh(b) * K));
-        if (sizeof(T) == 4 && K == 128) {
-            // two-stage 16 x 8 transforms (FP32: 16 complex registers)
-            allow_lds<T>((const void*)fft_plane_inv_kernel<T, 5, 8, 16, 8>, lds);
-            hipLaunchKernelGGL((fft_plane_inv_kernel<T, 5, 8, 16, 8>), grid, dim3(kPlaneThreads), lds, s,
-                               fa, d_spec.get(), d_real.get(), d_tw.get());
-        } else if (K == 64) {
-            allow_lds<T>((const void*)fft_plane_inv_kernel<T, 5, 8, 8, 8>, lds);
-            hipLaunchKernelGGL((fft_plane_inv_kernel<T, 5, 8, 8, 8>), grid, dim3(kPlaneThreads), lds, s,
-                               fa, d_spec.get(), d_real.get(), d_tw.get());
-        } else if (pv == 1) {
-            allow_lds<T>((const void*)fft_plane_inv_kernel<T, 5, 8, 0, 0>, lds);
-            hipLaunchKernelGGL((fft_plane_inv_kernel<T, 5, 8, 0, 0>), grid, dim3(kPlaneThreads), lds, s,
-                               fa, d_spec.get(), d_real.get(), d_tw.get());
-        } else if constexpr (sizeof(T) == 4) {
-            allow_lds<T>((const void*)fft_plane_inv_kernel<T, 8, 16, 0, 0>, lds);
-            hipLaunchKernelGGL((fft_plane_inv_kernel<T, 8, 16, 0, 0>), grid, dim3(kPlaneThreads), lds, s,
-                               fa, d_spec.get(), d_real.get(), d_tw.get());
-        }
-        SDT_HIP_CHECK(hipGetLastError());
-        return;
-    }
     const int lnp = pick_lnp<T>(K, 1, 48 * 1024);
     hipLaunchKernelGGL((fft_y_kernel<T, +1>), dim3(ceil_div(Kh, 1 << lnp) * nmesh(b) * K),
                        dim3(256), fft_lds_bytes<T>(K, 1 << lnp), s, fa, d_spec.get(), d_tw.get(),
@@ -2068,7 +1785,7 @@ void SpmeGpu<T>::interp(int b, double alpha, double beta, double* Y, hipStream_t
     else if constexpr (sizeof(T) == 4) SDT_INTERP_M(PP, 16, 4);
 #define SDT_INTERP_M(PP, RR, MM)                                                              \
     do {                                                                                      \
-    allow_lds<T>((const void*)interp_tile_kernel<T, PP, RR, MM>, lds);                            \
+    allow_lds((const void*)interp_tile_kernel<T, PP, RR, MM>, lds);                            \
     hipLaunchKernelGGL((interp_tile_kernel<T, PP, RR, MM>), grid, dim3(256), lds, s, K, ts, ntile, \
                        nsx, sxt, ch, d_tile_start.get(), d_frac.get(), d_base.get(),              \
                        poly ? d_a2.get() : (double*)nullptr, d_real.get(), b, RB, NC, a_eff, beta, \

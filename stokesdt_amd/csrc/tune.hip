@@ -6,6 +6,7 @@
 #include <fstream>
 #include <sstream>
 #include "block_gpu.hpp"
+#include "spme_fft.hpp"
 #include "tune.hpp"
 
 namespace sdt {
@@ -92,7 +93,8 @@ TuneResult autotune_spme(MobSpmeGpu* mob, int b, const std::string& cache_path) 
         };
         FFTPlan p0;
         make_fft_plan(mob->K(), &p0, 0);
-        for (int order = 1; order <= 2; order++) {
+        // the two-stage transforms have one stage order
+        for (int order = 1; order <= 2 && !Fft2Launch<float>::has(mob->K()); order++) {
             FFTPlan p;
             if (!make_fft_plan(mob->K(), &p, order)) continue;
             bool same = p.nst == p0.nst;
