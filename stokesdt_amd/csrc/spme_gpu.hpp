@@ -88,7 +88,6 @@ struct SpmeGpu {
                hipStream_t s, T* xb = nullptr, bool fill_xb = false);
     // columns per block of the copy the spread can read for b (0: none)
     int blocked_cols(int b) const;
-    bool point_owner() const;
 
     // stages (exposed for tests/benchmarks)
     void spread(int b, const double* X, hipStream_t s, const T* xb = nullptr);
@@ -99,6 +98,7 @@ struct SpmeGpu {
     int nmesh(int b) const { return (poly ? 6 : 3) * b; }
     StageTimer* timer = nullptr;
 
+    DevBuf<T> d_xs;        // the spread's own blocked copy of its input
     // scratch from prepare()
     DevBuf<double> d_frac_u;
     DevBuf<int> d_base_u;

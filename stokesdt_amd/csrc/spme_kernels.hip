@@ -93,14 +93,6 @@ __global__ void spme_gather_kernel(int npos, const int* __restrict__ perm,
 }
 
 // ------------------------------------------------------------- spread ------
-// Gather form: each workgroup owns a super-tile of 4 ts x ts x ts mesh tiles
-// along x (one per wave) for RB right-hand sides. Lane l of a wave owns the
-// x-row (y = l % ts, z = l / ts) of its tile and accumulates its ts points
-// in registers. The particles whose B-spline stencils reach the super-tile
-// (base points in the 4+1 x 2 x 2 surrounding tiles, filtered by overlap) are
-// staged in LDS with their weights and forces; every lane then walks the
-// staged list. No atomics: every mesh point is written once, by its owner.
-
 // exclusive prefix over the workgroup of a 0/1 predicate; returns this
 // thread's slot and the total (all threads must call)
 __device__ __forceinline__ int wg_compact(bool pred, int* s_wave, int* total) {
@@ -126,213 +118,15 @@ __device__ __forceinline__ int wrapk(int d, int K) {
     return d - ((d >= K) ? K : 0);
 }
 
-template <typename T, int P, int RBNC>
-__global__ void __launch_bounds__(256)
-spread_gather_kernel(int K, int ts, int ntile, int nsx, const int* __restrict__ tile_start,
-                     const double* __restrict__ frac, const int* __restrict__ base,
-                     const double* __restrict__ a2, const double* __restrict__ X, int b, int RB,
-                     int NC, int cap, T* __restrict__ mesh) {
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    // record: x weights in a zero-padded window wxp[0 .. P+13] (wxp[7 + k] =
-    // wx[k]), wy[P], wz[P], bx, by, bz, f[RBNC]. A wave reads the weight of
-    // its tile point x at wxp[7 - sd + x], sd = base - tile start in
-    // [-(P-1), ts-1]: no per-point selects or range tests.
-    constexpr int OWY = P + 14, OWZ = 2 * P + 14, OB = 3 * P + 14, OF = 3 * P + 17;
-    constexpr int REC = OF + RBNC;
-    T* stage = reinterpret_cast<T*>(smem_raw);
-    __shared__ int s_wave[4];
-    __shared__ int s_off[21];                   // candidate offsets of the base tiles
-    __shared__ int s_beg[20];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    // block -> (super-tile x, tile y, tile z), rhs chunk; XCD-contiguous
-    const unsigned lid = xcd_logical_id(blockIdx.x + blockIdx.y * gridDim.x, gridDim.x * gridDim.y);
-    const int bxl = (int)(lid % gridDim.x), byl = (int)(lid / gridDim.x);
-    const int sxi = bxl % nsx;
-    const int tyz = bxl / nsx;
-    const int ty = tyz % ntile, tz = tyz / ntile;
-    const int r0 = byl * RB;
-    const int rb = min(RB, b - r0);
-    const int rbnc = rb * NC;
-    const int stx = sxi * 4;                    // first x tile of the super-tile
-    const int nxt = min(4, ntile - stx);        // x tiles present
-    const int sx0 = stx * ts, sxlen = nxt * ts;
-    const int sy0 = ty * ts, sz0 = tz * ts;
-    // this lane's row and x range
-    const int wx0 = sx0 + wave * ts;
-    const bool wave_on = wave < nxt;
-    const bool lane_on = wave_on && lane < ts * ts;
-    const int yl = sy0 + (lane % ts), zl = sz0 + (lane / ts);
-    T acc[8][RBNC];
-#pragma unroll
-    for (int x = 0; x < 8; x++)
-#pragma unroll
-        for (int q = 0; q < RBNC; q++) acc[x][q] = T(0);
-
-    // contributor base tiles: x tiles stx-1 .. stx+nxt-1, y ty-1..ty, z tz-1..tz
-    const int nbx = min(nxt + 1, ntile);
-    const int nbt = 4 * nbx;
-    if (threadIdx.x == 0) {
-        int off = 0;
-        for (int k = 0; k < nbt; k++) {
-            const int jx = k % nbx, jy = (k / nbx) & 1, jz = k / (2 * nbx);
-            const int btz = (tz - 1 + jz + ntile) % ntile;
-            const int bty = (ty - 1 + jy + ntile) % ntile;
-            const int btx = (stx - 1 + jx + ntile) % ntile;
-            const int bt = (btz * ntile + bty) * ntile + btx;
-            const int pb = tile_start[bt], pe = tile_start[bt + 1];
-            s_beg[k] = pb;
-            s_off[k] = off;
-            off += pe - pb;
-        }
-        s_off[nbt] = off;
-    }
-    __syncthreads();
-    const int ncand = s_off[nbt];
-
-    auto accumulate = [&](int n) __attribute__((always_inline)) {
-        if (!lane_on) return;
-        for (int sidx = 0; sidx < n; sidx++) {
-            const T* rec = stage + (size_t)sidx * REC;
-            const int bx = (int)rec[OB], by = (int)rec[OB + 1], bz = (int)rec[OB + 2];
-            const int dxw = wrapk(bx - wx0, K);
-            if (!(dxw < ts || K - dxw < P)) continue;          // wave-uniform
-            const int ly = wrapk(yl - by, K), lz = wrapk(zl - bz, K);
-            if (ly >= P || lz >= P) continue;
-            const int sd = dxw < ts ? dxw : dxw - K;
-            const T* wxp = rec + (7 - sd);
-            // every load of the candidate is issued before the first use;
-            // points x >= ts accumulate window zeros / unused values and are
-            // never stored
-            T f[RBNC], wx8[8];
-#pragma unroll
-            for (int q = 0; q < RBNC; q++) f[q] = rec[OF + q];
-#pragma unroll
-            for (int x = 0; x < 8; x++) wx8[x] = wxp[x];
-            const T wyz = rec[OWY + ly] * rec[OWZ + lz];
-#pragma unroll
-            for (int x = 0; x < 8; x++) {
-                const T w = wx8[x] * wyz;
-#pragma unroll
-                for (int q = 0; q < RBNC; q++) acc[x][q] += w * f[q];
-            }
-        }
-    };
-
-    // candidates in rounds of 2 per thread: all loads of a round are in flight
-    // together; takers are compacted in candidate order (deterministic sums)
-    constexpr int U = 2;
-    int nst = 0;
-    for (int c0 = 0; c0 < ncand; c0 += U * 256) {
-        int is_u[U];
-        bool take_u[U];
-        int b3u[U][3];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int ci = c0 + u * 256 + (int)threadIdx.x;
-            is_u[u] = -1;
-            take_u[u] = false;
-            if (ci < ncand) {
-                int k = 0;
-                while (k + 1 < nbt && s_off[k + 1] <= ci) k++;
-                is_u[u] = s_beg[k] + (ci - s_off[k]);
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (is_u[u] >= 0) {
-                const int is = is_u[u];
-                b3u[u][0] = base[3 * is]; b3u[u][1] = base[3 * is + 1]; b3u[u][2] = base[3 * is + 2];
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (is_u[u] >= 0) {
-                const int dx = wrapk(b3u[u][0] - sx0, K);
-                const int dy = wrapk(b3u[u][1] - sy0, K);
-                const int dz = wrapk(b3u[u][2] - sz0, K);
-                take_u[u] = (dx < sxlen || K - dx < P) && (dy < ts || K - dy < P) &&
-                            (dz < ts || K - dz < P);
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            int tot;
-            const int slot = wg_compact(take_u[u], s_wave, &tot);
-            // the takers fill the stage in candidate order; a full stage is
-            // accumulated and emptied (tot may exceed the capacity)
-            for (int done = 0; done < tot;) {
-                if (nst == cap) {
-                    __syncthreads();
-                    accumulate(nst);
-                    __syncthreads();
-                    nst = 0;
-                }
-                const int take = min(cap - nst, tot - done);
-                if (take_u[u] && slot >= done && slot < done + take) {
-                    const int is = is_u[u];
-                    T* rec = stage + (size_t)(nst + slot - done) * REC;
-                    // forces: slot q holds rhs r, component c (mono: q = 3 r + c;
-                    // poly: q = 6 r + c for f, 6 r + 3 + c for a^2 f); every
-                    // index is a compile-time constant (no register arrays
-                    // indexed at run time)
-                    const double sc = (NC == 6) ? a2[is] : 1.0;
-#pragma unroll
-                    for (int q = 0; q < RBNC; q++) {
-                        const int r = (NC == 6) ? q / 6 : q / 3;
-                        const bool scaled = (NC == 6) && (q % 6) >= 3;
-                        T fv = T(0);
-                        if (r < rb) {
-                            const double x = X[(size_t)(3 * is + q % 3) * b + r0 + r];
-                            fv = (T)(scaled ? x * sc : x);
-                        }
-                        rec[OF + q] = fv;
-                    }
-                    T w[P];
-                    bspline_weights_r<T, P>(frac[3 * is], w);
-#pragma unroll
-                    for (int k = 0; k < 7; k++) rec[k] = T(0);
-#pragma unroll
-                    for (int k = 0; k < P; k++) rec[7 + k] = w[k];
-#pragma unroll
-                    for (int k = 7 + P; k < P + 14; k++) rec[k] = T(0);
-                    bspline_weights_r<T, P>(frac[3 * is + 1], w);
-#pragma unroll
-                    for (int k = 0; k < P; k++) rec[OWY + k] = w[k];
-                    bspline_weights_r<T, P>(frac[3 * is + 2], w);
-#pragma unroll
-                    for (int k = 0; k < P; k++) rec[OWZ + k] = w[k];
-#pragma unroll
-                    for (int d = 0; d < 3; d++) rec[OB + d] = (T)b3u[u][d];
-                }
-                nst += take;
-                done += take;
-            }
-        }
-        __syncthreads();
-    }
-    accumulate(nst);
-    if (!lane_on) return;
-    const size_t K3 = (size_t)K * K * K;
-    const size_t row = ((size_t)zl * K + yl) * K + wx0;
-#pragma unroll
-    for (int q = 0; q < RBNC; q++) {
-        if (q < rbnc) {
-            T* m = mesh + (size_t)(r0 * NC + q) * K3 + row;
-#pragma unroll
-            for (int x = 0; x < 8; x++)
-                if (x < ts) m[x] = acc[x][q];
-        }
-    }
-}
-
 // logical column block of a workgroup (the y part of its XCD-remapped id)
 __device__ __forceinline__ unsigned byl_of(unsigned linear, unsigned n, unsigned gx) {
     return xcd_logical_id(linear, n) / gx;
 }
 
-// Point-owner form (K % 4 == 0): a workgroup of 8 waves owns a 32 x 4 x 4
-// block of mesh points (wave w: x in [4w, 4w+4)), lane l one point
-// (x = l % 4, y = (l / 4) % 4, z = l / 16), and NQ meshes (NQ / NC
+// Point-owner form: a workgroup of 8 waves owns a 32 x 4 x 4 block of mesh
+// points (wave w: x in [4w, 4w+4); the last block of a dimension is partial, K
+// is even: 2 points of 4), lane l one point (x = l % 4, y = (l / 4) % 4,
+// z = l / 16), and NQ meshes (NQ / NC
 // right-hand sides) accumulated in registers. Candidates (base points whose
 // stencil reaches the block) are staged in LDS in candidate order; every wave
 // lists the candidates that reach its 4 x 4 x 4 sub-block, and each lane
@@ -342,17 +136,22 @@ constexpr int kPtThreads = 512;
 constexpr int kPtMaxTiles = 200;   // contributor bucket tiles of one block (host-checked)
 
 //
-// BLK: the forces come from the column-blocked copy Xb[cb][j][c][r] of the
-// packed input (NQ / 3 columns per block, arithmetic type T, monodisperse):
-// a candidate's NQ values are one contiguous run, staged with vector loads,
-// and accumulator q holds component q / (NQ / 3) of column q % (NQ / 3).
+// BLK: the forces come from a column-blocked copy Xb[cb][j][c][r] of the
+// packed input (NQ / 3 columns per block, arithmetic type T; with unequal
+// radii the columns are f and a^2 f of every right-hand side in turn): a
+// candidate's NQ values are one contiguous run, staged with vector loads, and
+// accumulator q holds component q / (NQ / 3) of column q % (NQ / 3). A
+// workgroup takes ncbw column blocks of its mesh block in turn. When all its
+// candidates fit the stage, they are found and their weights staged once;
+// each further column block then only loads the candidates' forces into the
+// stage before its sums and stores.
 //
 // WRAP: K < 32 + P - 1, a stencil can reach both ends of a block along x and
 // stencil offsets are taken modulo K.
 // SGF (with BLK): the forces are not staged; every wave reads a candidate's
 // NQ values at a wave-uniform address, through the scalar data cache into
 // scalar registers, so the FMAs take them as scalar operands and LDS serves
-// only the per-lane weights.
+// only the per-lane weights. One column block per workgroup.
 // MF (FP32, BLK, 48 meshes, staged forces): the sums run on the matrix
 // cores. A wave's sub-block is the product W F of its 64 points x listed
 // candidates weight matrix and the candidates' 48 forces, taken 4 candidates
@@ -360,25 +159,21 @@ constexpr int kPtMaxTiles = 200;   // contributor bucket tiles of one block (hos
 // (row i = 4 y + x), n-tile t = component t of the 16 columns. Each lane
 // forms its A entry (point l % 16, candidate l / 16) from the staged 1D
 // weights, so no lane is spent on points outside a stencil, and its result
-// registers hold 4 consecutive x points of one mesh (one 16-byte store).
-// MA (with MF): one workgroup per mesh block takes every 16-column block in
-// turn (grid y = 1). When all its candidates fit the stage, they are found
-// and their weights staged once; each further column block then only loads
-// the candidates' forces into the stage before its sums and stores. The
-// meshes leave through LDS tiles after the stage (16 columns x 4 rows x 32
-// points of one z plane and component at a time, rows padded to 132 floats
-// so that the waves' 16-byte pieces land in distinct banks; two tiles used
-// in turn): every store instruction then writes whole 128-byte rows.
+// registers hold 4 consecutive x points of one mesh. The meshes leave through
+// LDS tiles after the stage (16 columns x 4 rows x 32 points of one z plane
+// and component at a time, rows padded to 132 floats so that the waves'
+// 16-byte pieces land in distinct banks; two tiles used in turn): every store
+// instruction then writes whole 128-byte rows.
 constexpr int kMaTileStride = 132;                       // floats per column in the tile
 constexpr int kMaTileBytes = 2 * 16 * kMaTileStride * 4;     // two tiles, 16896
-template <typename T, int P, int NQ, bool BLK, bool WRAP, bool SGF = false, bool MF = false,
-          bool MA = false>
-__global__ void __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(NQ <= 12 ? 6 : (MA ? 4 : 1))))
+template <typename T, int P, int NQ, bool BLK, bool WRAP, bool SGF = false, bool MF = false>
+__global__ void __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(NQ <= 12 ? 6 : (BLK && !SGF ? 4 : 1))))
 spread_pt_kernel(int K, int ts, int ntile, int nsx, const int* __restrict__ tile_start,
                  const double* __restrict__ frac, const int* __restrict__ base,
                  const double* __restrict__ a2, const double* __restrict__ X,
-                 const T* __restrict__ Xb, int npos, int b, int RB, int NC, int cap,
+                 const T* __restrict__ Xb, int npos, int b, int ncbw, int NC, int cap,
                  T* __restrict__ mesh, int tiled_out) {
+    constexpr bool MA = BLK && !SGF;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     // record: wx[P] 0, wy[P] 0, wz[P] 0, base - block origin (3 ints in the
     // slots of bx by bz), pad, f[NQ] (16-byte aligned)
@@ -387,9 +182,8 @@ spread_pt_kernel(int K, int ts, int ntile, int nsx, const int* __restrict__ tile
     constexpr int REC = SGF ? OF : OF + NQ;
     static_assert(NQ % 4 == 0, "NQ must be a multiple of 4");
     static_assert(!SGF || BLK, "scalar force reads need the blocked copy");
-    static_assert(!MF || (BLK && !SGF && !WRAP && NQ == 48 && sizeof(T) == 4),
-                  "matrix-core sums: FP32, blocked staged forces, 48 meshes, no wrap");
-    static_assert(!MA || (BLK && !SGF && !WRAP), "column blocks in turn: blocked staged forces");
+    static_assert(!MF || (BLK && !SGF && NQ == 48 && sizeof(T) == 4),
+                  "matrix-core sums: FP32, blocked staged forces, 48 meshes");
     const T* __restrict__ xbb = Xb + (size_t)byl_of(blockIdx.x + blockIdx.y * gridDim.x,
                                                     gridDim.x * gridDim.y, gridDim.x) * npos * NQ;
     T* stage = reinterpret_cast<T*>(smem_raw);
@@ -404,23 +198,32 @@ spread_pt_kernel(int K, int ts, int ntile, int nsx, const int* __restrict__ tile
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const unsigned lid = xcd_logical_id(blockIdx.x + blockIdx.y * gridDim.x, gridDim.x * gridDim.y);
     const int bxl = (int)(lid % gridDim.x), byl = (int)(lid / gridDim.x);
-    const int K4 = K >> 2;
+    const int K4 = (K + 3) >> 2;
     const int sxi = bxl % nsx;
     const int yz = bxl / nsx;
     const int x0 = sxi * 32, y0 = (yz % K4) * 4, z0 = (yz / K4) * 4;
-    const int xlen = min(32, K - x0);
+    const int xlen = min(32, K - x0), ylen = min(4, K - y0), zlen = min(4, K - z0);
     int r0 = byl * (NQ / NC);
     int rb = min(NQ / NC, b - r0);
     int nq = rb * NC;
     const bool wave_on = 4 * wave < xlen;
+    const bool wave_full = 4 * wave + 4 <= xlen;   // else 2 points along x
     // this lane's point, relative to the block origin
     const int lx = 4 * wave + (lane & 3), ly = (lane >> 2) & 3, lz = lane >> 4;
     const int px = x0 + lx, py = y0 + ly, pz = z0 + lz;
+    const bool lane_on = lx < xlen && ly < ylen && lz < zlen;
     T acc[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; q++) acc[q] = T(0);
     // MF: result tiles [z plane m][component t]
     typedef float f4 __attribute__((ext_vector_type(4)));
+    // four points of a mesh row: rows start on 8 bytes where K % 4 != 0
+    typedef float f4m __attribute__((ext_vector_type(4), aligned(8)));
+    typedef float f2m __attribute__((ext_vector_type(2), aligned(8)));
+    auto put4 = [](T* dst, f4 v, bool full) __attribute__((always_inline)) {
+        if (full) *reinterpret_cast<f4m*>(dst) = v;
+        else *reinterpret_cast<f2m*>(dst) = f2m{v.x, v.y};
+    };
     f4 accm[4][3];
 #pragma unroll
     for (int m = 0; m < 4; m++)
@@ -433,7 +236,7 @@ spread_pt_kernel(int K, int ts, int ntile, int nsx, const int* __restrict__ tile
     if (wave == 0) {
         int first[3], cnt[3];
         const int lo[3] = {x0 - (P - 1), y0 - (P - 1), z0 - (P - 1)};
-        const int len[3] = {xlen + P - 1, 4 + P - 1, 4 + P - 1};
+        const int len[3] = {xlen + P - 1, ylen + P - 1, zlen + P - 1};
 #pragma unroll
         for (int d = 0; d < 3; d++) {
             if (len[d] >= K) { first[d] = 0; cnt[d] = ntile; continue; }
@@ -514,12 +317,14 @@ spread_pt_kernel(int K, int ts, int ntile, int nsx, const int* __restrict__ tile
                 if (k < cnt) {
                     const T* rec = stage + (size_t)list[k] * REC;
                     const int* rl = reinterpret_cast<const int*>(rec + OB);
-                    const int dx = (int)min((unsigned)(ax - rl[0]), (unsigned)P);
-                    const int dy = (int)min((unsigned)(ay - rl[1]), (unsigned)P);
-                    wxy = rec[dx] * rec[OWY + dy];
+                    // offset in the stencil (P, a zero weight, outside)
+                    auto off = [K](int d) __attribute__((always_inline)) {
+                        if constexpr (WRAP) return min(wrapk(d, K), P);
+                        else return (int)min((unsigned)d, (unsigned)P);
+                    };
+                    wxy = rec[off(ax - rl[0])] * rec[OWY + off(ay - rl[1])];
 #pragma unroll
-                    for (int m = 0; m < 4; m++)
-                        wz[m] = rec[OWZ + (int)min((unsigned)(m - rl[2]), (unsigned)P)];
+                    for (int m = 0; m < 4; m++) wz[m] = rec[OWZ + off(m - rl[2])];
 #pragma unroll
                     for (int t = 0; t < 3; t++) bf[t] = rec[OF + 16 * t + jj];
                 }
@@ -575,8 +380,8 @@ spread_pt_kernel(int K, int ts, int ntile, int nsx, const int* __restrict__ tile
 
     int nst = 0;
     bool staged_all = false;   // MA: the stage holds every candidate
-    [[maybe_unused]] const int ncb = MA ? (b + NQ / NC - 1) / (NQ / NC) : 1;
-    int cb = 0;
+    int cb = MA ? byl * ncbw : 0;
+    [[maybe_unused]] const int ncb = MA ? min(cb + ncbw, (b + NQ / NC - 1) / (NQ / NC)) : 1;
     // MA: the next column block starts here (a jump back, not a loop, so
     // that the other instances compile without one)
 next_column_block:
@@ -632,7 +437,8 @@ next_column_block:
             const int dx = wrapk(b3[0] - x0, K);
             const int dy = wrapk(b3[1] - y0, K);
             const int dz = wrapk(b3[2] - z0, K);
-            take = (dx < xlen || K - dx < P) && (dy < 4 || K - dy < P) && (dz < 4 || K - dz < P);
+            take = (dx < xlen || K - dx < P) && (dy < ylen || K - dy < P) &&
+                   (dz < zlen || K - dz < P);
         }
         int tot;
         const int slot = wg_compact(take, s_wave, &tot);
@@ -767,11 +573,12 @@ next_column_block:
                         *reinterpret_cast<f4*>(tb + jj * kMaTileStride + sy * 32 + 4 * wave) =
                             accm[m][t];
                     __syncthreads();
-                    if (sj < rb && sx < xlen) {
+                    if (sj < rb && sx < xlen && sr < ylen && m < zlen) {
                         const f4 v =
                             *reinterpret_cast<const f4*>(tb + sj * kMaTileStride + sr * 32 + sx);
-                        *reinterpret_cast<f4*>(mesh + ((size_t)(r0 + sj) * 3 + t) * K3 +
-                                               ((size_t)(z0 + m) * K + (y0 + sr)) * K + x0 + sx) = v;
+                        put4(mesh + ((size_t)(r0 + sj) * 3 + t) * K3 +
+                                 ((size_t)(z0 + m) * K + (y0 + sr)) * K + x0 + sx,
+                             v, sx + 4 <= xlen);
                     }
                 }
 #pragma unroll
@@ -783,15 +590,15 @@ next_column_block:
         }
         if (!tiled_out) {
             const int jj = lane & 15, sy = lane >> 4;
-            if (wave_on && jj < rb) {
+            if (wave_on && jj < rb && sy < ylen) {
 #pragma unroll
                 for (int m = 0; m < 4; m++)
 #pragma unroll
-                    for (int t = 0; t < 3; t++) {
-                        T* dst = mesh + ((size_t)(r0 + jj) * 3 + t) * K3 +
-                                 ((size_t)(z0 + m) * K + (y0 + sy)) * K + x0 + 4 * wave;
-                        *reinterpret_cast<f4*>(dst) = accm[m][t];
-                    }
+                    for (int t = 0; t < 3; t++)
+                        if (m < zlen)
+                            put4(mesh + ((size_t)(r0 + jj) * 3 + t) * K3 +
+                                     ((size_t)(z0 + m) * K + (y0 + sy)) * K + x0 + 4 * wave,
+                                 accm[m][t], wave_full);
             }
             if constexpr (MA) {
 #pragma unroll
@@ -806,7 +613,7 @@ next_column_block:
     if constexpr (MA && !MF) {
         // vector-ALU sums (FP64): per-lane stores, then the next column block
         if (!tiled_out) {
-            if (wave_on) {
+            if (lane_on) {
                 const size_t pt = ((size_t)pz * K + py) * K + px;
                 constexpr int RBB = NQ / 3;
 #pragma unroll
@@ -822,7 +629,7 @@ next_column_block:
         }
     }
     if (!tiled_out) {
-        if (!wave_on) return;
+        if (!lane_on) return;
         const size_t pt = ((size_t)pz * K + py) * K + px;
 #pragma unroll
         for (int q = 0; q < NQ; q++) {
@@ -878,7 +685,7 @@ next_column_block:
                 on = q < nq;
                 mi = (size_t)r0 * NC + q;
             }
-            if (on && x < xlen)
+            if (on && x < xlen && (rw & 3) < ylen && (rw >> 2) < zlen)
                 mesh[mi * K3 + ((size_t)(z0 + (rw >> 2)) * K + (y0 + (rw & 3))) * K + x0 + x] =
                     tile[e];
         }
@@ -1412,6 +1219,12 @@ void SpmeGpu<T>::create(int npos_, double box_, double xi_, int K_, int porder_,
         if (c >= porder - 1 && K % c == 0 && K / c >= 3) { ts = c; break; }
     SDT_REQUIRE(ts > 0, SDT_EINVAL, "no spread tile size divides the mesh dimension");
     ntile = K / ts;
+    // contributor bucket tiles of a 32 x 4 x 4 spread block: bases in
+    // intervals of length min(32, K) + P - 1 (x) and P + 3 (y, z)
+    auto tiles = [&](int len) { return std::min(ntile, (len + ts - 1) / ts + 1); };
+    SDT_REQUIRE(tiles(std::min(32, K) + porder - 1) * tiles(porder + 3) * tiles(porder + 3) <=
+                    kPtMaxTiles,
+                SDT_EINVAL, "spread: too many contributor tiles for this order and mesh");
     std::vector<double> tw(2 * K);
     for (int j = 0; j < K; j++) {
         tw[2 * j] = cos(-2.0 * M_PI * j / K);
@@ -1472,17 +1285,7 @@ void SpmeGpu<T>::gather_sorted(const int* d_perm, const double* d_pos, const dou
                                  hipMemcpyDeviceToDevice, s));
 }
 
-template <typename T>
-bool SpmeGpu<T>::point_owner() const {
-    // contributor bucket tiles of a 32 x 4 x 4 block: bases in intervals of
-    // length min(32, K) + P - 1 (x) and P + 3 (y, z)
-    const int pt_tiles = std::min(ntile, (std::min(32, K) + porder - 1 + ts - 1) / ts + 1) *
-                         std::min(ntile, (porder + 3 + ts - 1) / ts + 1) *
-                         std::min(ntile, (porder + 3 + ts - 1) / ts + 1);
-    return K % 4 == 0 && K >= 16 && pt_tiles <= kPtMaxTiles;
-}
-
-// point-owner meshes per workgroup: 12 when few are needed
+// meshes per workgroup of the spread: 4 or 12 when few are needed
 template <typename T>
 static int pt_meshes(int b, int NC) {
     if (b * NC <= 4) return 4;
@@ -1491,74 +1294,114 @@ static int pt_meshes(int b, int NC) {
 
 template <typename T>
 int SpmeGpu<T>::blocked_cols(int b) const {
-    if (poly || !point_owner()) return 0;
+    if (poly) return 0;
     const int NQ = pt_meshes<T>(b, 3);
     return NQ <= 12 ? 0 : NQ / 3;
+}
+
+// Xs[cb][j][c][r], RC columns per block and zero beyond the last: the spread's
+// own copy of the packed input where it cannot share the real space's. H = 1:
+// column v is right-hand side v; H = 2 (unequal radii): column 2 r + h is
+// right-hand side r, times a^2 for h = 1, so that mesh 3 v + c is mesh
+// 6 r + 3 h + c.
+template <typename T, int RC, int H>
+__global__ void spread_copy_kernel(int npos, int b, int nblk, const double* __restrict__ x,
+                                   const double* __restrict__ a2, T* __restrict__ y) {
+    const long long n = (long long)nblk * npos * 3 * RC;
+    const long long stride = (long long)gridDim.x * blockDim.x;
+    for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += stride) {
+        const int r = (int)(e % RC);
+        const long long q = e / RC;            // (cb npos + j) 3 + c
+        const long long row = q % (3LL * npos);
+        const int v = (int)(q / (3LL * npos)) * RC + r;
+        const int col = v / H;
+        double f = 0.0;
+        if (col < b) {
+            f = x[row * b + col];
+            if (H == 2 && (v & 1)) f *= a2[row / 3];
+        }
+        y[e] = (T)f;
+    }
 }
 
 template <typename T>
 void SpmeGpu<T>::spread(int b, const double* X, hipStream_t s, const T* xb) {
     SDT_REQUIRE(b <= bcap, SDT_ECAP, "spread: rhs count exceeds mesh capacity");
-    const int NC = poly ? 6 : 3;
     SDT_REQUIRE(xb == nullptr || blocked_cols(b) > 0, SDT_EINVAL,
                 "spread: no blocked input for this configuration");
-    if (point_owner()) {
-        const SpmeTuning& tn = tune[width_class(b)];
-        constexpr int NQL = sizeof(T) == 4 ? 48 : 24;
-        const int NQ = pt_meshes<T>(b, NC);
-        // Wide FP32 launches on the blocked copy sum on the matrix cores, one
-        // workgroup per mesh block over every column block (K = 128, 100
-        // columns: 1.08 ms against 2.17 ms for the vector-ALU sums with
-        // scalar force reads, the same sums to the bit); wide FP64 launches
-        // keep the vector-ALU sums over every column block in turn (2.85
-        // against 3.97 ms); where the stencil can wrap, FP32 reads the
-        // blocked forces through the scalar path and FP64 stages them in
-        // LDS per column block. Forms override this for tests.
-        const int fr = spread_form & 3;
-        const bool mf_ok = xb != nullptr && sizeof(T) == 4 && NQ == NQL && K >= 32 + porder - 1;
-        const bool mf = mf_ok && (fr == 0 || fr == 3);
-        const bool ma64 = sizeof(T) == 8 && xb != nullptr && NQ == NQL && K >= 32 + porder - 1 &&
-                          (fr == 0 || (spread_form & 8) != 0);
-        const bool ma = (mf && (fr == 0 || (spread_form & 8) != 0)) || ma64;
-        const bool sgf = xb != nullptr && sizeof(T) == 4 && !mf && fr != 1;
-        const int rec = ((3 * (porder + 1) + 3 + 3) & ~3) + (sgf ? 0 : NQ);
-        // few meshes: a 48 KB stage leaves room for three workgroups per CU
-        // 60 KB for the matrix-core form over every column block, whose two
-        // output tiles (16.5 KB) also fit two workgroups per CU
-        const int stage_bytes =
-            tn.spread_stage_kb > 0 ? tn.spread_stage_kb * 1024
-                                   : (NQ <= 12 ? 48 * 1024 : (mf && ma ? 60 * 1024 : 65536));
-        const int cap = (int)(stage_bytes / (rec * sizeof(T) + 9 * sizeof(int)));
-        // the output tiles reuse the stage's LDS: all meshes, or half of
-        // them above 48 KB (the allocation is at least that)
-        const size_t tile = (size_t)NQ * 512 * sizeof(T);
-        size_t lds = std::max((size_t)cap * (rec * sizeof(T) + 9 * sizeof(int)),
-                              tile <= 49152 ? tile : tile / 2);
-        if (mf && ma && !(spread_form & 4))
-            lds = (((size_t)cap * (rec * sizeof(T) + 9 * sizeof(int)) + 15) & ~(size_t)15) +
-                  kMaTileBytes;
-        const int nsx = (K + 31) / 32;
-        dim3 grid(nsx * (K / 4) * (K / 4), ma ? 1 : ceil_div(b, NQ / NC));
-#define SDT_SPREAD_PWS(PP, QQ, BB, WW, SS, MM, AA)                                             \
-    hipLaunchKernelGGL((spread_pt_kernel<T, PP, QQ, BB, WW, SS, MM, AA>), grid, dim3(kPtThreads), \
-                       lds, s,                                                                   \
-                       K, ts, ntile, nsx, d_tile_start.get(), d_frac.get(), d_base.get(),      \
-                       poly ? d_a2.get() : (double*)nullptr, X, xb, npos, b, NQ / NC, NC, cap, \
-                       d_real.get(), (spread_form & 4) ? 1 : 0)
+    const SpmeTuning& tn = tune[width_class(b)];
+    constexpr int NQL = sizeof(T) == 4 ? 48 : 24;
+    int NC = poly ? 6 : 3;
+    const int NQ = pt_meshes<T>(b, NC);
+    const int fr = spread_form & 3;
+    // Wide launches read a blocked copy and take the column blocks of a mesh
+    // block in turn. FP32 sums on the matrix cores (K = 128, 100 columns:
+    // 1.06 ms against 2.17 ms for the vector-ALU sums with scalar force
+    // reads, the same sums to the bit; unequal radii, 13 columns at K = 96:
+    // 0.10 against 0.19 ms; 8 columns at K = 216: 0.62 against 0.82 ms), FP64
+    // on the vector ALUs. K = 90, 100 FP32 columns: 0.40 ms, 16 FP64 columns:
+    // 0.14 ms (1.68 and 0.56 ms for a tile-owner form that kept mesh sides
+    // other than multiples of 4). Forms override this for tests.
+    int cols = b;
+    if (NQ == NQL && xb == nullptr && (sizeof(T) == 4 || !poly)) {
+        cols = poly ? 2 * b : b;
+        constexpr int RC = NQL / 3;
+        const int nblk = ceil_div(cols, RC);
+        const long long n = (long long)nblk * npos * 3 * RC;
+        d_xs.reserve((size_t)n);
+        const dim3 g((unsigned)std::min<long long>(ceil_div((size_t)n, 256), 8192));
+        if (poly)
+            hipLaunchKernelGGL((spread_copy_kernel<T, RC, 2>), g, dim3(256), 0, s, npos, b, nblk, X,
+                               d_a2.get(), d_xs.get());
+        else
+            hipLaunchKernelGGL((spread_copy_kernel<T, RC, 1>), g, dim3(256), 0, s, npos, b, nblk, X,
+                               (const double*)nullptr, d_xs.get());
+        SDT_HIP_CHECK(hipGetLastError());
+        xb = d_xs.get();
+    }
+    if (xb != nullptr) NC = 3;   // the copy's columns have three meshes each
+    const bool mf = xb != nullptr && sizeof(T) == 4 && (fr == 0 || fr == 3);
+    const bool sgf = xb != nullptr && sizeof(T) == 4 && !mf && fr != 1;
+    const int rec = ((3 * (porder + 1) + 3 + 3) & ~3) + (sgf ? 0 : NQ);
+    // few meshes: a 48 KB stage leaves room for three workgroups per CU;
+    // 60 KB for the matrix-core form, whose two output tiles (16.5 KB) also
+    // fit two workgroups per CU
+    const int stage_bytes = tn.spread_stage_kb > 0
+                                ? tn.spread_stage_kb * 1024
+                                : (NQ <= 12 ? 48 * 1024 : (mf ? 60 * 1024 : 65536));
+    const int cap = (int)(stage_bytes / (rec * sizeof(T) + 9 * sizeof(int)));
+    // the output tiles reuse the stage's LDS: all meshes, or half of
+    // them above 48 KB (the allocation is at least that)
+    const size_t tile = (size_t)NQ * 512 * sizeof(T);
+    size_t lds = std::max((size_t)cap * (rec * sizeof(T) + 9 * sizeof(int)),
+                          tile <= 49152 ? tile : tile / 2);
+    if (mf && !(spread_form & 4))
+        lds = (((size_t)cap * (rec * sizeof(T) + 9 * sizeof(int)) + 15) & ~(size_t)15) +
+              kMaTileBytes;
+    const int nsx = (K + 31) / 32;
+    const unsigned nblocks = nsx * ceil_div(K, 4) * ceil_div(K, 4);
+    const int ncb = ceil_div(cols, NQ / NC);
+    // column blocks a workgroup takes in turn: all of them where the mesh
+    // blocks alone fill the chip twice over (two workgroups per CU), fewer on
+    // small meshes; one with scalar force reads, and in the forms that ask
+    // for it
+    int ncbw = 1;
+    if (xb != nullptr && !sgf && (fr == 0 || (spread_form & 8)))
+        ncbw = ceil_div(ncb, std::min<unsigned>(ncb, ceil_div(1024, nblocks)));
+    const dim3 grid(nblocks, ceil_div(ncb, ncbw));
+#define SDT_SPREAD_PWS(PP, QQ, BB, WW, SS, MM)                                                 \
+    hipLaunchKernelGGL((spread_pt_kernel<T, PP, QQ, BB, WW, SS, MM>), grid, dim3(kPtThreads),  \
+                       lds, s, K, ts, ntile, nsx, d_tile_start.get(), d_frac.get(),           \
+                       d_base.get(), poly ? d_a2.get() : (double*)nullptr, X, xb, npos, cols, \
+                       ncbw, NC, cap, d_real.get(), (spread_form & 4) ? 1 : 0)
 #define SDT_SPREAD_PW(PP, QQ, BB, WW)                                                          \
     do {                                                                                      \
         if constexpr (BB && sizeof(T) == 4) {                                                 \
-            if (sgf) SDT_SPREAD_PWS(PP, QQ, BB, WW, true, false, false);                       \
-            else if constexpr (QQ == 48 && !WW) {                                             \
-                if (ma) SDT_SPREAD_PWS(PP, QQ, BB, WW, false, true, true);                     \
-                else if (mf) SDT_SPREAD_PWS(PP, QQ, BB, WW, false, true, false);               \
-                else SDT_SPREAD_PWS(PP, QQ, BB, WW, false, false, false);                      \
-            } else SDT_SPREAD_PWS(PP, QQ, BB, WW, false, false, false);                        \
-        } else if constexpr (BB && QQ == NQL && !WW) {                                      \
-            if (ma) SDT_SPREAD_PWS(PP, QQ, BB, WW, false, false, true);                        \
-            else SDT_SPREAD_PWS(PP, QQ, BB, WW, false, false, false);                          \
+            if (sgf) SDT_SPREAD_PWS(PP, QQ, BB, WW, true, false);                              \
+            else if (mf) SDT_SPREAD_PWS(PP, QQ, BB, WW, false, true);                          \
+            else SDT_SPREAD_PWS(PP, QQ, BB, WW, false, false);                                 \
         } else {                                                                              \
-            SDT_SPREAD_PWS(PP, QQ, BB, WW, false, false, false);                               \
+            SDT_SPREAD_PWS(PP, QQ, BB, WW, false, false);                                      \
         }                                                                                     \
     } while (0)
 #define SDT_SPREAD_PT(PP, QQ, BB)                                                              \
@@ -1566,41 +1409,24 @@ void SpmeGpu<T>::spread(int b, const double* X, hipStream_t s, const T* xb) {
         if (K < 32 + PP - 1) SDT_SPREAD_PW(PP, QQ, BB, true);                                  \
         else SDT_SPREAD_PW(PP, QQ, BB, false);                                                 \
     } while (0)
+#define SDT_SPREAD_WIDE(PP)                                                                    \
+    do {                                                                                      \
+        if constexpr (sizeof(T) == 4) SDT_SPREAD_PT(PP, NQL, true);                            \
+        else if (xb) SDT_SPREAD_PT(PP, NQL, true);                                             \
+        else SDT_SPREAD_PT(PP, NQL, false);                                                    \
+    } while (0)
 #define SDT_SPREAD_P(PP)                                                                       \
     case PP:                                                                                   \
         if (NQ == 4) SDT_SPREAD_PT(PP, 4, false);                                              \
         else if (NQ == 12) SDT_SPREAD_PT(PP, 12, false);                                       \
-        else if (xb) SDT_SPREAD_PT(PP, NQL, true);                                             \
-        else SDT_SPREAD_PT(PP, NQL, false);                                                    \
+        else SDT_SPREAD_WIDE(PP);                                                              \
         break;
-        switch (porder) { SDT_SPREAD_P(4) SDT_SPREAD_P(5) SDT_SPREAD_P(6) SDT_SPREAD_P(7) SDT_SPREAD_P(8) }
+    switch (porder) { SDT_SPREAD_P(4) SDT_SPREAD_P(5) SDT_SPREAD_P(6) SDT_SPREAD_P(7) SDT_SPREAD_P(8) }
 #undef SDT_SPREAD_P
+#undef SDT_SPREAD_WIDE
 #undef SDT_SPREAD_PT
 #undef SDT_SPREAD_PW
 #undef SDT_SPREAD_PWS
-        SDT_HIP_CHECK(hipGetLastError());
-        return;
-    }
-    // right-hand sides per workgroup: RB * NC register accumulators per point
-    const int RBNC = poly ? 12 : 12;
-    const int RB = RBNC / NC;
-    const int nsx = (ntile + 3) / 4;
-    const int rec = 3 * porder + 17 + RBNC;
-    // staging list of up to 64 KB (any capacity works: a full stage is
-    // accumulated and emptied)
-    const int cap = (int)(65536 / (rec * sizeof(T)));
-    SDT_REQUIRE(cap >= 64, SDT_EINVAL, "spread: staging buffer too small");
-    const size_t lds = (size_t)cap * rec * sizeof(T);
-    dim3 grid(nsx * ntile * ntile, ceil_div(b, RB));
-#define SDT_SPREAD(PP)                                                                        \
-    case PP:                                                                                  \
-        hipLaunchKernelGGL((spread_gather_kernel<T, PP, 12>), grid, dim3(256), lds, s, K, ts, \
-                           ntile, nsx, d_tile_start.get(), d_frac.get(), d_base.get(),        \
-                           poly ? d_a2.get() : (double*)nullptr, X, b, RB, NC, cap,          \
-                           d_real.get());                                                     \
-        break;
-    switch (porder) { SDT_SPREAD(4) SDT_SPREAD(5) SDT_SPREAD(6) SDT_SPREAD(7) SDT_SPREAD(8) }
-#undef SDT_SPREAD
     SDT_HIP_CHECK(hipGetLastError());
 }
 
