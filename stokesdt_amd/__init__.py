@@ -289,9 +289,8 @@ class MobSpme:
     def set_forms(self, interp=0, z=0, spread=0, fft=0):
         """Launch forms (testing and measurement): interp meshes per LDS pass
         (0 built-in, 1, 2 or 4 (FP32)); z transform shape (0 built-in,
-        1 .. 5); spread form (0 built-in, 1 forces in LDS, 2 scalar force
-        reads, 3 matrix-core sums; plus 4 for row-tiled mesh stores, plus 8
-        for column blocks in turn); x / y transforms (0 fused planes where
+        1 .. 5); spread form (0 built-in matrix-core sums, 1 or 2 vector-ALU
+        sums, 3 one column block per workgroup); x / y transforms (0 fused planes where
         they fit, 1 separate passes)."""
         _check(lib().sdt_debug_spme_forms(self.h, int(interp), int(z), int(spread), int(fft)))
 

@@ -54,9 +54,8 @@ struct SpmeGpu {
     // z transform launch shape: 0 the built-in choice, 1 .. 5 at most
     // (threads, pencils) = (256, 16), (128, 16), (256, 8), (128, 8), (256, 4)
     int z_form = 0;
-    // spread launch form: bits 0-1, force reads of wide FP32 launches (0
-    // built-in = scalar loads, 1 staged in LDS, 2 scalar loads); bit 2, mesh
-    // stores as whole rows through LDS instead of per lane
+    // spread launch form, low bits: 0 matrix cores, 1 and 2 the vector-ALU
+    // comparison form, 3 one column block per workgroup (with 8: in turn)
     int spread_form = 0;
     // x / y transforms: 0 the fused plane kernels where a plane fits LDS,
     // 1 the separate x and y passes
@@ -66,9 +65,14 @@ struct SpmeGpu {
     DevBuf<double> d_tw;   // K roots of unity (cos, sin) of -2*pi*j/K
     DevBuf<double> d_fac;  // influence factor per wavenumber index, K entries
     DevBuf<double> d_frac; // 3N fractional offsets (sorted order)
+    DevBuf<T> d_sten;      // stencil records (sorted order), sten_n values each
+    int sten_n = 0;
     DevBuf<int> d_base;    // 3N B-spline base mesh indices (sorted order)
     DevBuf<double> d_a2;   // N radii squared (sorted order), poly only
     DevBuf<int> d_tile_start;  // ntile^3 + 1
+    // candidates of every 32 x 4 x 4 spread block: (offset, count) into d_ids
+    DevBuf<int2> d_blk;
+    DevBuf<int> d_ids, d_nids;
     DevBuf<T> d_real;      // nmesh * K^3
     DevBuf<cplx<T>> d_spec;    // nmesh * K*K*Kh
 

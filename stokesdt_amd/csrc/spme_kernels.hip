@@ -2,12 +2,12 @@
 //
 // Reference algorithm: src/mob/spme.cc (UpdateSpmeEngine_ :366-509, Spread
 // :313-363, ApplyInfluence :201-310, Interpolate :163-198, ComputeSpline
-// :71-160, ComputeSpmeRecip_ :714-839). The GPU form recomputes B-spline
-// weights from per-particle fractional offsets instead of storing the
-// N x p^3 P/ind tables, fuses all b right-hand sides into each launch,
-// spreads by owner-computes mesh tiles accumulated in LDS (plain stores, no
-// global atomics, no zero-fill pass), and fuses the influence multiply
-// between the forward and inverse z-transforms.
+// :71-160, ComputeSpmeRecip_ :714-839). The GPU form keeps 3 p weights per
+// particle or its fractional offsets instead of the N x p^3 P/ind tables,
+// fuses all b right-hand sides into each launch, spreads by mesh blocks that
+// sum their own points on the matrix cores (plain stores, no global atomics,
+// no zero-fill pass), and fuses the influence multiply between the forward
+// and inverse z-transforms.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -76,634 +76,605 @@ __global__ void spme_prepare_kernel(int npos, const double* __restrict__ pos, do
     key[i] = (t[2] * ntile + t[1]) * ntile + t[0];
 }
 
-template <typename T>
+// One particle's stencil record, made once per update and read by every
+// spread: the base index (3 ints in one 16-byte slot), then
+// the 1D weights 0 0 0 wx[P] 0 0 0 wy[P] 0 0 0 wz[P] 0 0 0, padded to 16
+// bytes. The zeros are the weights of the points up to 3 outside a stencil, so
+// that 4 points of a mesh block read theirs without a range test. (The
+// interpolation makes its weights from the offsets again: a record's bytes per
+// group of 4 columns cost it more, 3.56 against 3.19 ms for 100 FP64 columns
+// at K = 128.)
+template <typename T, int P>
+struct Sten {
+    static constexpr int V = 16 / (int)sizeof(T);    // values per 16 bytes
+    static constexpr int RUN = P + 3;                // from one run to the next
+    static constexpr int OW = V + 3;                 // wx[0]
+    static constexpr int N = (V + 3 * RUN + 3 + V - 1) / V * V;
+};
+
+template <typename T, int P>
 __global__ void spme_gather_kernel(int npos, const int* __restrict__ perm,
                                    const double* __restrict__ frac_u, const int* __restrict__ base_u,
-                                   const double* __restrict__ rdi, double* __restrict__ frac,
-                                   int* __restrict__ base, double* __restrict__ a2) {
+                                   const double* __restrict__ rdi, T* __restrict__ sten,
+                                   double* __restrict__ frac, int* __restrict__ base,
+                                   double* __restrict__ a2, int* __restrict__ nids) {
+    typedef Sten<T, P> St;
     const int is = blockIdx.x * blockDim.x + threadIdx.x;
+    if (is == 0) *nids = 0;   // for spread_list_kernel, next on the stream
     if (is >= npos) return;
     const int i = perm[is];
+    T* rec = sten + (size_t)is * St::N;
+    int* rb = reinterpret_cast<int*>(rec);
 #pragma unroll
     for (int d = 0; d < 3; d++) {
-        frac[3 * is + d] = frac_u[3 * i + d];
-        base[3 * is + d] = base_u[3 * i + d];
+        const int b = base_u[3 * i + d];
+        base[3 * is + d] = b;
+        rb[d] = b;
+        const double fr = frac_u[3 * i + d];
+        frac[3 * is + d] = fr;
+        T w[P];
+        bspline_weights_r<T, P>(fr, w);
+#pragma unroll
+        for (int k = 0; k < P; k++) rec[St::OW + d * St::RUN + k] = w[k];
+#pragma unroll
+        for (int k = 1; k <= 3; k++) rec[St::OW + d * St::RUN - k] = T(0);
     }
+#pragma unroll
+    for (int k = St::V + 3 * St::RUN; k < St::N; k++) rec[k] = T(0);
     if (a2) a2[is] = rdi[i] * rdi[i];
 }
 
 // ------------------------------------------------------------- spread ------
-// exclusive prefix over the workgroup of a 0/1 predicate; returns this
-// thread's slot and the total (all threads must call)
-__device__ __forceinline__ int wg_compact(bool pred, int* s_wave, int* total) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const unsigned long long m = __ballot(pred);
-    const int before = __popcll(m & ((1ull << lane) - 1ull));
-    if (lane == 0) s_wave[wave] = __popcll(m);
-    __syncthreads();
-    int off = 0, tot = 0;
-    const int nw = blockDim.x >> 6;
-    for (int w = 0; w < nw; w++) {
-        const int c = s_wave[w];
-        off += (w < wave) ? c : 0;
-        tot += c;
-    }
-    __syncthreads();
-    *total = tot;
-    return off + before;
-}
-
 __device__ __forceinline__ int wrapk(int d, int K) {
     d += (d < 0) ? K : 0;
     return d - ((d >= K) ? K : 0);
 }
 
-// logical column block of a workgroup (the y part of its XCD-remapped id)
-__device__ __forceinline__ unsigned byl_of(unsigned linear, unsigned n, unsigned gx) {
-    return xcd_logical_id(linear, n) / gx;
-}
-
 // Point-owner form: a workgroup of 8 waves owns a 32 x 4 x 4 block of mesh
 // points (wave w: x in [4w, 4w+4); the last block of a dimension is partial, K
-// is even: 2 points of 4), lane l one point (x = l % 4, y = (l / 4) % 4,
-// z = l / 16), and NQ meshes (NQ / NC
-// right-hand sides) accumulated in registers. Candidates (base points whose
-// stencil reaches the block) are staged in LDS in candidate order; every wave
-// lists the candidates that reach its 4 x 4 x 4 sub-block, and each lane
-// adds w = wx[x - bx] wy[y - by] wz[z - bz] (0 outside the stencil) times the
-// NQ forces. Deterministic, no atomics, small per-candidate overhead.
+// is even: 2 points of 4). The block's candidates (particles whose stencil
+// reaches it, spread_list_kernel) are staged in LDS in list order, stencil
+// record and forces; every wave lists the candidates that reach its 4 x 4 x 4
+// sub-block and adds w = wx[x - bx] wy[y - by] wz[z - bz] (0 outside the
+// stencil) times their forces. Deterministic, no atomics.
 constexpr int kPtThreads = 512;
-constexpr int kPtMaxTiles = 200;   // contributor bucket tiles of one block (host-checked)
 
+// The candidates of every 32 x 4 x 4 mesh block, listed once per update: one
+// wave per block goes through the particles of the tiles its window touches
+// (the tiles of a row along x are one range of the sorted order, two where
+// they wrap) and keeps those whose stencil reaches the block, in that order.
+// blk[block] = (offset, count) into ids; the offsets come from an atomic
+// counter, so segments lie in any order, but each one's content is fixed.
+// Finding the candidates inside every spread took a third of its 89 us for one
+// column at K = 128, N = 100 000 (62 us from the lists).
+constexpr int kListWaves = 16;
+constexpr int kListRanges = 64;   // ranges of one block (host-checked)
+constexpr int kListMasks = 32;    // candidate groups whose test is kept for the second pass
+
+template <int P>
+__global__ void __launch_bounds__(64 * kListWaves)
+spread_list_kernel(int K, int ts, int ntile, int nsx, int nblocks,
+                   const int* __restrict__ tile_start, const int* __restrict__ base,
+                   int* __restrict__ nids, int2* __restrict__ blk, int* __restrict__ ids) {
+    __shared__ int s_off_[kListWaves][kListRanges], s_beg_[kListWaves][kListRanges];
+    __shared__ unsigned long long s_mask_[kListWaves][kListMasks];
+    __shared__ int s_tot[kListWaves];
+    __shared__ int s_base;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // waves past the last block repeat it and keep nothing
+    const bool real = blockIdx.x * kListWaves + wave < nblocks;
+    const int bl = min((int)(blockIdx.x * kListWaves + wave), nblocks - 1);
+    int* s_off = s_off_[wave];
+    int* s_beg = s_beg_[wave];
+    unsigned long long* s_mask = s_mask_[wave];
+    const int K4 = (K + 3) >> 2;
+    const int yz = bl / nsx;
+    const int org[3] = {(bl % nsx) * 32, (yz % K4) * 4, (yz / K4) * 4};
+    const int ext[3] = {min(32, K - org[0]), min(4, K - org[1]), min(4, K - org[2])};
+    // base tiles of the window [org - (P - 1), org + ext) in each dimension
+    int first[3], cnt[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const int lo = org[d] - (P - 1), len = ext[d] + P - 1;
+        if (len >= K) { first[d] = 0; cnt[d] = ntile; continue; }
+        const int a = (lo >= 0) ? lo / ts : -((-lo + ts - 1) / ts);
+        const int e = lo + len - 1;              // >= 0
+        cnt[d] = min(e / ts - a + 1, ntile);
+        first[d] = ((a % ntile) + ntile) % ntile;
+    }
+    const int nr = 2 * cnt[1] * cnt[2];
+    int pb = 0, n = 0;
+    if (lane < nr) {
+        const int row = lane >> 1;
+        const int ty = (first[1] + row % cnt[1]) % ntile, tz = (first[2] + row / cnt[1]) % ntile;
+        const int n1 = min(cnt[0], ntile - first[0]);    // tiles before the wrap
+        const int t0 = (tz * ntile + ty) * ntile + ((lane & 1) ? 0 : first[0]);
+        const int nt = (lane & 1) ? cnt[0] - n1 : n1;
+        pb = tile_start[t0];
+        n = tile_start[t0 + nt] - pb;
+    }
+    int inc = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int t = __shfl_up(inc, o);
+        if (lane >= o) inc += t;
+    }
+    s_off[lane] = inc - n;
+    s_beg[lane] = pb;
+    const int ncand = __shfl(inc, 63);
+    // the LDS tables are this wave's own (its accesses complete in order)
+    __builtin_amdgcn_wave_barrier();
+    // particle of candidate ci: the last range whose offset is <= ci
+    auto particle = [&](int ci) __attribute__((always_inline)) {
+        int k = 0, hi = nr - 1;
+        while (k < hi) {
+            const int mid = (k + hi + 1) >> 1;
+            if (s_off[mid] <= ci) k = mid;
+            else hi = mid - 1;
+        }
+        return s_beg[k] + (ci - s_off[k]);
+    };
+    auto reaches = [&](const int* b3) __attribute__((always_inline)) {
+        bool take = true;
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            const int r = wrapk(b3[d] - org[d], K);
+            take = take && (r < ext[d] || K - r < P);
+        }
+        return take;
+    };
+    // U groups of 64 at a time, their loads in flight together
+    constexpr int U = 4;
+    int total = 0;
+    for (int c0 = 0, g = 0; c0 < ncand; c0 += 64 * U, g += U) {
+        int b3[U][3];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int is = particle(min(c0 + 64 * u + lane, ncand - 1));
+#pragma unroll
+            for (int d = 0; d < 3; d++) b3[u][d] = base[3 * is + d];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const unsigned long long m = __ballot(c0 + 64 * u + lane < ncand && reaches(b3[u]));
+            if (lane == 0 && g + u < kListMasks) s_mask[g + u] = m;
+            total += __popcll(m);
+        }
+    }
+    // one atomic a workgroup: same-address atomics of every wave took 35 us
+    if (!real) total = 0;
+    if (lane == 0) s_tot[wave] = total;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int sum = 0;
+        for (int w = 0; w < kListWaves; w++) {
+            const int t = s_tot[w];
+            s_tot[w] = sum;
+            sum += t;
+        }
+        s_base = sum > 0 ? atomicAdd(nids, sum) : 0;
+    }
+    __syncthreads();
+    if (!real) return;
+    int off = s_base + s_tot[wave];
+    if (lane == 0) blk[bl] = make_int2(off, total);
+    for (int c0 = 0, g = 0; c0 < ncand; c0 += 64, g++) {
+        const int ci = c0 + lane;
+        const int is = particle(min(ci, ncand - 1));
+        const unsigned long long m =
+            g < kListMasks ? s_mask[g] : __ballot(ci < ncand && reaches(base + 3 * is));
+        if ((m >> lane) & 1) ids[off + __popcll(m & ((1ull << lane) - 1ull))] = is;
+        off += __popcll(m);
+    }
+}
+
+
+// The sums run on the matrix cores (v_mfma_*_16x16x4): a wave's sub-block is
+// the product W F of its 64 points x listed candidates weight matrix and the
+// candidates' forces, 4 candidates at a time; m-tile m = the 16 points of z
+// plane m (row i = 4 y + x), NT n-tiles of 16 force values. Each lane forms
+// its A entry (point l % 16, candidate l / 16) from the staged 1D weights, so
+// no lane is spent on points outside a stencil. The matrix cores add the 4
+// products of a step in candidate order with one rounding each, so the sums
+// are those of the vector form below to the bit.
 //
-// BLK: the forces come from a column-blocked copy Xb[cb][j][c][r] of the
-// packed input (NQ / 3 columns per block, arithmetic type T; with unequal
-// radii the columns are f and a^2 f of every right-hand side in turn): a
-// candidate's NQ values are one contiguous run, staged with vector loads, and
-// accumulator q holds component q / (NQ / 3) of column q % (NQ / 3). A
+// BLK (wide launches): the forces come from a column-blocked copy
+// Xb[cb][j][c][r] of the packed input (NQ / 3 columns per block, arithmetic
+// type T; with unequal radii the columns are f and a^2 f of every right-hand
+// side in turn), so a candidate's NQ values are one contiguous run; value q
+// belongs to component q / (NQ / 3) of column q % (NQ / 3). FP32: 48 values, 3
+// n-tiles. FP64: 24 values, 2 n-tiles (8 slots of the second idle). A
 // workgroup takes ncbw column blocks of its mesh block in turn. When all its
-// candidates fit the stage, they are found and their weights staged once;
-// each further column block then only loads the candidates' forces into the
-// stage before its sums and stores.
+// candidates fit the stage they are staged and listed once; each further
+// column block then only loads the candidates' forces before its sums and
+// stores.
+// Otherwise (at most 16 meshes): the forces of mesh q = NC r + c are read from
+// the packed input, NQ = 4 or 16 slots, one n-tile.
 //
-// WRAP: K < 32 + P - 1, a stencil can reach both ends of a block along x and
-// stencil offsets are taken modulo K.
-// SGF (with BLK): the forces are not staged; every wave reads a candidate's
-// NQ values at a wave-uniform address, through the scalar data cache into
-// scalar registers, so the FMAs take them as scalar operands and LDS serves
-// only the per-lane weights. One column block per workgroup.
-// MF (FP32, BLK, 48 meshes, staged forces): the sums run on the matrix
-// cores. A wave's sub-block is the product W F of its 64 points x listed
-// candidates weight matrix and the candidates' 48 forces, taken 4 candidates
-// at a time by v_mfma_f32_16x16x4f32: m-tile m = the 16 points of z plane m
-// (row i = 4 y + x), n-tile t = component t of the 16 columns. Each lane
-// forms its A entry (point l % 16, candidate l / 16) from the staged 1D
-// weights, so no lane is spent on points outside a stencil, and its result
-// registers hold 4 consecutive x points of one mesh. The meshes leave through
-// LDS tiles after the stage (16 columns x 4 rows x 32 points of one z plane
-// and component at a time, rows padded to 132 floats so that the waves'
-// 16-byte pieces land in distinct banks; two tiles used in turn): every store
-// instruction then writes whole 128-byte rows.
-constexpr int kMaTileStride = 132;                       // floats per column in the tile
-constexpr int kMaTileBytes = 2 * 16 * kMaTileStride * 4;     // two tiles, 16896
-template <typename T, int P, int NQ, bool BLK, bool WRAP, bool SGF = false, bool MF = false>
-__global__ void __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(NQ <= 12 ? 6 : (BLK && !SGF ? 4 : 1))))
-spread_pt_kernel(int K, int ts, int ntile, int nsx, const int* __restrict__ tile_start,
-                 const double* __restrict__ frac, const int* __restrict__ base,
-                 const double* __restrict__ a2, const double* __restrict__ X,
-                 const T* __restrict__ Xb, int npos, int b, int ncbw, int NC, int cap,
-                 T* __restrict__ mesh, int tiled_out) {
-    constexpr bool MA = BLK && !SGF;
+// The meshes leave through LDS tiles after the stage (16 force values x 4 rows
+// x 32 points of one z plane at a time; 4 values x 4 planes for NQ = 4; rows
+// padded so that the waves' pieces land in distinct banks): every store
+// instruction then writes whole rows of the block. Stores of 16-byte pieces
+// per lane reached HBM 1.4 times. FP32 uses two tiles in turn, one barrier a
+// round; FP64 one, to fit two workgroups per CU.
+//
+// Measured (with the candidates found and their weights made in every launch
+// and the vector ALUs for narrow and FP64 launches -> now): one FP32 column,
+// K = 128, N = 100 000: 96 -> 62 us (30 M wave instructions bounded it); 16
+// columns 210 -> 180 us, 100 columns 1.06 -> 1.01 ms (the meshes alone take
+// 0.5 ms to write); 8 columns, K = 216, N = 200 000: 620 -> 440 us; FP64, 100
+// columns, K = 128: 3.2 -> 2.7 ms, 16 columns, K = 90: 144 -> 114 us.
+constexpr int kTileRow = 132;    // values per force value and plane in a tile
+
+template <typename T, int NQ>
+struct SpreadTile {
+    static constexpr int cols = NQ < 16 ? NQ : 16;      // force values of a round
+    static constexpr int planes = NQ == 4 ? 4 : 1;      // z planes of a round
+    static constexpr int bufs = sizeof(T) == 4 && planes == 1 ? 2 : 1;
+    static constexpr size_t bytes = (size_t)bufs * planes * cols * kTileRow * sizeof(T);
+};
+
+// values per staged candidate: record, forces, and a pad that makes it an odd
+// number of 16-byte slots (lanes reading consecutive candidates' bases then
+// spread over the banks)
+template <typename T>
+__host__ __device__ constexpr int spread_slot(int sten_n, int nq) {
+    constexpr int V = 16 / (int)sizeof(T);
+    return ((sten_n + nq) / V | 1) * V;
+}
+// and its LDS bytes, with the eight waves' lists and the particle id
+template <typename T>
+static size_t spread_slot_bytes(int sten_n, int nq) {
+    return (size_t)spread_slot<T>(sten_n, nq) * sizeof(T) + 8 * sizeof(unsigned) + sizeof(int);
+}
+
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef double d4v __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ f4v mfma16(float a, float b, f4v c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ d4v mfma16(double a, double b, d4v c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// stages candidates list_g[0 .. n) of a block: their records with the base
+// relative to the block origin (in (-P, K - P]), with NV > 0 followed by 16 NV
+// bytes of blocked forces each; 16 bytes per load, the loads of a thread in
+// flight together
+template <typename T, int P, int NV>
+__device__ __forceinline__ void spread_stage(int n, const int* __restrict__ list_g,
+                                             const T* __restrict__ sten,
+                                             const T* __restrict__ frc, const int* org, int K,
+                                             int rec_n, T* stage, int* s_pid) {
+    typedef Sten<T, P> St;
+    typedef T VT __attribute__((ext_vector_type(16 / sizeof(T))));
+    typedef int I4 __attribute__((ext_vector_type(4)));
+    constexpr int HV = St::N / St::V, SV = HV + NV, U = NV > 0 ? 4 : 2;
+    const VT* rec_g = reinterpret_cast<const VT*>(sten);
+    const VT* frc_g = reinterpret_cast<const VT*>(frc);
+    for (int e0 = threadIdx.x; e0 < n * SV; e0 += kPtThreads * U) {
+        VT v[U];
+        int pid[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) pid[u] = list_g[min(e0 + u * kPtThreads, n * SV - 1) / SV];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int e = min(e0 + u * kPtThreads, n * SV - 1), q = e - (e / SV) * SV;
+            v[u] = NV == 0 || q < HV ? rec_g[(size_t)pid[u] * HV + q]
+                                     : frc_g[(size_t)pid[u] * NV + (q - HV)];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int e = e0 + u * kPtThreads;
+            if (e >= n * SV) continue;
+            const int sl = e / SV, q = e - sl * SV;
+            if (q == 0) {
+                s_pid[sl] = pid[u];
+                I4 b3 = *reinterpret_cast<I4*>(&v[u]);
+#pragma unroll
+                for (int d = 0; d < 3; d++) {
+                    const int r = wrapk(b3[d] - org[d], K);
+                    b3[d] = r > K - P ? r - K : r;
+                }
+                v[u] = *reinterpret_cast<VT*>(&b3);
+            }
+            *reinterpret_cast<VT*>(stage + (size_t)sl * rec_n + q * St::V) = v[u];
+        }
+    }
+}
+
+// the blocked forces of the staged candidates for another column block
+template <typename T, int NQ>
+__device__ __forceinline__ void spread_restage(int n, const int* s_pid, const T* __restrict__ frc,
+                                               int rec_n, T* out) {
+    typedef T VT __attribute__((ext_vector_type(16 / sizeof(T))));
+    constexpr int V = 16 / (int)sizeof(T), NV = NQ / V, U = 4;
+    const VT* src = reinterpret_cast<const VT*>(frc);
+    for (int e0 = threadIdx.x; e0 < n * NV; e0 += kPtThreads * U) {
+        VT v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int e = min(e0 + u * kPtThreads, n * NV - 1);
+            v[u] = src[(size_t)s_pid[e / NV] * NV + e % NV];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int e = e0 + u * kPtThreads;
+            if (e < n * NV)
+                *reinterpret_cast<VT*>(out + (size_t)(e / NV) * rec_n + e % NV * V) = v[u];
+        }
+    }
+}
+
+// forces of the staged candidates from the packed input: slot q holds mesh
+// q0 + q, mesh NC r + c the component c % 3 of right-hand side r, times a^2
+// for c >= 3; zero beyond the last mesh. A thread serves one slot.
+template <typename T, int NQ>
+__device__ __forceinline__ void spread_stage_packed(int n, const int* s_pid,
+                                                    const double* __restrict__ X,
+                                                    const double* __restrict__ a2, int b, int NC,
+                                                    int q0, int rec_n, T* frc) {
+    static_assert(kPtThreads % NQ == 0, "one slot per thread");
+    constexpr int U = 2, S = kPtThreads / NQ;
+    const int q = threadIdx.x % NQ, r = (q0 + q) / NC, c = (q0 + q) - r * NC;
+    const bool on = r < b, scaled = c >= 3;
+    const double* x = X + (size_t)(c % 3) * b + r;
+    for (int i0 = threadIdx.x / NQ; i0 < n; i0 += U * S) {
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            v[u] = 0.0;
+            if (on && i0 + u * S < n) {
+                const int p = s_pid[i0 + u * S];
+                v[u] = x[(size_t)(3 * p) * b];
+                if (scaled) v[u] *= a2[p];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (i0 + u * S < n) frc[(size_t)(i0 + u * S) * rec_n + q] = (T)v[u];
+    }
+}
+
+// lists the staged candidates (n of them) whose stencil reaches this wave's
+// 4 x 4 x 4 sub-block; returns their number. An entry holds the record's value
+// index (16 bits: the stage has fewer than 2^16 values) and the base relative
+// to the sub-block, in (-P, 4) (K >= 16 > P + 3: one offset only), so that the
+// sums need no second look at the record's base. The list is written and read
+// by this wave only (LDS accesses of a wave complete in order).
+template <typename T, int P>
+__device__ __forceinline__ int spread_hits(int n, const T* stage, int rec_n, int K, int wave,
+                                           int lane, unsigned* list) {
+    int cnt = 0;
+    for (int c0 = 0; c0 < n; c0 += 64) {
+        const int c = c0 + lane;
+        bool hit = c < n;
+        unsigned entry = (unsigned)(c * rec_n);
+        if (hit) {
+            const int* rl = reinterpret_cast<const int*>(stage + c * rec_n);
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                int r = wrapk(rl[d] - (d == 0 ? 4 * wave : 0), K);
+                r = r > K - P ? r - K : r;
+                hit = hit && r < 4;
+                entry |= (unsigned)(r + 8) << (16 + 4 * d);
+            }
+        }
+        const unsigned long long m = __ballot(hit);
+        if (hit) list[cnt + __popcll(m & ((1ull << lane) - 1ull))] = entry;
+        cnt += __popcll(m);
+    }
+    __builtin_amdgcn_wave_barrier();
+    return cnt;
+}
+
+// value index of a listed candidate's weight for coordinate x of the sub-block
+// along dimension d (0 <= x < 4; a zero outside the stencil)
+template <typename T, int P>
+__device__ __forceinline__ int sten_at(int x, unsigned entry, int d) {
+    typedef Sten<T, P> St;
+    return (int)(entry & 0xffffu) + (St::OW + d * St::RUN + 8 + x) -
+           (int)((entry >> (16 + 4 * d)) & 15u);
+}
+
+template <typename T, int P, int NQ, bool BLK>
+__global__ void __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(BLK ? 4 : (sizeof(T) == 4 ? 6 : 5))))
+spread_mx_kernel(int K, int nsx, const int2* __restrict__ blk, const int* __restrict__ ids,
+                 const T* __restrict__ sten, const double* __restrict__ a2,
+                 const double* __restrict__ X, const T* __restrict__ Xb, int npos, int b,
+                 int ncbw, int NC, int cap, T* __restrict__ mesh) {
+    typedef Sten<T, P> St;
+    typedef SpreadTile<T, NQ> Tile;
+    typedef T V4 __attribute__((ext_vector_type(4)));
+    // four or two points of a mesh row: rows start on two values where K % 4 != 0
+    typedef T V4m __attribute__((ext_vector_type(4), aligned(2 * sizeof(T))));
+    typedef T V2m __attribute__((ext_vector_type(2), aligned(2 * sizeof(T))));
+    constexpr int OF = St::N, REC = spread_slot<T>(OF, NQ), NT = (NQ + 15) / 16;
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    // record: wx[P] 0, wy[P] 0, wz[P] 0, base - block origin (3 ints in the
-    // slots of bx by bz), pad, f[NQ] (16-byte aligned)
-    constexpr int OWY = P + 1, OWZ = 2 * (P + 1), OB = 3 * (P + 1);
-    constexpr int OF = (OB + 3 + 3) & ~3;
-    constexpr int REC = SGF ? OF : OF + NQ;
-    static_assert(NQ % 4 == 0, "NQ must be a multiple of 4");
-    static_assert(!SGF || BLK, "scalar force reads need the blocked copy");
-    static_assert(!MF || (BLK && !SGF && NQ == 48 && sizeof(T) == 4),
-                  "matrix-core sums: FP32, blocked staged forces, 48 meshes");
-    const T* __restrict__ xbb = Xb + (size_t)byl_of(blockIdx.x + blockIdx.y * gridDim.x,
-                                                    gridDim.x * gridDim.y, gridDim.x) * npos * NQ;
     T* stage = reinterpret_cast<T*>(smem_raw);
-    int* s_list = reinterpret_cast<int*>(stage + (size_t)cap * REC);   // [8][cap]
-    int* s_pid = s_list + 8 * cap;                                       // [cap]
-    // MA: output tile after the stage (16-byte aligned)
-    [[maybe_unused]] T* ma_tile =
-        reinterpret_cast<T*>(smem_raw + ((((size_t)cap * (REC * sizeof(T) + 9 * sizeof(int))) + 15) & ~(size_t)15));
-    __shared__ int s_wave[kPtThreads / 64];
-    __shared__ int s_off[kPtMaxTiles + 1];
-    __shared__ int s_beg[kPtMaxTiles];
+    int* s_pid = reinterpret_cast<int*>(stage + (size_t)cap * REC);            // [cap]
+    unsigned* s_list = reinterpret_cast<unsigned*>(s_pid + cap);               // [8][cap]
+    T* s_tile = reinterpret_cast<T*>(
+        smem_raw + (((size_t)cap * (REC * sizeof(T) + 36) + 15) & ~(size_t)15));
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const unsigned lid = xcd_logical_id(blockIdx.x + blockIdx.y * gridDim.x, gridDim.x * gridDim.y);
     const int bxl = (int)(lid % gridDim.x), byl = (int)(lid / gridDim.x);
+    const int2 seg = blk[bxl];
+    const int ncand = seg.y;
+    const int* __restrict__ list_g = ids + seg.x;
     const int K4 = (K + 3) >> 2;
-    const int sxi = bxl % nsx;
     const int yz = bxl / nsx;
-    const int x0 = sxi * 32, y0 = (yz % K4) * 4, z0 = (yz / K4) * 4;
+    const int org[3] = {(bxl % nsx) * 32, (yz % K4) * 4, (yz / K4) * 4};
+    const int x0 = org[0], y0 = org[1], z0 = org[2];
     const int xlen = min(32, K - x0), ylen = min(4, K - y0), zlen = min(4, K - z0);
-    int r0 = byl * (NQ / NC);
-    int rb = min(NQ / NC, b - r0);
-    int nq = rb * NC;
     const bool wave_on = 4 * wave < xlen;
-    const bool wave_full = 4 * wave + 4 <= xlen;   // else 2 points along x
-    // this lane's point, relative to the block origin
-    const int lx = 4 * wave + (lane & 3), ly = (lane >> 2) & 3, lz = lane >> 4;
-    const int px = x0 + lx, py = y0 + ly, pz = z0 + lz;
-    const bool lane_on = lx < xlen && ly < ylen && lz < zlen;
-    T acc[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; q++) acc[q] = T(0);
-    // MF: result tiles [z plane m][component t]
-    typedef float f4 __attribute__((ext_vector_type(4)));
-    // four points of a mesh row: rows start on 8 bytes where K % 4 != 0
-    typedef float f4m __attribute__((ext_vector_type(4), aligned(8)));
-    typedef float f2m __attribute__((ext_vector_type(2), aligned(8)));
-    auto put4 = [](T* dst, f4 v, bool full) __attribute__((always_inline)) {
-        if (full) *reinterpret_cast<f4m*>(dst) = v;
-        else *reinterpret_cast<f2m*>(dst) = f2m{v.x, v.y};
-    };
-    f4 accm[4][3];
-#pragma unroll
-    for (int m = 0; m < 4; m++)
-#pragma unroll
-        for (int t = 0; t < 3; t++) accm[m][t] = f4{0.f, 0.f, 0.f, 0.f};
-
-    // contributor base tiles (distinct, with wrap): bases in [lo, lo + len);
-    // wave 0 reads the bucket bounds of 64 tiles at a time and scans the
-    // counts into the candidate offsets
-    if (wave == 0) {
-        int first[3], cnt[3];
-        const int lo[3] = {x0 - (P - 1), y0 - (P - 1), z0 - (P - 1)};
-        const int len[3] = {xlen + P - 1, ylen + P - 1, zlen + P - 1};
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            if (len[d] >= K) { first[d] = 0; cnt[d] = ntile; continue; }
-            const int a = (lo[d] >= 0) ? lo[d] / ts : -((-lo[d] + ts - 1) / ts);
-            const int e = lo[d] + len[d] - 1;
-            const int bt = (e >= 0) ? e / ts : -((-e + ts - 1) / ts);
-            cnt[d] = min(bt - a + 1, ntile);
-            first[d] = ((a % ntile) + ntile) % ntile;
-        }
-        const int ntot = cnt[0] * cnt[1] * cnt[2];
-        int run = 0;
-        for (int k0 = 0; k0 < ntot; k0 += 64) {
-            const int k = k0 + lane;
-            int pb = 0, n = 0;
-            if (k < ntot) {
-                const int jx = k % cnt[0], jyz = k / cnt[0];
-                const int jy = jyz % cnt[1], jz = jyz / cnt[1];
-                const int tt = (((first[2] + jz) % ntile) * ntile + (first[1] + jy) % ntile) *
-                                   ntile + (first[0] + jx) % ntile;
-                pb = tile_start[tt];
-                n = tile_start[tt + 1] - pb;
-            }
-            int inc = n;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int t = __shfl_up(inc, o);
-                if (lane >= o) inc += t;
-            }
-            if (k < ntot) {
-                s_beg[k] = pb;
-                s_off[k] = run + inc - n;
-            }
-            run += __shfl(inc, 63);
-        }
-        if (lane == 0) {
-            s_off[ntot] = run;
-            s_wave[0] = ntot;   // tile count, read below before s_wave is reused
-        }
-    }
-    __syncthreads();
-    const int nbt = s_wave[0];
-    const int ncand = s_off[nbt];
-    __syncthreads();
-
-    // accumulate the first n staged candidates
-    auto accumulate = [&](int n) __attribute__((always_inline)) {
-        int* list = s_list + wave * cap;
-        int cnt = 0;
-        if (wave_on) {
-            for (int c0 = 0; c0 < n; c0 += 64) {
-                const int c = c0 + lane;
-                bool hit = false;
-                if (c < n) {
-                    const int* rl = reinterpret_cast<const int*>(stage + (size_t)c * REC + OB);
-                    const int dx = wrapk(rl[0] - 4 * wave, K);
-                    const int dy = wrapk(rl[1], K);
-                    const int dz = wrapk(rl[2], K);
-                    hit = (dx < 4 || K - dx < P) && (dy < 4 || K - dy < P) && (dz < 4 || K - dz < P);
-                }
-                const unsigned long long m = __ballot(hit);
-                if (hit) list[cnt + __popcll(m & ((1ull << lane) - 1ull))] = c;
-                cnt += __popcll(m);
-            }
-        }
-        // the list is written and read by this wave only (LDS accesses of a
-        // wave complete in order)
-        __builtin_amdgcn_wave_barrier();
-        if constexpr (MF) {
-            // A entry of lane l: point (x, y) = (l % 4, (l / 4) % 4) of the
-            // sub-block, candidate l / 16 of the step; B entry: force
-            // component t of column l % 16 of the same candidate. Past the
-            // list end both are 0.
-            const int kq = lane >> 4, jj = lane & 15;
-            const int ax = 4 * wave + (lane & 3), ay = (lane >> 2) & 3;
-            for (int k0 = 0; k0 < cnt; k0 += 4) {
-                const int k = k0 + kq;
-                T wxy = T(0), wz[4] = {T(0), T(0), T(0), T(0)}, bf[3] = {T(0), T(0), T(0)};
-                if (k < cnt) {
-                    const T* rec = stage + (size_t)list[k] * REC;
-                    const int* rl = reinterpret_cast<const int*>(rec + OB);
-                    // offset in the stencil (P, a zero weight, outside)
-                    auto off = [K](int d) __attribute__((always_inline)) {
-                        if constexpr (WRAP) return min(wrapk(d, K), P);
-                        else return (int)min((unsigned)d, (unsigned)P);
-                    };
-                    wxy = rec[off(ax - rl[0])] * rec[OWY + off(ay - rl[1])];
-#pragma unroll
-                    for (int m = 0; m < 4; m++) wz[m] = rec[OWZ + off(m - rl[2])];
-#pragma unroll
-                    for (int t = 0; t < 3; t++) bf[t] = rec[OF + 16 * t + jj];
-                }
-#pragma unroll
-                for (int m = 0; m < 4; m++) {
-                    const T a = wxy * wz[m];
-#pragma unroll
-                    for (int t = 0; t < 3; t++)
-                        accm[m][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, bf[t], accm[m][t], 0, 0, 0);
-                }
-            }
-        } else if constexpr (!WRAP) {
-            // no stencil reaches both ends of the block: the offset of this
-            // lane's point in a candidate's stencil is a plain difference
-            // (out of the stencil: P, a zero weight)
-            for (int k = 0; k < cnt; k++) {
-                const T* rec = stage + (size_t)list[k] * REC;
-                const int* rl = reinterpret_cast<const int*>(rec + OB);
-                const int dx = (int)min((unsigned)(lx - rl[0]), (unsigned)P);
-                const int dy = (int)min((unsigned)(ly - rl[1]), (unsigned)P);
-                const int dz = (int)min((unsigned)(lz - rl[2]), (unsigned)P);
-                const T w = rec[dx] * rec[OWY + dy] * rec[OWZ + dz];
-                if constexpr (SGF) {
-                    const int pid = __builtin_amdgcn_readfirstlane(s_pid[list[k]]);
-                    const T* fp = xbb + (size_t)pid * NQ;
-#pragma unroll
-                    for (int q = 0; q < NQ; q++) acc[q] += w * fp[q];
-                } else {
-#pragma unroll
-                    for (int q = 0; q < NQ; q++) acc[q] += w * rec[OF + q];
-                }
-            }
-        } else {
-            for (int k = 0; k < cnt; k++) {
-                const T* rec = stage + (size_t)list[k] * REC;
-                const int* rl = reinterpret_cast<const int*>(rec + OB);
-                const int dx = min(wrapk(lx - rl[0], K), P);
-                const int dy = min(wrapk(ly - rl[1], K), P);
-                const int dz = min(wrapk(lz - rl[2], K), P);
-                const T w = rec[dx] * rec[OWY + dy] * rec[OWZ + dz];
-                if constexpr (SGF) {
-                    const int pid = __builtin_amdgcn_readfirstlane(s_pid[list[k]]);
-                    const T* fp = xbb + (size_t)pid * NQ;
-#pragma unroll
-                    for (int q = 0; q < NQ; q++) acc[q] += w * fp[q];
-                } else {
-#pragma unroll
-                    for (int q = 0; q < NQ; q++) acc[q] += w * rec[OF + q];
-                }
-            }
-        }
-    };
-
-    int nst = 0;
-    bool staged_all = false;   // MA: the stage holds every candidate
-    int cb = MA ? byl * ncbw : 0;
-    [[maybe_unused]] const int ncb = MA ? min(cb + ncbw, (b + NQ / NC - 1) / (NQ / NC)) : 1;
-    // MA: the next column block starts here (a jump back, not a loop, so
-    // that the other instances compile without one)
-next_column_block:
-    {
-    const int cbl = MA ? cb : byl;
-    if constexpr (MA) {
-        r0 = cb * (NQ / NC);
-        rb = min(NQ / NC, b - r0);
-        nq = rb * NC;
-        __syncthreads();   // every wave is done with the previous block's forces
-    }
-    if (staged_all) {
-        // the staged candidates' forces of this column block
-        constexpr int VW = 16 / sizeof(T);
-        constexpr int NV = NQ / VW;
-        constexpr int U = 4;
-        typedef T VT __attribute__((ext_vector_type(16 / sizeof(T))));
-        const VT* src = reinterpret_cast<const VT*>(Xb + (size_t)cbl * npos * NQ);
-        for (int e0 = threadIdx.x; e0 < nst * NV; e0 += kPtThreads * U) {
-            VT v[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const int e = e0 + u * kPtThreads;
-                v[u] = VT(0);
-                if (e < nst * NV) v[u] = src[(size_t)s_pid[e / NV] * NV + (e - (e / NV) * NV)];
-            }
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const int e = e0 + u * kPtThreads;
-                if (e < nst * NV)
-                    *reinterpret_cast<VT*>(stage + (size_t)(e / NV) * REC + OF + (e - (e / NV) * NV) * VW) = v[u];
-            }
-        }
-        __syncthreads();
-        accumulate(nst);
-    } else {
-    nst = 0;
-    bool flushed = false;
-    for (int c0 = 0; c0 < ncand; c0 += kPtThreads) {
-        const int ci = c0 + (int)threadIdx.x;
-        int is = -1, b3[3] = {0, 0, 0};
-        bool take = false;
-        if (ci < ncand) {
-            // the last tile whose offset is <= ci (empty tiles skipped)
-            int k = 0, hi = nbt - 1;
-            while (k < hi) {
-                const int mid = (k + hi + 1) >> 1;
-                if (s_off[mid] <= ci) k = mid;
-                else hi = mid - 1;
-            }
-            is = s_beg[k] + (ci - s_off[k]);
-            b3[0] = base[3 * is]; b3[1] = base[3 * is + 1]; b3[2] = base[3 * is + 2];
-            const int dx = wrapk(b3[0] - x0, K);
-            const int dy = wrapk(b3[1] - y0, K);
-            const int dz = wrapk(b3[2] - z0, K);
-            take = (dx < xlen || K - dx < P) && (dy < ylen || K - dy < P) &&
-                   (dz < zlen || K - dz < P);
-        }
-        int tot;
-        const int slot = wg_compact(take, s_wave, &tot);
-        for (int done = 0; done < tot;) {
-            if (nst == cap) {
-                __syncthreads();
-                accumulate(nst);
-                __syncthreads();
-                nst = 0;
-                flushed = true;
-            }
-            const int taken = min(cap - nst, tot - done);
-            const int first = nst;
-            if (take && slot >= done && slot < done + taken) {
-                const int sl = first + slot - done;
-                T* rec = stage + (size_t)sl * REC;
-                T w[P];
-                // base relative to the block origin, as an int in (-P, K - P]
-                int* rl = reinterpret_cast<int*>(rec + OB);
-                const int org[3] = {x0, y0, z0};
-#pragma unroll
-                for (int d = 0; d < 3; d++) {
-                    bspline_weights_r<T, P>(frac[3 * is + d], w);
-#pragma unroll
-                    for (int k = 0; k < P; k++) rec[d * (P + 1) + k] = w[k];
-                    rec[d * (P + 1) + P] = T(0);
-                    const int r = wrapk(b3[d] - org[d], K);
-                    rl[d] = r > K - P ? r - K : r;
-                }
-                s_pid[sl] = is;
-            }
-            __syncthreads();
-            if constexpr (SGF) {
-                // forces are read in the accumulation
-            } else if constexpr (BLK) {
-                // NQ contiguous values per slot, 16 bytes per load, the loads
-                // of a thread in flight together
-                constexpr int VW = 16 / sizeof(T);
-                constexpr int NV = NQ / VW;
-                constexpr int U = 4;
-                typedef T VT __attribute__((ext_vector_type(16 / sizeof(T))));
-                const VT* src = reinterpret_cast<const VT*>(Xb + (size_t)cbl * npos * NQ);
-                for (int e0 = threadIdx.x; e0 < taken * NV; e0 += kPtThreads * U) {
-                    VT v[U];
-#pragma unroll
-                    for (int u = 0; u < U; u++) {
-                        const int e = e0 + u * kPtThreads;
-                        v[u] = VT(0);
-                        if (e < taken * NV) {
-                            const int sl = first + e / NV;
-                            v[u] = src[(size_t)s_pid[sl] * NV + (e - (e / NV) * NV)];
-                        }
-                    }
-#pragma unroll
-                    for (int u = 0; u < U; u++) {
-                        const int e = e0 + u * kPtThreads;
-                        if (e < taken * NV) {
-                            const int sl = first + e / NV, vv = e - (e / NV) * NV;
-                            *reinterpret_cast<VT*>(stage + (size_t)sl * REC + OF + vv * VW) = v[u];
-                        }
-                    }
-                }
-            } else {
-                // forces of the new slots: slot q holds rhs r, component c
-                // (mono: q = 3 r + c; poly: q = 6 r + c for f, 6 r + 3 + c
-                // for a^2 f); the loads of a thread in flight together
-                constexpr int U = 4;
-                for (int e0 = threadIdx.x; e0 < taken * NQ; e0 += kPtThreads * U) {
-                    T fv[U];
-#pragma unroll
-                    for (int u = 0; u < U; u++) {
-                        const int idx = e0 + u * kPtThreads;
-                        fv[u] = T(0);
-                        if (idx < taken * NQ) {
-                            const int sl = first + idx / NQ, q = idx % NQ;
-                            const int p = s_pid[sl];
-                            const int r = q / NC, cc = q - r * NC;
-                            if (r < rb) {
-                                const double x = X[(size_t)(3 * p + cc % 3) * b + r0 + r];
-                                fv[u] = (T)((cc >= 3) ? x * a2[p] : x);
-                            }
-                        }
-                    }
-#pragma unroll
-                    for (int u = 0; u < U; u++) {
-                        const int idx = e0 + u * kPtThreads;
-                        if (idx < taken * NQ)
-                            stage[(size_t)(first + idx / NQ) * REC + OF + idx % NQ] = fv[u];
-                    }
-                }
-            }
-            nst += taken;
-            done += taken;
-        }
-        __syncthreads();
-    }
-    __syncthreads();
-    accumulate(nst);
-    // the mesh tiles below reuse the stage
-    staged_all = MA && !flushed && !tiled_out;
-    }
-    // Mesh stores. Default: each lane stores its own point (a wave writes
-    // 16-byte pieces of 16 rows; the eight waves' pieces of a row reach HBM
-    // about 1.4x). tiled_out: the meshes leave through LDS (the stage is free
-    // now), QC at a time (up to 48 KB): each wave writes its 4 x 4 x 4
-    // sub-block into a 16-row x 32 tile per mesh, then every 32 threads store
-    // one whole x row (128 bytes for xlen = 32). Exactly the mesh bytes reach
-    // HBM, but the extra LDS round trip and barriers cost about 5 % of the
-    // kernel at K = 128 and 100 columns, so it is not the default.
-    constexpr int QC = (NQ * 512 * (int)sizeof(T) <= 49152) ? NQ : NQ / 2;
-    static_assert(NQ % QC == 0, "mesh groups must divide NQ");
-    T* tile = stage;
     const size_t K3 = (size_t)K * K * K;
-    if constexpr (MF) {
-        // result register v of lane l holds row 4 (l / 16) + v of a tile:
-        // x = v, y = l / 16 of z plane m; column l % 16 of component t
-        if (MA && !tiled_out) {
-            // through the LDS tiles: wave w writes x in [4w, 4w + 4) of every
-            // (column, row); thread e then stores 16 bytes of row e / 8. The
-            // rounds alternate between two tiles, so one barrier per round
-            // suffices: a thread writes a tile again only after the next
-            // round's barrier, which every thread reaches after its reads.
-            const int jj = lane & 15, sy = lane >> 4;
-            const int e = threadIdx.x;
-            const int sj = e >> 5, sr = (e >> 3) & 3, sx = (e & 7) * 4;
+    V4 acc[4][NT];
+    auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
-            for (int m = 0; m < 4; m++)
+        for (int m = 0; m < 4; m++)
 #pragma unroll
-                for (int t = 0; t < 3; t++) {
-                    T* tb = ma_tile + ((m * 3 + t) & 1) * (16 * kMaTileStride);
-                    if (wave_on)
-                        *reinterpret_cast<f4*>(tb + jj * kMaTileStride + sy * 32 + 4 * wave) =
-                            accm[m][t];
-                    __syncthreads();
-                    if (sj < rb && sx < xlen && sr < ylen && m < zlen) {
-                        const f4 v =
-                            *reinterpret_cast<const f4*>(tb + sj * kMaTileStride + sr * 32 + sx);
-                        put4(mesh + ((size_t)(r0 + sj) * 3 + t) * K3 +
-                                 ((size_t)(z0 + m) * K + (y0 + sr)) * K + x0 + sx,
-                             v, sx + 4 <= xlen);
-                    }
-                }
+            for (int t = 0; t < NT; t++) acc[m][t] = V4(T(0));
+    };
+    clear();
+    // adds the first n staged candidates, listed anew or as they were
+    int cnt = 0;
+    auto accumulate = [&](int n, bool relist) __attribute__((always_inline)) {
+        if (!wave_on) return;
+        unsigned* list = s_list + wave * cap;
+        if (relist) cnt = spread_hits<T, P>(n, stage, REC, K, wave, lane, list);
+        if (cnt == 0) return;
+        // A entry of lane l: point (x, y) = (l % 4, (l / 4) % 4) of the
+        // sub-block, candidate l / 16 of the step (weight 0 past the list's
+        // end); B entry: force value 16 t + l % 16 of the same candidate.
+        const int kq = lane >> 4, jj = lane & 15, ax = lane & 3, ay = (lane >> 2) & 3;
+        unsigned next = list[min(kq, cnt - 1)];
+        for (int k0 = 0; k0 < cnt; k0 += 4) {
+            const unsigned entry = next;
+            next = list[min(k0 + 4 + kq, cnt - 1)];
+            T wxy = stage[sten_at<T, P>(ax, entry, 0)] * stage[sten_at<T, P>(ay, entry, 1)];
+            wxy = k0 + kq < cnt ? wxy : T(0);
+            const T* wz = stage + sten_at<T, P>(0, entry, 2);
+            const T* f = stage + (entry & 0xffffu) + OF + jj;
+            T bf[NT];
 #pragma unroll
-            for (int m = 0; m < 4; m++)
+            for (int t = 0; t < NT; t++)
+                bf[t] = (NQ % 16 == 0 || 16 * t + jj < NQ) ? f[16 * t] : T(0);
 #pragma unroll
-                for (int t = 0; t < 3; t++) accm[m][t] = f4{0.f, 0.f, 0.f, 0.f};
-            if (++cb < ncb) goto next_column_block;
-            return;
-        }
-        if (!tiled_out) {
-            const int jj = lane & 15, sy = lane >> 4;
-            if (wave_on && jj < rb && sy < ylen) {
+            for (int m = 0; m < 4; m++) {
+                const T a = wxy * wz[m];
 #pragma unroll
-                for (int m = 0; m < 4; m++)
-#pragma unroll
-                    for (int t = 0; t < 3; t++)
-                        if (m < zlen)
-                            put4(mesh + ((size_t)(r0 + jj) * 3 + t) * K3 +
-                                     ((size_t)(z0 + m) * K + (y0 + sy)) * K + x0 + 4 * wave,
-                                 accm[m][t], wave_full);
+                for (int t = 0; t < NT; t++) acc[m][t] = mfma16(a, bf[t], acc[m][t]);
             }
-            if constexpr (MA) {
-#pragma unroll
-                for (int m = 0; m < 4; m++)
-#pragma unroll
-                    for (int t = 0; t < 3; t++) accm[m][t] = f4{0.f, 0.f, 0.f, 0.f};
-                if (++cb < ncb) goto next_column_block;
-            }
-            return;
         }
-    }
-    if constexpr (MA && !MF) {
-        // vector-ALU sums (FP64): per-lane stores, then the next column block
-        if (!tiled_out) {
-            if (lane_on) {
-                const size_t pt = ((size_t)pz * K + py) * K + px;
-                constexpr int RBB = NQ / 3;
-#pragma unroll
-                for (int q = 0; q < NQ; q++) {
-                    const int c = q / RBB, r = q % RBB;
-                    if (r < rb) mesh[((size_t)(r0 + r) * 3 + c) * K3 + pt] = acc[q];
-                }
+    };
+    constexpr int RBB = BLK ? NQ / 3 : 1;   // columns per block
+    int cb = BLK ? byl * ncbw : 0;
+    const int ncb = BLK ? min(cb + ncbw, (b + RBB - 1) / RBB) : 1;
+    bool staged_all = false;   // the stage holds every candidate
+    for (;;) {
+        const T* frc = BLK ? Xb + (size_t)cb * npos * NQ : nullptr;
+        constexpr int NV = BLK ? NQ / St::V : 0;
+        for (int c0 = 0;; c0 += cap) {
+            const int n = min(cap, ncand - c0);
+            if (BLK && staged_all)
+                spread_restage<T, NQ>(n, s_pid, frc, REC, stage + OF);
+            else
+                spread_stage<T, P, NV>(n, list_g + c0, sten, frc, org, K, REC, stage, s_pid);
+            __syncthreads();
+            if constexpr (!BLK) {
+                spread_stage_packed<T, NQ>(n, s_pid, X, a2, b, NC, 0, REC, stage + OF);
+                __syncthreads();
             }
-#pragma unroll
-            for (int q = 0; q < NQ; q++) acc[q] = T(0);
-            if (++cb < ncb) goto next_column_block;
-            return;
+            accumulate(n, !staged_all);
+            if (c0 + cap >= ncand) break;
+            __syncthreads();   // a full stage is summed and emptied
         }
-    }
-    if (!tiled_out) {
-        if (!lane_on) return;
-        const size_t pt = ((size_t)pz * K + py) * K + px;
+        staged_all = ncand <= cap;
+        // stores. FP32: result register v of lane l holds row 4 (l / 16) + v,
+        // x = v and y = l / 16; FP64: row l / 16 + 4 v, x = l / 16 and y = v;
+        // force value 16 t + l % 16 of z plane m
+        const int jj = lane & 15, hi = lane >> 4;
+        const int e = threadIdx.x;
+        const int sx = (e & 7) * 4, sr = (e >> 3) & 3;
+        const int sj = (e >> 5) % Tile::cols, sm = (e >> 5) / Tile::cols;
 #pragma unroll
-        for (int q = 0; q < NQ; q++) {
-            size_t mi;
-            bool on;
-            if constexpr (BLK) {
-                constexpr int RBB = NQ / 3;
-                const int c = q / RBB, r = q % RBB;
-                on = r < rb;
-                mi = (size_t)(r0 + r) * 3 + c;
-            } else {
-                on = q < nq;
-                mi = (size_t)r0 * NC + q;
-            }
-            if (on) mesh[mi * K3 + pt] = acc[q];
-        }
-        return;
-    }
-    __syncthreads();   // every wave is done reading the stage
+        for (int t = 0; t < NT; t++)
 #pragma unroll
-    for (int q0 = 0; q0 < NQ; q0 += QC) {
-        if (wave_on) {
-            if constexpr (MF) {
-                const int jj = lane & 15, sy = lane >> 4;
+            for (int m0 = 0; m0 < 4; m0 += Tile::planes) {
+                T* tb = s_tile + (Tile::bufs == 2 ? ((t * 4 + m0) & 1) : 0) *
+                                     (Tile::planes * Tile::cols * kTileRow);
+                if (wave_on && jj < Tile::cols) {
 #pragma unroll
-                for (int m = 0; m < 4; m++)
+                    for (int m = m0; m < m0 + Tile::planes; m++) {
+                        T* to = tb + ((m - m0) * Tile::cols + jj) * kTileRow + 4 * wave;
+                        if constexpr (sizeof(T) == 4) {
+                            *reinterpret_cast<V4*>(to + hi * 32) = acc[m][t];
+                        } else {
 #pragma unroll
-                    for (int t = 0; t < 3; t++) {
-                        const int qq = 16 * t + jj - q0;
-                        if (qq >= 0 && qq < QC) {
-#pragma unroll
-                            for (int v = 0; v < 4; v++)
-                                tile[(qq * 16 + m * 4 + sy) * 32 + 4 * wave + v] = accm[m][t][v];
+                            for (int v = 0; v < 4; v++) to[v * 32 + hi] = acc[m][t][v];
                         }
                     }
-            } else {
-#pragma unroll
-                for (int qq = 0; qq < QC; qq++) tile[(qq * 16 + lz * 4 + ly) * 32 + lx] = acc[q0 + qq];
+                }
+                __syncthreads();
+                const int q = 16 * t + sj, m = m0 + sm;
+                int mi;
+                bool on;
+                if constexpr (BLK) {
+                    const int r = cb * RBB + q % RBB;
+                    on = q < NQ && r < b;
+                    mi = r * 3 + q / RBB;
+                } else {
+                    on = q < b * NC;
+                    mi = q;
+                }
+                if (on && sm < Tile::planes && sx < xlen && sr < ylen && m < zlen) {
+                    const V4 v = *reinterpret_cast<const V4*>(
+                        tb + (sm * Tile::cols + sj) * kTileRow + sr * 32 + sx);
+                    T* dst = mesh + (size_t)mi * K3 + ((size_t)(z0 + m) * K + (y0 + sr)) * K + x0 + sx;
+                    if (sx + 4 <= xlen) *reinterpret_cast<V4m*>(dst) = v;
+                    else *reinterpret_cast<V2m*>(dst) = V2m{v.x, v.y};
+                }
+                if (Tile::bufs == 1) __syncthreads();
             }
+        if (++cb >= ncb) return;
+        clear();
+        // two tiles: a thread may be a round ahead, in the sums' LDS even more;
+        // every wave is done with this column block's forces
+        __syncthreads();
+    }
+}
+
+// The same sums on the vector ALUs, kept as the comparison form: lane = point
+// (x = l % 4, y = (l / 4) % 4, z = l / 16 of the wave's sub-block), kVecQ
+// meshes in registers, one candidate at a time, forces from the packed input.
+constexpr int kVecQ = 16;
+
+template <typename T, int P>
+__global__ void __launch_bounds__(kPtThreads)
+spread_vec_kernel(int K, int nsx, const int2* __restrict__ blk, const int* __restrict__ ids,
+                  const T* __restrict__ sten, const double* __restrict__ a2,
+                  const double* __restrict__ X, int b, int NC, int cap, T* __restrict__ mesh) {
+    typedef Sten<T, P> St;
+    constexpr int OF = St::N, REC = spread_slot<T>(OF, kVecQ);
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    T* stage = reinterpret_cast<T*>(smem_raw);
+    int* s_pid = reinterpret_cast<int*>(stage + (size_t)cap * REC);
+    unsigned* s_list = reinterpret_cast<unsigned*>(s_pid + cap);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int bxl = blockIdx.x, q0 = blockIdx.y * kVecQ;
+    const int2 seg = blk[bxl];
+    const int K4 = (K + 3) >> 2;
+    const int yz = bxl / nsx;
+    const int org[3] = {(bxl % nsx) * 32, (yz % K4) * 4, (yz / K4) * 4};
+    const int lx = 4 * wave + (lane & 3), ly = (lane >> 2) & 3, lz = lane >> 4;
+    T acc[kVecQ];
+#pragma unroll
+    for (int q = 0; q < kVecQ; q++) acc[q] = T(0);
+    for (int c0 = 0; c0 < seg.y; c0 += cap) {
+        const int n = min(cap, seg.y - c0);
+        spread_stage<T, P, 0>(n, ids + seg.x + c0, sten, nullptr, org, K, REC, stage, s_pid);
+        __syncthreads();
+        spread_stage_packed<T, kVecQ>(n, s_pid, X, a2, b, NC, q0, REC, stage + OF);
+        __syncthreads();
+        unsigned* list = s_list + wave * cap;
+        const int cnt = spread_hits<T, P>(n, stage, REC, K, wave, lane, list);
+        for (int k = 0; k < cnt; k++) {
+            const unsigned entry = list[k];
+            const T* rec = stage + (entry & 0xffffu);
+            const T w = stage[sten_at<T, P>(lane & 3, entry, 0)] *
+                        stage[sten_at<T, P>(ly, entry, 1)] * stage[sten_at<T, P>(lz, entry, 2)];
+#pragma unroll
+            for (int q = 0; q < kVecQ; q++) acc[q] = fma(w, rec[OF + q], acc[q]);
         }
         __syncthreads();
-        for (int e = threadIdx.x; e < QC * 512; e += kPtThreads) {
-            const int x = e & 31, rw = (e >> 5) & 15, qq = e >> 9;
-            const int q = q0 + qq;
-            size_t mi;
-            bool on;
-            if constexpr (BLK) {
-                constexpr int RBB = NQ / 3;
-                const int c = q / RBB, r = q % RBB;
-                on = r < rb;
-                mi = (size_t)(r0 + r) * 3 + c;
-            } else {
-                on = q < nq;
-                mi = (size_t)r0 * NC + q;
-            }
-            if (on && x < xlen && (rw & 3) < ylen && (rw >> 2) < zlen)
-                mesh[mi * K3 + ((size_t)(z0 + (rw >> 2)) * K + (y0 + (rw & 3))) * K + x0 + x] =
-                    tile[e];
-        }
-        __syncthreads();
     }
-    if constexpr (MA) {
-        if constexpr (MF) {
+    const int px = org[0] + lx, py = org[1] + ly, pz = org[2] + lz;
+    if (lx >= 32 || px >= K || py >= K || pz >= K) return;
+    const size_t K3 = (size_t)K * K * K, pt = ((size_t)pz * K + py) * K + px;
 #pragma unroll
-            for (int m = 0; m < 4; m++)
-#pragma unroll
-                for (int t = 0; t < 3; t++) accm[m][t] = f4{0.f, 0.f, 0.f, 0.f};
-        } else {
-#pragma unroll
-            for (int q = 0; q < NQ; q++) acc[q] = T(0);
-        }
-        if (++cb < ncb) goto next_column_block;
-    }
-    }
+    for (int q = 0; q < kVecQ; q++)
+        if (q0 + q < b * NC) mesh[(q0 + q) * K3 + pt] = acc[q];
 }
 
 // ------------------------------------------------------ x transforms -------
@@ -1219,12 +1190,30 @@ void SpmeGpu<T>::create(int npos_, double box_, double xi_, int K_, int porder_,
         if (c >= porder - 1 && K % c == 0 && K / c >= 3) { ts = c; break; }
     SDT_REQUIRE(ts > 0, SDT_EINVAL, "no spread tile size divides the mesh dimension");
     ntile = K / ts;
-    // contributor bucket tiles of a 32 x 4 x 4 spread block: bases in
-    // intervals of length min(32, K) + P - 1 (x) and P + 3 (y, z)
-    auto tiles = [&](int len) { return std::min(ntile, (len + ts - 1) / ts + 1); };
-    SDT_REQUIRE(tiles(std::min(32, K) + porder - 1) * tiles(porder + 3) * tiles(porder + 3) <=
-                    kPtMaxTiles,
-                SDT_EINVAL, "spread: too many contributor tiles for this order and mesh");
+    // tile rows of a 32 x 4 x 4 spread block's window, two ranges each
+    const int trow = std::min(ntile, (porder + 3 + ts - 1) / ts + 1);
+    SDT_REQUIRE(2 * trow * trow <= kListRanges, SDT_EINVAL,
+                "spread: too many contributor tiles for this order and mesh");
+    // blocks that one stencil can reach: the most over its base points, per
+    // dimension (blocks of 32 or 4 points, the last one partial)
+    auto reach = [&](int len) {
+        int most = 0;
+        for (int b0 = 0; b0 < K; b0++) {
+            std::vector<int> got;
+            for (int q = 0; q < porder; q++) {
+                const int bl = ((b0 + q) % K) / len;
+                if (std::find(got.begin(), got.end(), bl) == got.end()) got.push_back(bl);
+            }
+            most = std::max(most, (int)got.size());
+        }
+        return (long long)most;
+    };
+    const long long ids_cap = reach(32) * reach(4) * reach(4) * npos;
+    SDT_REQUIRE(ids_cap < (1LL << 31), SDT_EINVAL, "spread: too many particles");
+    const size_t nblocks = (size_t)ceil_div(K, 32) * ceil_div(K, 4) * ceil_div(K, 4);
+    d_nids.reserve(1);
+    d_ids.reserve((size_t)ids_cap);
+    d_blk.reserve(nblocks);
     std::vector<double> tw(2 * K);
     for (int j = 0; j < K; j++) {
         tw[2 * j] = cos(-2.0 * M_PI * j / K);
@@ -1241,6 +1230,10 @@ void SpmeGpu<T>::create(int npos_, double box_, double xi_, int K_, int porder_,
     }
     d_fac.reserve(K);
     SDT_HIP_CHECK(sync_memcpy(d_fac.get(), bs.data(), sizeof(double) * K, hipMemcpyHostToDevice));
+    // the stencil records: Sten<T, P>::N values
+    const int sv = 16 / (int)sizeof(T);
+    sten_n = (sv + 3 * (porder + 3) + 3 + sv - 1) / sv * sv;
+    d_sten.reserve((size_t)sten_n * npos);
     d_frac.reserve(3 * (size_t)npos);
     d_base.reserve(3 * (size_t)npos);
     d_frac_u.reserve(3 * (size_t)npos);
@@ -1276,27 +1269,39 @@ template <typename T>
 void SpmeGpu<T>::gather_sorted(const int* d_perm, const double* d_pos, const double* d_rdi,
                                const int* d_tile_start_in, hipStream_t s) {
     (void)d_pos;
-    hipLaunchKernelGGL((spme_gather_kernel<T>), dim3(ceil_div(npos, 256)), dim3(256), 0, s, npos,
-                       d_perm, d_frac_u.get(), d_base_u.get(), d_rdi, d_frac.get(), d_base.get(),
-                       poly ? d_a2.get() : (double*)nullptr);
+    const int nsx = (K + 31) / 32;
+    const int nblocks = nsx * (int)ceil_div(K, 4) * (int)ceil_div(K, 4);
+#define SDT_GATHER(PP)                                                                        \
+    case PP:                                                                                  \
+        hipLaunchKernelGGL((spme_gather_kernel<T, PP>), dim3(ceil_div(npos, 256)), dim3(256), 0, s, \
+                           npos, d_perm, d_frac_u.get(), d_base_u.get(), d_rdi, d_sten.get(), \
+                           d_frac.get(), d_base.get(), poly ? d_a2.get() : (double*)nullptr, d_nids.get()); \
+        hipLaunchKernelGGL((spread_list_kernel<PP>), dim3(ceil_div(nblocks, kListWaves)),     \
+                           dim3(64 * kListWaves), 0, s, K, ts, ntile, nsx, nblocks,           \
+                           d_tile_start_in, d_base.get(), d_nids.get(), d_blk.get(),          \
+                           d_ids.get());                                                      \
+        break;
+    switch (porder) { SDT_GATHER(4) SDT_GATHER(5) SDT_GATHER(6) SDT_GATHER(7) SDT_GATHER(8) }
+#undef SDT_GATHER
     SDT_HIP_CHECK(hipGetLastError());
     const size_t nt3 = (size_t)ntile * ntile * ntile + 1;
     SDT_HIP_CHECK(hipMemcpyAsync(d_tile_start.get(), d_tile_start_in, sizeof(int) * nt3,
                                  hipMemcpyDeviceToDevice, s));
 }
 
-// meshes per workgroup of the spread: 4 or 12 when few are needed
+// force values per workgroup of the spread: 4 or 16 when few meshes are
+// needed, else a column block of 16 (FP32) or 8 (FP64) columns
 template <typename T>
-static int pt_meshes(int b, int NC) {
+static int spread_values(int b, int NC) {
     if (b * NC <= 4) return 4;
-    return (b * NC <= 12) ? 12 : (sizeof(T) == 4 ? 48 : 24);
+    return (b * NC <= 16) ? 16 : (sizeof(T) == 4 ? 48 : 24);
 }
 
 template <typename T>
 int SpmeGpu<T>::blocked_cols(int b) const {
     if (poly) return 0;
-    const int NQ = pt_meshes<T>(b, 3);
-    return NQ <= 12 ? 0 : NQ / 3;
+    const int NQ = spread_values<T>(b, 3);
+    return NQ <= 16 ? 0 : NQ / 3;
 }
 
 // Xs[cb][j][c][r], RC columns per block and zero beyond the last: the spread's
@@ -1331,21 +1336,33 @@ void SpmeGpu<T>::spread(int b, const double* X, hipStream_t s, const T* xb) {
                 "spread: no blocked input for this configuration");
     const SpmeTuning& tn = tune[width_class(b)];
     constexpr int NQL = sizeof(T) == 4 ? 48 : 24;
-    int NC = poly ? 6 : 3;
-    const int NQ = pt_meshes<T>(b, NC);
+    const int NC = poly ? 6 : 3;
+    const int NQ = spread_values<T>(b, NC);
     const int fr = spread_form & 3;
-    // Wide launches read a blocked copy and take the column blocks of a mesh
-    // block in turn. FP32 sums on the matrix cores (K = 128, 100 columns:
-    // 1.06 ms against 2.17 ms for the vector-ALU sums with scalar force
-    // reads, the same sums to the bit; unequal radii, 13 columns at K = 96:
-    // 0.10 against 0.19 ms; 8 columns at K = 216: 0.62 against 0.82 ms), FP64
-    // on the vector ALUs. K = 90, 100 FP32 columns: 0.40 ms, 16 FP64 columns:
-    // 0.14 ms (1.68 and 0.56 ms for a tile-owner form that kept mesh sides
-    // other than multiples of 4). Forms override this for tests.
-    int cols = b;
-    if (NQ == NQL && xb == nullptr && (sizeof(T) == 4 || !poly)) {
-        cols = poly ? 2 * b : b;
-        constexpr int RC = NQL / 3;
+    const int nsx = (K + 31) / 32;
+    const unsigned nblocks = nsx * ceil_div(K, 4) * ceil_div(K, 4);
+    if (fr == 1 || fr == 2) {
+        // the vector-ALU comparison form
+        const size_t slot = spread_slot_bytes<T>(sten_n, kVecQ);
+        const int cap = (int)(48 * 1024 / slot);
+        const dim3 grid(nblocks, ceil_div(b * NC, kVecQ));
+#define SDT_VEC(PP)                                                                            \
+    case PP:                                                                                   \
+        hipLaunchKernelGGL((spread_vec_kernel<T, PP>), grid, dim3(kPtThreads), cap * slot, s, \
+                           K, nsx, d_blk.get(), d_ids.get(), d_sten.get(), d_a2.get(), X, b,  \
+                           NC, cap, d_real.get());                                            \
+        break;
+        switch (porder) { SDT_VEC(4) SDT_VEC(5) SDT_VEC(6) SDT_VEC(7) SDT_VEC(8) }
+#undef SDT_VEC
+        SDT_HIP_CHECK(hipGetLastError());
+        return;
+    }
+    // Wide launches read a blocked copy, their own where the real space's is
+    // not there
+    const bool wide = NQ == NQL;
+    const int cols = wide && poly ? 2 * b : b;
+    constexpr int RC = NQL / 3;
+    if (wide && xb == nullptr) {
         const int nblk = ceil_div(cols, RC);
         const long long n = (long long)nblk * npos * 3 * RC;
         d_xs.reserve((size_t)n);
@@ -1359,74 +1376,40 @@ void SpmeGpu<T>::spread(int b, const double* X, hipStream_t s, const T* xb) {
         SDT_HIP_CHECK(hipGetLastError());
         xb = d_xs.get();
     }
-    if (xb != nullptr) NC = 3;   // the copy's columns have three meshes each
-    const bool mf = xb != nullptr && sizeof(T) == 4 && (fr == 0 || fr == 3);
-    const bool sgf = xb != nullptr && sizeof(T) == 4 && !mf && fr != 1;
-    const int rec = ((3 * (porder + 1) + 3 + 3) & ~3) + (sgf ? 0 : NQ);
-    // few meshes: a 48 KB stage leaves room for three workgroups per CU;
-    // 60 KB for the matrix-core form, whose two output tiles (16.5 KB) also
-    // fit two workgroups per CU
-    const int stage_bytes = tn.spread_stage_kb > 0
-                                ? tn.spread_stage_kb * 1024
-                                : (NQ <= 12 ? 48 * 1024 : (mf ? 60 * 1024 : 65536));
-    const int cap = (int)(stage_bytes / (rec * sizeof(T) + 9 * sizeof(int)));
-    // the output tiles reuse the stage's LDS: all meshes, or half of
-    // them above 48 KB (the allocation is at least that)
-    const size_t tile = (size_t)NQ * 512 * sizeof(T);
-    size_t lds = std::max((size_t)cap * (rec * sizeof(T) + 9 * sizeof(int)),
-                          tile <= 49152 ? tile : tile / 2);
-    if (mf && !(spread_form & 4))
-        lds = (((size_t)cap * (rec * sizeof(T) + 9 * sizeof(int)) + 15) & ~(size_t)15) +
-              kMaTileBytes;
-    const int nsx = (K + 31) / 32;
-    const unsigned nblocks = nsx * ceil_div(K, 4) * ceil_div(K, 4);
-    const int ncb = ceil_div(cols, NQ / NC);
+    // stage: two workgroups per CU beside the output tiles for wide launches,
+    // four (FP32, NQ = 4), three or (FP64 with 16 values) two for narrow ones
+    const size_t slot = spread_slot_bytes<T>(sten_n, NQ);
+    const size_t tile = NQ == 4 ? SpreadTile<T, 4>::bytes : SpreadTile<T, 16>::bytes;
+    const int stage_kb = tn.spread_stage_kb > 0 ? tn.spread_stage_kb
+                                                : (wide ? 62
+                                                        : (sizeof(T) == 4 ? (NQ == 4 ? 31 : 35)
+                                                                          : (NQ == 4 ? 35 : 62)));
+    const int cap = (int)(stage_kb * 1024 / slot);
+    const size_t lds = ((cap * slot + 15) & ~(size_t)15) + tile;
     // column blocks a workgroup takes in turn: all of them where the mesh
     // blocks alone fill the chip twice over (two workgroups per CU), fewer on
-    // small meshes; one with scalar force reads, and in the forms that ask
-    // for it
+    // small meshes; one in form 3
+    const int ncb = wide ? ceil_div(cols, RC) : 1;
     int ncbw = 1;
-    if (xb != nullptr && !sgf && (fr == 0 || (spread_form & 8)))
+    if (fr == 0 || (spread_form & 8))
         ncbw = ceil_div(ncb, std::min<unsigned>(ncb, ceil_div(1024, nblocks)));
     const dim3 grid(nblocks, ceil_div(ncb, ncbw));
-#define SDT_SPREAD_PWS(PP, QQ, BB, WW, SS, MM)                                                 \
-    hipLaunchKernelGGL((spread_pt_kernel<T, PP, QQ, BB, WW, SS, MM>), grid, dim3(kPtThreads),  \
-                       lds, s, K, ts, ntile, nsx, d_tile_start.get(), d_frac.get(),           \
-                       d_base.get(), poly ? d_a2.get() : (double*)nullptr, X, xb, npos, cols, \
-                       ncbw, NC, cap, d_real.get(), (spread_form & 4) ? 1 : 0)
-#define SDT_SPREAD_PW(PP, QQ, BB, WW)                                                          \
+#define SDT_SPREAD_Q(PP, QQ, BB)                                                               \
     do {                                                                                      \
-        if constexpr (BB && sizeof(T) == 4) {                                                 \
-            if (sgf) SDT_SPREAD_PWS(PP, QQ, BB, WW, true, false);                              \
-            else if (mf) SDT_SPREAD_PWS(PP, QQ, BB, WW, false, true);                          \
-            else SDT_SPREAD_PWS(PP, QQ, BB, WW, false, false);                                 \
-        } else {                                                                              \
-            SDT_SPREAD_PWS(PP, QQ, BB, WW, false, false);                                      \
-        }                                                                                     \
-    } while (0)
-#define SDT_SPREAD_PT(PP, QQ, BB)                                                              \
-    do {                                                                                      \
-        if (K < 32 + PP - 1) SDT_SPREAD_PW(PP, QQ, BB, true);                                  \
-        else SDT_SPREAD_PW(PP, QQ, BB, false);                                                 \
-    } while (0)
-#define SDT_SPREAD_WIDE(PP)                                                                    \
-    do {                                                                                      \
-        if constexpr (sizeof(T) == 4) SDT_SPREAD_PT(PP, NQL, true);                            \
-        else if (xb) SDT_SPREAD_PT(PP, NQL, true);                                             \
-        else SDT_SPREAD_PT(PP, NQL, false);                                                    \
+        allow_lds((const void*)spread_mx_kernel<T, PP, QQ, BB>, lds);                         \
+        hipLaunchKernelGGL((spread_mx_kernel<T, PP, QQ, BB>), grid, dim3(kPtThreads), lds, s, \
+                           K, nsx, d_blk.get(), d_ids.get(), d_sten.get(), d_a2.get(), X, xb, \
+                           npos, cols, ncbw, NC, cap, d_real.get());                          \
     } while (0)
 #define SDT_SPREAD_P(PP)                                                                       \
     case PP:                                                                                   \
-        if (NQ == 4) SDT_SPREAD_PT(PP, 4, false);                                              \
-        else if (NQ == 12) SDT_SPREAD_PT(PP, 12, false);                                       \
-        else SDT_SPREAD_WIDE(PP);                                                              \
+        if (wide) SDT_SPREAD_Q(PP, NQL, true);                                                 \
+        else if (NQ == 4) SDT_SPREAD_Q(PP, 4, false);                                          \
+        else SDT_SPREAD_Q(PP, 16, false);                                                      \
         break;
     switch (porder) { SDT_SPREAD_P(4) SDT_SPREAD_P(5) SDT_SPREAD_P(6) SDT_SPREAD_P(7) SDT_SPREAD_P(8) }
 #undef SDT_SPREAD_P
-#undef SDT_SPREAD_WIDE
-#undef SDT_SPREAD_PT
-#undef SDT_SPREAD_PW
-#undef SDT_SPREAD_PWS
+#undef SDT_SPREAD_Q
     SDT_HIP_CHECK(hipGetLastError());
 }
 
