@@ -77,8 +77,6 @@ void MobSpmeGpu::init() {
     d_key_.reserve(npos_);
     d_perm_.reserve(npos_);
     d_iperm_.reserve(npos_);
-    const int nt = prec_ == kFP32 ? spme32_->ntile : spme64_->ntile;
-    d_tstart_.reserve((size_t)nt * nt * nt + 1);
     inited_ = true;
 }
 
@@ -120,12 +118,12 @@ void MobSpmeGpu::update(const double* pos, const double* rdi, bool dev) {
         spme64_->prepare(d_pos_.get(), d_key_.get(), s);
         nt = spme64_->ntile;
     }
-    bucket_sort(d_key_.get(), npos_, nt * nt * nt, d_perm_.get(), d_tstart_.get(), d_iperm_.get(),
-                sc_, s);
+    int* tstart = prec_ == kFP32 ? spme32_->d_tile_start.get() : spme64_->d_tile_start.get();
+    bucket_sort(d_key_.get(), npos_, nt * nt * nt, d_perm_.get(), tstart, d_iperm_.get(), sc_, s);
     if (prec_ == kFP32)
-        spme32_->gather_sorted(d_perm_.get(), d_pos_.get(), d_rdi_.get(), d_tstart_.get(), s);
+        spme32_->gather_sorted(d_perm_.get(), d_pos_.get(), d_rdi_.get(), s);
     else
-        spme64_->gather_sorted(d_perm_.get(), d_pos_.get(), d_rdi_.get(), d_tstart_.get(), s);
+        spme64_->gather_sorted(d_perm_.get(), d_pos_.get(), d_rdi_.get(), s);
     hipLaunchKernelGGL(gather_sorted_kernel, dim3(ceil_div(npos_, 256)), dim3(256), 0, s, npos_,
                        d_perm_.get(), d_pos_.get(), d_rdi_.get(), d_pos_s_.get(), d_rdi_s_.get());
     SDT_HIP_CHECK(hipGetLastError());

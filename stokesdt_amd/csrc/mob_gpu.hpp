@@ -111,7 +111,7 @@ class MobSpmeGpu : public MobGpu {
     DevBuf<double> d_xblk_;   // column-blocked copy of the packed input (real space)
     SortScratch sc_;
     DevBuf<double> d_pos_, d_rdi_, d_pos_s_, d_rdi_s_;
-    DevBuf<int> d_key_, d_perm_, d_iperm_, d_tstart_;
+    DevBuf<int> d_key_, d_perm_, d_iperm_;
     DevBuf<double> d_io_f_, d_io_v_, d_X_, d_Y_;
     long long real_nnz_ = 0;
     StageTimer* timer_ = nullptr;

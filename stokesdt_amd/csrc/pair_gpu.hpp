@@ -20,6 +20,7 @@ struct PairListGpu {
     DevBuf<int> d_sidx;         // 4 ints per stencil entry: dx, dy, dz, all
     DevBuf<double> d_ssum;      // 2 doubles per stencil entry: min_sum, max_sum
     DevBuf<double> d_pos0;      // wrapped positions
+    DevBuf<double> d_pos_c, d_rdi_c;   // wrapped positions and radii in cell order
     DevBuf<int> d_cidx;         // cell of each particle
     DevBuf<int> d_cell_perm, d_cell_start;
     DevBuf<int> d_cnt, d_rowptr, d_colidx;

@@ -35,89 +35,123 @@ __device__ __forceinline__ int wrapc(int c, int nc1) {
     return c < 0 ? c + nc1 : c;
 }
 
-// One thread per row. PASS 0 counts, PASS 1 writes column ids.
+// positions (and radii, if given) in cell order: a cell's members, and the
+// neighbouring cells' along z, lie side by side
+__global__ void gather_cells_kernel(int npos, const int* __restrict__ cell_perm,
+                                    const double* __restrict__ pos0, const double* __restrict__ rdi,
+                                    double* __restrict__ pos_c, double* __restrict__ rdi_c) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= npos) return;
+    const int j = cell_perm[t];
+#pragma unroll
+    for (int d = 0; d < 3; d++) pos_c[3 * t + d] = pos0[3 * j + d];
+    if (rdi_c) rdi_c[t] = rdi[j];
+}
+
+// kPairLanes lanes per row, each taking one cell of a round of kPairLanes
+// consecutive search cells: the row's columns come in cell order, a cell's in
+// member order, as with one thread per row. A cell's first 64 decisions are
+// kept as bits between the round's count and its writes (PASS 1). The searches
+// are chains of dependent loads (cell bounds, then members); with a thread per
+// row they had 3 waves per SIMD to hide them at N = 50 000: 206 and 177 us for
+// the two passes, 61 and 43 us now (N = 50 000, volume fraction 0.3, cutoff 5).
+constexpr int kPairLanes = 16;
+
+// PASS 0 counts, PASS 1 writes column ids.
 template <char MODE, int PASS>
-__global__ void find_pairs_kernel(int npos, const int* __restrict__ row_map,
-                                  const int* __restrict__ col_map, const double* __restrict__ pos0,
-                                  const double* __restrict__ rdi, const int* __restrict__ cidx,
-                                  const int* __restrict__ cell_start,
-                                  const int* __restrict__ cell_perm, const int* __restrict__ sidx,
-                                  const double* __restrict__ ssum, int nsidx, int nc1, double box,
-                                  double cutoff, double min_radius, double max_radius,
-                                  int* __restrict__ cnt, const int* __restrict__ rowptr,
-                                  int* __restrict__ colidx) {
-    const int row = blockIdx.x * blockDim.x + threadIdx.x;
-    if (row >= npos) return;
+__global__ void __launch_bounds__(256)
+find_pairs_kernel(int npos, const int* __restrict__ row_map, const int* __restrict__ col_map,
+                  const double* __restrict__ pos0, const double* __restrict__ rdi,
+                  const int* __restrict__ cidx, const int* __restrict__ cell_start,
+                  const int* __restrict__ cell_perm, const double* __restrict__ pos_c,
+                  const double* __restrict__ rdi_c, const int* __restrict__ sidx,
+                  const double* __restrict__ ssum, int nsidx, int nc1, double box, double cutoff,
+                  double min_radius, double max_radius, int* __restrict__ cnt,
+                  const int* __restrict__ rowptr, int* __restrict__ colidx) {
+    const long long tid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int sub = (int)(tid % kPairLanes);
+    const bool on = tid / kPairLanes < npos;
+    const int row = on ? (int)(tid / kPairLanes) : npos - 1;
     const int i = row_map ? row_map[row] : row;
     const int c1 = cidx[i];
     const int ix1 = c1 / (nc1 * nc1), iy1 = (c1 / nc1) % nc1, iz1 = c1 % nc1;
     const double x1 = pos0[3 * i], y1 = pos0[3 * i + 1], z1 = pos0[3 * i + 2];
     const double r1 = rdi[i];
     const double half = box / 2.0;
-    int n = 0;
-    int out = (PASS == 1) ? rowptr[row] : 0;
-    for (int k = 0; k < nsidx; k++) {
-        const int ix2 = wrapc(ix1 + sidx[4 * k], nc1);
-        const int iy2 = wrapc(iy1 + sidx[4 * k + 1], nc1);
-        const int iz2 = wrapc(iz1 + sidx[4 * k + 2], nc1);
-        const int c2 = (ix2 * nc1 + iy2) * nc1 + iz2;
-        const int jb = cell_start[c2], je = cell_start[c2 + 1];
-        if (MODE == 'R') {
-            const bool all = sidx[4 * k + 3] != 0;
-            for (int t = jb; t < je; t++) {
-                const int j = cell_perm[t];
-                bool take = all;
-                if (!all) {
-                    double rx = fabs(pos0[3 * j] - x1);
-                    double ry = fabs(pos0[3 * j + 1] - y1);
-                    double rz = fabs(pos0[3 * j + 2] - z1);
-                    rx = (rx > half ? rx - box : rx);
-                    ry = (ry > half ? ry - box : ry);
-                    rz = (rz > half ? rz - box : rz);
-                    double rr = rx * rx + ry * ry + rz * rz;
-                    take = sqrt(rr) <= cutoff;
-                }
-                if (take) {
-                    if (PASS == 1) colidx[out++] = col_map ? col_map[j] : j;
-                    n++;
-                }
-            }
-        } else {
-            const double min_sum = ssum[2 * k], max_sum = ssum[2 * k + 1];
-            if (r1 + min_radius > max_sum) {
-                for (int t = jb; t < je; t++) {
-                    const int j = cell_perm[t];
-                    if (PASS == 1) colidx[out++] = col_map ? col_map[j] : j;
-                    n++;
-                }
-            } else if (r1 + max_radius > min_sum) {
-                for (int t = jb; t < je; t++) {
-                    const int j = cell_perm[t];
-                    const double r2 = rdi[j];
-                    bool take = false;
-                    if (r1 + r2 > max_sum) {
-                        take = true;
-                    } else if (r1 + r2 > min_sum) {
-                        double rx = fabs(pos0[3 * j] - x1);
-                        double ry = fabs(pos0[3 * j + 1] - y1);
-                        double rz = fabs(pos0[3 * j + 2] - z1);
-                        rx = (rx > half ? rx - box : rx);
-                        ry = (ry > half ? ry - box : ry);
-                        rz = (rz > half ? rz - box : rz);
-                        double rr = rx * rx + ry * ry + rz * rz;
-                        if (rr == 0.0) rr = 1.0e-10;
-                        double s = 2.0 * sqrt(rr) / (r1 + r2);
-                        take = s < cutoff;
-                    }
-                    if (take) {
-                        if (PASS == 1) colidx[out++] = col_map ? col_map[j] : j;
-                        n++;
-                    }
-                }
+    // the FP64 distance of member t, as the reference's tests take it
+    auto dist2 = [&](int t) {
+        double rx = fabs(pos_c[3 * t] - x1);
+        double ry = fabs(pos_c[3 * t + 1] - y1);
+        double rz = fabs(pos_c[3 * t + 2] - z1);
+        rx = (rx > half ? rx - box : rx);
+        ry = (ry > half ? ry - box : ry);
+        rz = (rz > half ? rz - box : rz);
+        return rx * rx + ry * ry + rz * rz;
+    };
+    int n = 0, out = (PASS == 1) ? rowptr[row] : 0;
+    for (int k0 = 0; k0 < nsidx; k0 += kPairLanes) {
+        const int k = k0 + sub;
+        int jb = 0, je = 0;
+        bool all = false;
+        double min_sum = 0.0, max_sum = 0.0;
+        if (on && k < nsidx) {
+            const int ix2 = wrapc(ix1 + sidx[4 * k], nc1);
+            const int iy2 = wrapc(iy1 + sidx[4 * k + 1], nc1);
+            const int iz2 = wrapc(iz1 + sidx[4 * k + 2], nc1);
+            const int c2 = (ix2 * nc1 + iy2) * nc1 + iz2;
+            jb = cell_start[c2];
+            je = cell_start[c2 + 1];
+            if (MODE == 'R') {
+                all = sidx[4 * k + 3] != 0;
+            } else {
+                min_sum = ssum[2 * k];
+                max_sum = ssum[2 * k + 1];
+                all = r1 + min_radius > max_sum;
+                if (!all && !(r1 + max_radius > min_sum)) je = jb;
             }
         }
+        auto take = [&](int t) -> bool {
+            if (all) return true;
+            if (MODE == 'R') return sqrt(dist2(t)) <= cutoff;
+            const double rs = r1 + rdi_c[t];
+            if (rs > max_sum) return true;
+            if (!(rs > min_sum)) return false;
+            double rr = dist2(t);
+            if (rr == 0.0) rr = 1.0e-10;
+            const double s = 2.0 * sqrt(rr) / rs;
+            return s < cutoff;
+        };
+        int m = 0;
+        unsigned long long bits = 0;
+        for (int t = jb; t < je; t++) {
+            const bool hit = take(t);
+            m += hit;
+            if (PASS == 1 && t - jb < 64) bits |= (unsigned long long)hit << (t - jb);
+        }
+        if (PASS == 0) {
+            n += m;
+        } else {
+            int inc = m;
+#pragma unroll
+            for (int o = 1; o < kPairLanes; o <<= 1) {
+                const int v = __shfl_up(inc, o, kPairLanes);
+                if (sub >= o) inc += v;
+            }
+            int w = out + inc - m;
+            for (int t = jb; t < je; t++) {
+                const bool hit = t - jb < 64 ? (bits >> (t - jb)) & 1 : take(t);
+                if (!hit) continue;
+                const int j = cell_perm[t];
+                colidx[w++] = col_map ? col_map[j] : j;
+            }
+            out += __shfl(inc, kPairLanes - 1, kPairLanes);
+        }
     }
-    if (PASS == 0) cnt[row] = n;
+    if (PASS == 0) {
+#pragma unroll
+        for (int o = kPairLanes / 2; o > 0; o >>= 1) n += __shfl_xor(n, o, kPairLanes);
+        if (on && sub == 0) cnt[row] = n;
+    }
 }
 
 __global__ void sort_rows_kernel(int nrows, const int* __restrict__ rowptr, int* __restrict__ colidx) {
@@ -187,6 +221,8 @@ int PairListGpu::init(int npos_, const double* h_rdi, double box_, double cutoff
     SDT_HIP_CHECK(sync_memcpy(d_rdi.get(), h_rdi, sizeof(double) * npos, hipMemcpyHostToDevice));
     d_pos0.reserve(3 * (size_t)npos);
     d_cidx.reserve(npos);
+    d_pos_c.reserve(3 * (size_t)npos);
+    if (mode == 'S') d_rdi_c.reserve(npos);
     d_cell_perm.reserve(npos);
     d_cell_start.reserve((size_t)nc3 + 1);
     d_cnt.reserve(npos);
@@ -210,10 +246,14 @@ int PairListGpu::build(const double* d_pos, const int* row_map, const int* col_m
     hipLaunchKernelGGL(cell_assign_kernel, dim3(g), dim3(256), 0, s, npos, d_pos, box, nc1,
                        d_pos0.get(), d_cidx.get());
     bucket_sort(d_cidx.get(), npos, nc3, d_cell_perm.get(), d_cell_start.get(), nullptr, sc, s);
+    hipLaunchKernelGGL(gather_cells_kernel, dim3(g), dim3(256), 0, s, npos, d_cell_perm.get(),
+                       d_pos0.get(), d_rdi.get(), d_pos_c.get(),
+                       mode == 'S' ? d_rdi_c.get() : (double*)nullptr);
+    const unsigned gp = ceil_div((size_t)npos * kPairLanes, 256);
 #define SDT_FIND(M, PS)                                                                        \
-    hipLaunchKernelGGL((find_pairs_kernel<M, PS>), dim3(g), dim3(256), 0, s, npos, row_map,     \
+    hipLaunchKernelGGL((find_pairs_kernel<M, PS>), dim3(gp), dim3(256), 0, s, npos, row_map,    \
                        col_map, d_pos0.get(), d_rdi.get(), d_cidx.get(), d_cell_start.get(),    \
-                       d_cell_perm.get(), d_sidx.get(), d_ssum.get(), nsidx, nc1, box, cutoff,  \
+                       d_cell_perm.get(), d_pos_c.get(), d_rdi_c.get(), d_sidx.get(), d_ssum.get(), nsidx, nc1, box, cutoff,  \
                        min_radius, max_radius, d_cnt.get(), d_rowptr.get(), d_colidx.get())
     if (mode == 'R') SDT_FIND('R', 0); else SDT_FIND('S', 0);
     exclusive_scan(d_cnt.get(), npos, d_rowptr.get(), sc.scan, s);

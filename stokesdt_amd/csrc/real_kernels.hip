@@ -228,14 +228,22 @@ __device__ __forceinline__ bool overlapping(int i, int j, const double* pos, con
     return pair_rr(dx, dy, dz) < sab * sab;
 }
 
+constexpr int kOvLanes = 8;
+
 __global__ void overlap_count_kernel(int npos, const int* __restrict__ rowptr,
                                      const int* __restrict__ colidx, const double* __restrict__ pos,
                                      const double* __restrict__ rdi, double box,
                                      int* __restrict__ cnt, int* __restrict__ has) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= npos) return;
+    // kOvLanes lanes per row
+    const long long tid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = (int)(tid / kOvLanes), sub = (int)(tid % kOvLanes);
     int c = 0;
-    for (int k = rowptr[i]; k < rowptr[i + 1]; k++) c += overlapping(i, colidx[k], pos, rdi, box);
+    if (i < npos)
+        for (int k = rowptr[i] + sub; k < rowptr[i + 1]; k += kOvLanes)
+            c += overlapping(i, colidx[k], pos, rdi, box);
+#pragma unroll
+    for (int o = kOvLanes / 2; o > 0; o >>= 1) c += __shfl_xor(c, o, kOvLanes);
+    if (i >= npos || sub != 0) return;
     cnt[i] = c;
     has[i] = c > 0;
 }
@@ -263,7 +271,8 @@ void RealOverlap::build(int npos, const int* d_rowptr, const int* d_colidx, cons
     rowptr.reserve((size_t)npos + 1);
     hrp.reserve((size_t)npos + 1);
     const unsigned g = ceil_div((size_t)npos, 256);
-    hipLaunchKernelGGL(overlap_count_kernel, dim3(g), dim3(256), 0, s, npos, d_rowptr, d_colidx,
+    hipLaunchKernelGGL(overlap_count_kernel, dim3(ceil_div((size_t)npos * kOvLanes, 256)),
+                       dim3(256), 0, s, npos, d_rowptr, d_colidx,
                        d_pos, d_rdi, box, cnt.get(), has.get());
     SDT_HIP_CHECK(hipGetLastError());
     exclusive_scan(cnt.get(), npos, rowptr.get(), scratch, s);

@@ -82,8 +82,8 @@ struct SpmeGpu {
     // sort key of every particle in key_out (original order)
     void prepare(const double* d_pos, int* d_key_out, hipStream_t s);
     // after the shared sort: gather per-particle data into sorted order
-    void gather_sorted(const int* d_perm, const double* d_pos, const double* d_rdi,
-                       const int* d_tile_start_in, hipStream_t s);
+    // (d_tile_start filled by it)
+    void gather_sorted(const int* d_perm, const double* d_pos, const double* d_rdi, hipStream_t s);
     // Y = alpha * M_recip X + beta * Y, packed FP64 vectors, b RHS; xb:
     // optional column-blocked copy of X in T with blocked_cols(b) columns
     // per block (Xb[cb][j][c][r], zero-padded), which the spread then reads

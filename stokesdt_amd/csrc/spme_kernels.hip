@@ -1267,7 +1267,7 @@ void SpmeGpu<T>::prepare(const double* d_pos, int* d_key, hipStream_t s) {
 
 template <typename T>
 void SpmeGpu<T>::gather_sorted(const int* d_perm, const double* d_pos, const double* d_rdi,
-                               const int* d_tile_start_in, hipStream_t s) {
+                               hipStream_t s) {
     (void)d_pos;
     const int nsx = (K + 31) / 32;
     const int nblocks = nsx * (int)ceil_div(K, 4) * (int)ceil_div(K, 4);
@@ -1278,15 +1278,12 @@ void SpmeGpu<T>::gather_sorted(const int* d_perm, const double* d_pos, const dou
                            d_frac.get(), d_base.get(), poly ? d_a2.get() : (double*)nullptr, d_nids.get()); \
         hipLaunchKernelGGL((spread_list_kernel<PP>), dim3(ceil_div(nblocks, kListWaves)),     \
                            dim3(64 * kListWaves), 0, s, K, ts, ntile, nsx, nblocks,           \
-                           d_tile_start_in, d_base.get(), d_nids.get(), d_blk.get(),          \
+                           d_tile_start.get(), d_base.get(), d_nids.get(), d_blk.get(),          \
                            d_ids.get());                                                      \
         break;
     switch (porder) { SDT_GATHER(4) SDT_GATHER(5) SDT_GATHER(6) SDT_GATHER(7) SDT_GATHER(8) }
 #undef SDT_GATHER
     SDT_HIP_CHECK(hipGetLastError());
-    const size_t nt3 = (size_t)ntile * ntile * ntile + 1;
-    SDT_HIP_CHECK(hipMemcpyAsync(d_tile_start.get(), d_tile_start_in, sizeof(int) * nt3,
-                                 hipMemcpyDeviceToDevice, s));
 }
 
 // force values per workgroup of the spread: 4 or 16 when few meshes are
