@@ -13,6 +13,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include "fft_lds.hpp"
 #include "spme_fft.hpp"
 #include "real_gpu.hpp"
@@ -1077,6 +1078,172 @@ interp_tile_kernel(int K, int ts, int ntile, int nsx, int sxt, int ch,
     }
 }
 
+// The same interpolation from blocks of tiles. A workgroup of 512 threads
+// takes the particles whose base points lie in an st.x x st.y x st.z block of
+// tiles (16 x 16 x 16 points where they are dense), for RB right-hand sides. A
+// mesh's region is then (16 + P - 1)^3 points, 2.3 reads per mesh point (P =
+// 6) where the strips above read each 3.1 times. An item (particle, z line)
+// stays with its thread for all meshes, its x weights and stencil origin in
+// registers (y and z weights in LDS: with all in registers the 128 that two
+// workgroups per CU leave spilled, 1.95 against 1.78 ms); the particle sums of
+// a pass run beside the next region's stores, two barriers a pass.
+// Bound by the regions' loads, LDS reads with random bank conflicts and the
+// barriers between them. Interpolation of 100 FP32 columns, strips -> blocks:
+// K = 128, N = 100 000: 1.95 -> 1.78 ms, K = 108, N = 50 000: 1.39 -> 1.06; 32
+// columns, K = 100, N = 50 000: 446 -> 302 us; 16 FP64 columns, K = 90,
+// N = 20 011: 302 -> 188 us.
+constexpr int kIbThreads = 512, kIbItems = 3;
+
+template <typename T, int P, int RREG, bool POLY>
+__global__ void __launch_bounds__(kIbThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 2)))
+interp_block_kernel(int K, int ts, int ntile, int3 nb, int3 st, const int* __restrict__ tile_start,
+                    const T* __restrict__ sten, const double* __restrict__ a2,
+                    const T* __restrict__ mesh, int b, int RB, double alpha, double beta,
+                    double* __restrict__ Y) {
+    typedef Sten<T, P> St;
+    typedef typename std::conditional<POLY, double, T>::type RT;
+    constexpr int NC = POLY ? 6 : 3, CH = kIbThreads * kIbItems / P;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    __shared__ int s_beg[16], s_off[17];
+    const unsigned lid = xcd_logical_id(blockIdx.x + blockIdx.y * gridDim.x, gridDim.x * gridDim.y);
+    const int bxl = (int)(lid % gridDim.x), byl = (int)(lid / gridDim.x);
+    const int tx = bxl % nb.x * st.x, ty = bxl / nb.x % nb.y * st.y, tz = bxl / (nb.x * nb.y) * st.z;
+    const int ntx = min(st.x, ntile - tx), nty = min(st.y, ntile - ty), ntz = min(st.z, ntile - tz);
+    const int r0 = byl * RB, rb = min(RB, b - r0), nmesh = rb * NC;
+    const int sx0 = tx * ts, sy0 = ty * ts, sz0 = tz * ts;
+    const int RX = ntx * ts + P - 1, RY = nty * ts + P - 1, RZ = ntz * ts + P - 1;
+    const int nreg = RX * RY * RZ;
+    // LDS: region T[nreg] | partial sums T[2][CH][P] | results RT[CH][RB][3] | ids
+    const int nreg_max = (st.x * ts + P - 1) * (st.y * ts + P - 1) * (st.z * ts + P - 1);
+    T* region = reinterpret_cast<T*>(smem_raw);
+    T* s_part = region + ((nreg_max + 3) & ~3);
+    constexpr int WS = 2 * P + 1;   // wy, wz of a particle
+    T* s_w = s_part + 2 * CH * P;
+    RT* s_res = reinterpret_cast<RT*>(s_w + ((CH * WS + 3) & ~3));
+    int* s_id = reinterpret_cast<int*>(s_res + CH * RB * 3);
+    // the particles: one range of the sorted order per tile row
+    if (threadIdx.x < 64) {
+        const int nrow = nty * ntz, r = threadIdx.x;
+        int pb = 0, n = 0;
+        if (r < nrow) {
+            const int t = ((tz + r / nty) * ntile + ty + r % nty) * ntile + tx;
+            pb = tile_start[t];
+            n = tile_start[t + ntx] - pb;
+        }
+        int inc = n;
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) {
+            const int v = __shfl_up(inc, o);
+            if (r >= o) inc += v;
+        }
+        if (r < 16) {
+            s_beg[r] = pb;
+            s_off[r] = inc - n;
+            if (r == 15) s_off[16] = inc;
+        }
+    }
+    const size_t K3 = (size_t)K * K * K;
+    unsigned offb[RREG];
+    {
+        const unsigned rx_m = 0xffffffffu / (unsigned)RX + 1u;
+        const unsigned ry_m = 0xffffffffu / (unsigned)RY + 1u;
+#pragma unroll
+        for (int u = 0; u < RREG; u++) {
+            const int i = min((int)threadIdx.x + kIbThreads * u, nreg - 1);
+            const int row = (int)fdiv(i, rx_m), lx = i - row * RX;
+            const int lz = (int)fdiv(row, ry_m), ly = row - lz * RY;
+            offb[u] = (unsigned)((wrapk(sz0 + lz, K) * K + wrapk(sy0 + ly, K)) * K +
+                                 wrapk(sx0 + lx, K)) * (unsigned)sizeof(T);
+        }
+    }
+    const unsigned char* mbase = reinterpret_cast<const unsigned char*>(mesh + (size_t)r0 * NC * K3);
+    T v[RREG];
+    auto prefetch = [&](int q) __attribute__((always_inline)) {
+        const unsigned char* m = mbase + (size_t)q * K3 * sizeof(T);
+#pragma unroll
+        for (int u = 0; u < RREG; u++) v[u] = *reinterpret_cast<const T*>(m + offb[u]);
+    };
+    __syncthreads();
+    const int np = s_off[16];
+    for (int c0 = 0; c0 < np; c0 += CH) {
+        const int cnt = min(CH, np - c0);
+        // the items' weights and stencil origins
+        T wx[kIbItems][P];
+        int at[kIbItems];
+#pragma unroll
+        for (int u = 0; u < kIbItems; u++) {
+            const int it = threadIdx.x + u * kIbThreads, t = it / P, iz = it - t * P;
+            at[u] = -1;
+            if (t < cnt) {
+                int k = 0;
+                while (s_off[k + 1] <= c0 + t) k++;
+                const int is = s_beg[k] + c0 + t - s_off[k];
+                if (iz == 0) s_id[t] = is;
+                const T* rec = sten + (size_t)is * St::N;
+                const int* b3 = reinterpret_cast<const int*>(rec);
+#pragma unroll
+                for (int i = 0; i < P; i++) wx[u][i] = rec[St::OW + i];
+                s_w[t * WS + iz] = rec[St::OW + St::RUN + iz];
+                s_w[t * WS + P + iz] = rec[St::OW + 2 * St::RUN + iz];
+                at[u] = ((wrapk(b3[2] - sz0, K) + iz) * RY + wrapk(b3[1] - sy0, K)) * RX +
+                        wrapk(b3[0] - sx0, K);
+            }
+        }
+        prefetch(0);
+        // one more round than meshes: round pi stores region pi and adds up
+        // the particle sums of mesh pi - 1
+        for (int pi = 0; pi <= nmesh; pi++) {
+            if (pi < nmesh) {
+#pragma unroll
+                for (int u = 0; u < RREG; u++) {
+                    const int i = (int)threadIdx.x + kIbThreads * u;
+                    if (i < nreg) region[i] = v[u];
+                }
+            }
+            if (pi > 0) {
+                const T* sp = s_part + ((pi - 1) & 1) * CH * P;
+                const int q = pi - 1, r = q / NC, c = q - r * NC;
+                for (int t = threadIdx.x; t < cnt; t += kIbThreads) {
+                    T sum = T(0);
+#pragma unroll
+                    for (int iz = 0; iz < P; iz++) sum += sp[t * P + iz];
+                    RT* o = s_res + (t * RB + r) * 3 + c % 3;
+                    if (c < 3) *o = (RT)sum;
+                    else *o += (RT)sum * (RT)a2[s_id[t]];
+                }
+            }
+            __syncthreads();
+            if (pi == nmesh) break;
+            if (pi + 1 < nmesh) prefetch(pi + 1);
+            T* sp = s_part + (pi & 1) * CH * P;
+#pragma unroll
+            for (int u = 0; u < kIbItems; u++) {
+                if (at[u] < 0) continue;
+                const int it = threadIdx.x + u * kIbThreads, t = it / P;
+                const T* rp = region + at[u];
+                const T* w = s_w + t * WS;
+                T acc = T(0);
+#pragma unroll 2
+                for (int iy = 0; iy < P; iy++) {
+                    T row = T(0);
+#pragma unroll
+                    for (int ix = 0; ix < P; ix++) row += wx[u][ix] * rp[iy * RX + ix];
+                    acc += w[iy] * row;
+                }
+                sp[it] = acc * w[P + it - t * P];
+            }
+            __syncthreads();
+        }
+        for (int i = threadIdx.x; i < cnt * rb * 3; i += kIbThreads) {
+            const int t = i / (rb * 3), cr = i - t * rb * 3;
+            const int c = cr / rb, r = cr - c * rb;
+            double* y = &Y[(size_t)(3 * s_id[t] + c) * b + r0 + r];
+            *y = (beta == 0.0 ? 0.0 : beta * *y) + alpha * (double)s_res[(t * RB + r) * 3 + c];
+        }
+        __syncthreads();
+    }
+}
+
 // ------------------------------------------------------------ host side ----
 void bspline_moduli(int K, int P, std::vector<double>& out) {
     // |b(m)|^2 = 1 / |sum_{i<P-1} M_P(i+1) e^{2 pi i m i / K}|^2
@@ -1549,6 +1716,80 @@ void SpmeGpu<T>::interp(int b, double alpha, double beta, double* Y, hipStream_t
     const double a_eff = alpha / (box * box * box);
     const int RB = 4;
     const int R = porder - 1;
+    // Cubes of tiles, unless the tuning or a form asks for strips. Sides by
+    // tile side and order (measured over K = 36 .. 216, p = 4 .. 8, both
+    // precisions): the larger the block the fewer its halo reads, up to 19
+    // region points in a thread's prefetch registers and to the particles of
+    // a chunk; sparse FP32 meshes of 8-point tiles (fewer than 2.2 particles
+    // per 4^3 points) take flatter blocks, whose passes are shorter (K = 216, 8
+    // columns: 550 against 640 us for cubes and 585 for strips). Strips stay
+    // faster on large sparse meshes, whose passes are all staging (three
+    // workgroups per CU against two): with 8-point tiles, below 48 particles a
+    // block on a grid above 2048 (K = 192, 16 columns, 26 particles a block:
+    // 677 against 706 us).
+    const SpmeTuning& tn = tune[width_class(b)];
+    const double dens = (double)npos / ((double)K * K * K);
+    int sd[3] = {2, 2, 2};
+    if (ts == 6) { sd[0] = 3; }
+    else if (ts == 5) { sd[0] = 4; sd[1] = 3; }
+    else if (ts == 4) { sd[0] = 4; sd[1] = 4; sd[2] = 3; }
+    else if (porder >= 7) { sd[2] = 1; }
+    else if (sizeof(T) == 4 && dens * 64 < 2.2) { sd[0] = ntile >= 6 ? 3 : 2; sd[2] = 1; }
+    for (int d = 0; d < 3; d++) sd[d] = std::min(sd[d], ntile);
+    auto blocks = [&]() {
+        size_t n = 1;
+        for (int d = 0; d < 3; d++) n *= ceil_div(ntile, sd[d]);
+        return n;
+    };
+    auto particles = [&]() { return dens * sd[0] * sd[1] * sd[2] * ts * ts * ts; };
+    const bool strips = interp_form > 0 || tn.interp_sxt > 0 || tn.interp_ch > 0 ||
+                        (ts == 8 && particles() < 48 && blocks() * ceil_div(b, RB) > 2048);
+    if (!strips) {
+        const int CH = kIbThreads * kIbItems / porder;
+        auto reg_of = [&]() {
+            return (size_t)(sd[0] * ts + R) * (sd[1] * ts + R) * (sd[2] * ts + R);
+        };
+        auto lds_b = [&](int rb) {
+            return ((reg_of() + 3) / 4 * 4 + 2 * (size_t)CH * porder +
+                    (CH * (2 * porder + 1) + 3) / 4 * 4) * sizeof(T) +
+                   (size_t)CH * rb * 3 * (poly ? 8 : sizeof(T)) + CH * sizeof(int);
+        };
+        // smaller blocks where the particles exceed a chunk and on small
+        // meshes, where the grid would leave CUs idle
+        for (int d = 2; sd[0] > 1 || sd[1] > 1 || sd[2] > 1; d = (d + 2) % 3) {
+            if (reg_of() <= 19u * kIbThreads && lds_b(1) <= 150 * 1024 &&
+                particles() <= 0.9 * CH && blocks() * b >= 512)
+                break;
+            if (sd[d] > 1) sd[d]--;
+        }
+        int rbk = std::min(b, porder >= 7 && !poly ? 2 * RB : RB);
+        while (rbk > 1 && (lds_b(rbk) > (sizeof(T) == 4 ? 80 : 155) * 1024 ||
+                           blocks() * ceil_div(b, rbk) < 512))
+            rbk--;
+        const size_t lds = lds_b(rbk);
+        const int rreg = (int)ceil_div(reg_of(), kIbThreads);
+        SDT_REQUIRE(rreg <= 19 && lds <= max_lds_bytes(), SDT_EINVAL, "interp: region too large");
+        const int3 nb = make_int3(ceil_div(ntile, sd[0]), ceil_div(ntile, sd[1]), ceil_div(ntile, sd[2]));
+        const dim3 grid(nb.x * nb.y * nb.z, ceil_div(b, rbk));
+#define SDT_IB_R(PP, RR, PO)                                                                  \
+    do {                                                                                      \
+        allow_lds((const void*)interp_block_kernel<T, PP, RR, PO>, lds);                      \
+        hipLaunchKernelGGL((interp_block_kernel<T, PP, RR, PO>), grid, dim3(kIbThreads), lds, s, K, \
+                           ts, ntile, nb, make_int3(sd[0], sd[1], sd[2]), d_tile_start.get(), \
+                           d_sten.get(), d_a2.get(), d_real.get(), b, rbk, a_eff, beta, Y);   \
+    } while (0)
+#define SDT_IB(PP)                                                                            \
+    case PP:                                                                                  \
+        if (rreg <= 8) { if (poly) SDT_IB_R(PP, 8, true); else SDT_IB_R(PP, 8, false); }      \
+        else if (rreg <= 16) { if (poly) SDT_IB_R(PP, 16, true); else SDT_IB_R(PP, 16, false); } \
+        else { if (poly) SDT_IB_R(PP, 19, true); else SDT_IB_R(PP, 19, false); }              \
+        break;
+        switch (porder) { SDT_IB(4) SDT_IB(5) SDT_IB(6) SDT_IB(7) SDT_IB(8) }
+#undef SDT_IB
+#undef SDT_IB_R
+        SDT_HIP_CHECK(hipGetLastError());
+        return;
+    }
     // strip width (tiles along x) and particle chunk (measured at K = 128,
     // p = 6): FP32 4-tile strips, FP64 2-tile strips
     // interp_form > 0 overrides the meshes per pass (FP32 1, 2 or 4; FP64 1
@@ -1559,7 +1800,6 @@ void SpmeGpu<T>::interp(int b, double alpha, double beta, double* Y, hipStream_t
                 "interp: meshes per pass must be 1, 2 or (FP32) 4");
     const int rlim = MV == 4 ? 16 : 26;
     int sxt = sizeof(T) == 8 ? 2 : 4, ch = sizeof(T) == 8 ? 64 : 128;
-    const SpmeTuning& tn = tune[width_class(b)];
     if (tn.interp_sxt > 0) sxt = tn.interp_sxt;
     if (tn.interp_ch > 0) ch = tn.interp_ch;
     auto lds_of = [&](int sx, int c) {
