@@ -1,5 +1,6 @@
 // Tall-skinny FP64 block kernels for block Lanczos (packed row-major n x b
 // blocks) and vector layout conversion.
+#include <algorithm>
 #include "block_gpu.hpp"
 #include "fft_lds.hpp"
 
@@ -16,14 +17,23 @@ namespace sdt {
 // zero. Consecutive workgroups take the groups of one row chunk, so the rows
 // are read from HBM once and re-read from L2. Partials are reduced by a
 // second kernel in fixed order (deterministic).
-constexpr int kGramRows = 2048;   // rows per workgroup
 constexpr int kGramThreads = 256;
+
+// rows per workgroup: up to 2048, fewer for short blocks so that about 48
+// chunks run side by side (a wave takes 32 rows a step: 16 serial steps in
+// 2048). By n alone: a group's sums do not depend on the batch it is in.
+// n = 2100, 20 columns: 17 -> 8 us.
+static int gram_rows(long long n) {
+    const long long r = (n / 48 + 127) / 128 * 128;
+    return (int)std::min(2048LL, std::max(128LL, r));
+}
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 
 __global__ void __launch_bounds__(kGramThreads)
-gram_partial_kernel(long long n, int btot, int bs, int ngroup, const double* __restrict__ A,
-                    const double* __restrict__ B, double* __restrict__ part) {
+gram_partial_kernel(long long n, int btot, int bs, int ngroup, int rows,
+                    const double* __restrict__ A, const double* __restrict__ B,
+                    double* __restrict__ part) {
     __shared__ double s_red[kGramThreads / 64][256];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -34,8 +44,8 @@ gram_partial_kernel(long long n, int btot, int bs, int ngroup, const double* __r
     const int chunk = (int)(lid / ngroup);
     const int c0 = g * bs;
     const int bg = min(bs, btot - c0);
-    const long long row0 = (long long)chunk * kGramRows;
-    const long long rend = min(row0 + kGramRows, n);
+    const long long row0 = (long long)chunk * rows;
+    const long long rend = min(row0 + rows, n);
     // fragment layout of v_mfma_f64_16x16x4f64 (measured on gfx950): A
     // operand lane l holds A[m = l % 16][k = l / 16]; B operand lane l holds
     // B[k = l / 16][n = l % 16]; result register v of lane l holds
@@ -95,10 +105,11 @@ void gram_groups(long long n, int btot, int bs, const double* A, const double* B
                  DevBuf<double>& part, hipStream_t s) {
     SDT_REQUIRE(bs >= 1 && bs <= 16 && btot >= 1, SDT_EINVAL, "group width must be in [1, 16]");
     const int ngroup = (btot + bs - 1) / bs;
-    const unsigned nchunk = ceil_div(n, kGramRows);
+    const int rows = gram_rows(n);
+    const unsigned nchunk = ceil_div(n, rows);
     part.reserve((size_t)nchunk * ngroup * 256);
     hipLaunchKernelGGL(gram_partial_kernel, dim3(nchunk * ngroup), dim3(kGramThreads), 0, s, n,
-                       btot, bs, ngroup, A, B, part.get());
+                       btot, bs, ngroup, rows, A, B, part.get());
     hipLaunchKernelGGL(gram_reduce_kernel, dim3(ngroup), dim3(256), 0, s, (int)nchunk, ngroup,
                        part.get(), d_G);
     SDT_HIP_CHECK(hipGetLastError());
@@ -122,14 +133,16 @@ void gram(long long n, int b, const double* A, const double* B, double* d_G, Dev
 // is followed by one unused slot (row length btot + ngroup), so the groups a
 // wave reads at once fall on distinct banks. C may alias A when nblk = 1
 // (in-place C = C S): a tile is in LDS before any of its rows is written.
-constexpr int kTsRows = 32;
+// kTsRows = 32, or 8 where 32 would leave fewer than 1024 workgroups (rows are
+// independent: the same result).
 constexpr int kTsCols = 128;   // widest packed block of the tile kernel
-constexpr int kTsLoads = kTsRows * kTsCols / 256;   // tile elements per thread
 
+template <int kTsRows>
 __global__ void __launch_bounds__(256)
 tsmm_tile_kernel(long long n, int btot, int bs, unsigned bmag, int nblk, const double* A,
                  long long blk_stride, const double* __restrict__ S, double alpha, double beta,
                  double* C) {
+    constexpr int kTsLoads = kTsRows * kTsCols / 256;   // tile elements per thread
     extern __shared__ double tile[];   // [kTsRows][ld]
     const int ld = btot + (btot + bs - 1) / bs;
     const long long row0 = (long long)blockIdx.x * kTsRows;
@@ -236,10 +249,15 @@ static void launch_tsmm(long long n, int btot, int bs, int nblk, const double* A
                         long long blk_stride, const double* d_S, double alpha, double beta,
                         double* C, hipStream_t s) {
     if (btot <= kTsCols) {
-        const size_t lds = sizeof(double) * kTsRows * (btot + (btot + bs - 1) / bs);
-        hipLaunchKernelGGL(tsmm_tile_kernel, dim3(ceil_div(n, kTsRows)), dim3(256), lds, s, n,
-                           btot, bs, fft_magic((unsigned)bs), nblk, A, blk_stride, d_S, alpha,
-                           beta, C);
+        const size_t row = sizeof(double) * (btot + (btot + bs - 1) / bs);
+        if (n >= 32 * 1024)
+            hipLaunchKernelGGL((tsmm_tile_kernel<32>), dim3(ceil_div(n, 32)), dim3(256), 32 * row, s,
+                               n, btot, bs, fft_magic((unsigned)bs), nblk, A, blk_stride, d_S,
+                               alpha, beta, C);
+        else
+            hipLaunchKernelGGL((tsmm_tile_kernel<8>), dim3(ceil_div(n, 8)), dim3(256), 8 * row, s, n,
+                               btot, bs, fft_magic((unsigned)bs), nblk, A, blk_stride, d_S, alpha,
+                               beta, C);
     } else {
         // rows are read and written by different threads: no aliasing
         SDT_REQUIRE(C != A, SDT_EINVAL, "tsmm: in-place product needs at most 128 columns");
@@ -384,61 +402,65 @@ lz_coef_kernel(int bs, int btot, const int* __restrict__ mask, const double* __r
 // keeps R in R1[g]; pass 1 writes B_g = R R1[g] (mul_upper) into the record.
 // A masked group, or one whose pivot is not positive (numerically rank
 // deficient: the pass zeroes its columns), gets S = 0, B = 0 and ok = 0.
-// Lane c (< 16) holds column c; the width is padded to 16 with the identity.
+// Lane c (< W) holds column c; the width is padded to W = 4, 8 or 16 with the
+// identity. A chain of square roots, divisions and shuffles bounds it: W steps
+// of W - j updates, so the narrowest W that holds the groups is taken (same
+// bits; 8 columns: 11 us at W = 16).
+template <int W>
 __global__ void __launch_bounds__(64)
 lz_chol_kernel(int bs, int btot, const int* __restrict__ mask, const double* __restrict__ G,
                double* __restrict__ R1, double* __restrict__ rec, double* __restrict__ S,
                int pass) {
-    const int g = blockIdx.x, c = threadIdx.x & 15;
-    const bool lead = threadIdx.x < 16;
+    const int g = blockIdx.x, c = threadIdx.x & (W - 1);
+    const bool lead = threadIdx.x < W;
     const int b = min(bs, btot - g * bs);
     double* rg = rec + (size_t)g * kLzRec;
     bool ok = mask[g] != 0;
     if (pass == 1) ok = ok && rg[512] != 0.0;
     const double* Gg = G + (size_t)g * 256;
-    double a[16];
+    double a[W];
 #pragma unroll
-    for (int r = 0; r < 16; r++)
+    for (int r = 0; r < W; r++)
         a[r] = (r < b && c < b) ? 0.5 * (Gg[r * 16 + c] + Gg[c * 16 + r]) : (r == c ? 1.0 : 0.0);
-    double rc[16];   // column c of R
+    double rc[W];   // column c of R
 #pragma unroll
-    for (int j = 0; j < 16; j++) {
+    for (int j = 0; j < W; j++) {
         const double p = __shfl(a[j], j);
         if (!(p > 0.0)) ok = false;
         const double rjj = p > 0.0 ? sqrt(p) : 1.0;
         const double rjc = c == j ? rjj : (c > j ? a[j] / rjj : 0.0);
         rc[j] = rjc;
 #pragma unroll
-        for (int i = j + 1; i < 16; i++) a[i] -= __shfl(rjc, i) * rjc;
+        for (int i = j + 1; i < W; i++) a[i] -= __shfl(rjc, i) * rjc;
     }
     // column c of R^{-1} by back substitution
-    double x[16];
+    double x[W];
 #pragma unroll
-    for (int r = 15; r >= 0; r--) {
+    for (int r = W - 1; r >= 0; r--) {
         double t = r == c ? 1.0 : 0.0;
 #pragma unroll
-        for (int k = r + 1; k < 16; k++) t -= __shfl(rc[r], k) * x[k];
+        for (int k = r + 1; k < W; k++) t -= __shfl(rc[r], k) * x[k];
         x[r] = r <= c ? t / __shfl(rc[r], r) : 0.0;
     }
     if (lead) {
         if (c < bs)
 #pragma unroll
-            for (int i = 0; i < 16; i++)
+            for (int i = 0; i < W; i++)
                 if (i < bs) S[((size_t)g * bs + i) * bs + c] = (ok && i < b && c < b) ? x[i] : 0.0;
         if (pass == 0) {
 #pragma unroll
-            for (int r = 0; r < 16; r++) R1[(size_t)g * 256 + r * 16 + c] = rc[r];
+            for (int r = 0; r < W; r++) R1[(size_t)g * 256 + r * 16 + c] = rc[r];
         }
     }
     if (pass == 1) {
-        double r1[16];
+        double r1[W];
 #pragma unroll
-        for (int k = 0; k < 16; k++) r1[k] = R1[(size_t)g * 256 + k * 16 + c];
+        for (int k = 0; k < W; k++) r1[k] = R1[(size_t)g * 256 + k * 16 + c];
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
+        for (int i = 0; i < W; i++) {
             double t = 0.0;
 #pragma unroll
-            for (int k = i; k < 16; k++) t += __shfl(rc[i], k) * r1[k];
+            for (int k = i; k < W; k++) t += __shfl(rc[i], k) * r1[k];
             if (lead) rg[256 + i * 16 + c] = (ok && c >= i) ? t : 0.0;
         }
     }
@@ -453,7 +475,11 @@ void lz_coef(int ng, int bs, int btot, const int* d_mask, const double* d_G, con
 
 void lz_chol(int ng, int bs, int btot, const int* d_mask, const double* d_G, double* d_R1,
              double* d_rec, double* d_S, int pass, hipStream_t s) {
-    lz_chol_kernel<<<ng, 64, 0, s>>>(bs, btot, d_mask, d_G, d_R1, d_rec, d_S, pass);
+    if (bs <= 4) lz_chol_kernel<4><<<ng, 64, 0, s>>>(bs, btot, d_mask, d_G, d_R1, d_rec, d_S, pass);
+    else if (bs <= 8)
+        lz_chol_kernel<8><<<ng, 64, 0, s>>>(bs, btot, d_mask, d_G, d_R1, d_rec, d_S, pass);
+    else
+        lz_chol_kernel<16><<<ng, 64, 0, s>>>(bs, btot, d_mask, d_G, d_R1, d_rec, d_S, pass);
     SDT_HIP_CHECK(hipGetLastError());
 }
 
