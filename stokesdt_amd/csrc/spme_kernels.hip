@@ -923,6 +923,26 @@ fft_z_influence_kernel(FFTArgs fa, cplx<T>* __restrict__ spec, const double* __r
 // meshes with vector LDS reads, and each particle adds its P slices in fixed
 // order (src/mob/spme.h:219-265 without the stored P/ind tables).
 // Y = beta Y + alpha (sum_U + a^2 sum_W).
+// A point's place within one mesh, in 32 bits: bytes where a mesh is no longer
+// than 2^32 of them (FP32 up to K = 1024: one scaled add less per load), else
+// elements (K^3 <= 2^30), widened before they are scaled (an FP64 mesh passes
+// 2^32 bytes from K = 813).
+constexpr int kMaxSide = 1024;
+template <typename T>
+struct MeshPoint {
+    static constexpr bool bytes = (size_t)kMaxSide * kMaxSide * kMaxSide * sizeof(T) <= 1ull << 32;
+    static_assert((size_t)kMaxSide * kMaxSide * kMaxSide <= 1ull << 32, "32-bit element index");
+    static __device__ __forceinline__ unsigned at(int x, int y, int z, int K) {
+        return (unsigned)((z * K + y) * K + x) * (bytes ? (unsigned)sizeof(T) : 1u);
+    }
+    static __device__ __forceinline__ T load(const T* mesh, unsigned at) {
+        if constexpr (bytes)
+            return *reinterpret_cast<const T*>(reinterpret_cast<const unsigned char*>(mesh) + at);
+        else
+            return mesh[at];
+    }
+};
+
 template <typename T, int MV>
 struct InterpVec {
     typedef T type __attribute__((ext_vector_type(MV)));
@@ -959,10 +979,10 @@ interp_tile_kernel(int K, int ts, int ntile, int nsx, int sxt, int ch,
     double* s_res = reinterpret_cast<double*>(
         (reinterpret_cast<uintptr_t>(s_b + ch * 3) + 7) & ~(uintptr_t)7);
     const size_t K3 = (size_t)K * K * K;
-    // byte offsets within one mesh of this thread's region points (the same
-    // for every mesh; 32-bit, added to the wave-uniform mesh base): point u is
-    // region index threadIdx.x + 256 u
-    unsigned offb[RREG];
+    // this thread's region points within one mesh (the same for every mesh,
+    // added to its wave-uniform base): point u is region index
+    // threadIdx.x + 256 u
+    unsigned pt[RREG];
     {
         const unsigned rx_m = 0xffffffffu / (unsigned)RX + 1u;
         const unsigned ry_m = 0xffffffffu / (unsigned)RY + 1u;
@@ -971,22 +991,20 @@ interp_tile_kernel(int K, int ts, int ntile, int nsx, int sxt, int ch,
             const int i = min((int)threadIdx.x + 256 * u, nreg - 1);
             const int row = (int)fdiv(i, rx_m), lx = i - row * RX;
             const int lz = (int)fdiv(row, ry_m), ly = row - lz * RY;
-            offb[u] = (unsigned)((wrapk(sz0 + lz, K) * K + wrapk(sy0 + ly, K)) * K +
-                                 wrapk(sx0 + lx, K)) * (unsigned)sizeof(T);
+            pt[u] = MeshPoint<T>::at(wrapk(sx0 + lx, K), wrapk(sy0 + ly, K), wrapk(sz0 + lz, K), K);
         }
     }
-    const unsigned char* mbase =
-        reinterpret_cast<const unsigned char*>(mesh + (size_t)r0 * NC * K3);
+    const T* mbase = mesh + (size_t)r0 * NC * K3;
     VT v[RREG];
     auto prefetch = [&](int pi) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < MV; j++) {
             const int q = pi * MV + j;
-            const unsigned char* m = mbase + (size_t)min(q, nmesh - 1) * K3 * sizeof(T);
+            const T* m = mbase + (size_t)min(q, nmesh - 1) * K3;
             const bool on = q < nmesh;
 #pragma unroll
             for (int u = 0; u < RREG; u++) {
-                const T x = *reinterpret_cast<const T*>(m + offb[u]);
+                const T x = MeshPoint<T>::load(m, pt[u]);
                 v[u][j] = on ? x : T(0);
             }
         }
@@ -1143,7 +1161,7 @@ interp_block_kernel(int K, int ts, int ntile, int3 nb, int3 st, const int* __res
         }
     }
     const size_t K3 = (size_t)K * K * K;
-    unsigned offb[RREG];
+    unsigned pt[RREG];
     {
         const unsigned rx_m = 0xffffffffu / (unsigned)RX + 1u;
         const unsigned ry_m = 0xffffffffu / (unsigned)RY + 1u;
@@ -1152,16 +1170,15 @@ interp_block_kernel(int K, int ts, int ntile, int3 nb, int3 st, const int* __res
             const int i = min((int)threadIdx.x + kIbThreads * u, nreg - 1);
             const int row = (int)fdiv(i, rx_m), lx = i - row * RX;
             const int lz = (int)fdiv(row, ry_m), ly = row - lz * RY;
-            offb[u] = (unsigned)((wrapk(sz0 + lz, K) * K + wrapk(sy0 + ly, K)) * K +
-                                 wrapk(sx0 + lx, K)) * (unsigned)sizeof(T);
+            pt[u] = MeshPoint<T>::at(wrapk(sx0 + lx, K), wrapk(sy0 + ly, K), wrapk(sz0 + lz, K), K);
         }
     }
-    const unsigned char* mbase = reinterpret_cast<const unsigned char*>(mesh + (size_t)r0 * NC * K3);
+    const T* mbase = mesh + (size_t)r0 * NC * K3;
     T v[RREG];
     auto prefetch = [&](int q) __attribute__((always_inline)) {
-        const unsigned char* m = mbase + (size_t)q * K3 * sizeof(T);
+        const T* m = mbase + (size_t)q * K3;
 #pragma unroll
-        for (int u = 0; u < RREG; u++) v[u] = *reinterpret_cast<const T*>(m + offb[u]);
+        for (int u = 0; u < RREG; u++) v[u] = MeshPoint<T>::load(m, pt[u]);
     };
     __syncthreads();
     const int np = s_off[16];
@@ -1346,7 +1363,7 @@ void SpmeGpu<T>::create(int npos_, double box_, double xi_, int K_, int porder_,
                 "map is incomplete)");
     SDT_REQUIRE(make_fft_plan(K, &plan), SDT_EINVAL,
                 "mesh dimension must factor into 2, 3 and 5 on the GPU path");
-    SDT_REQUIRE(K <= 1024, SDT_EINVAL, "mesh dimension must be <= 1024");
+    SDT_REQUIRE(K <= kMaxSide, SDT_EINVAL, "mesh dimension must be <= 1024");
     plans[0] = plans[1] = plan;
     tune[0] = tune[1] = SpmeTuning();
     // tile side: a divisor of K in [P-1, 8], preferring 8 (one wave owns
