@@ -11,10 +11,14 @@
 
 namespace sdt {
 
+// v1: the line's form, a key and four choices; kernels: the kernels that the
+// choices were timed on. An entry of other kernels is not read and its system
+// is tuned anew. 2: interp_sxt and interp_ch select the strip kernel (0: blocks
+// of tiles), spread_stage_kb sizes the stage of stencil records and forces.
 static std::string tune_key(MobSpmeGpu* m, int b) {
     char buf[160];
     const int oct = (int)std::lround(std::log2((double)m->npos()));
-    std::snprintf(buf, sizeof(buf), "spme-v1 prec=%d K=%d p=%d poly=%d noct=%d b=%d",
+    std::snprintf(buf, sizeof(buf), "spme-v1 kernels=2 prec=%d K=%d p=%d poly=%d noct=%d b=%d",
                   m->precision(), m->K(), m->porder(), m->mono() ? 0 : 1, oct, b);
     return buf;
 }
