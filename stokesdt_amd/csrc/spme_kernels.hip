@@ -658,8 +658,11 @@ spread_vec_kernel(int K, int nsx, const int2* __restrict__ blk, const int* __res
         __syncthreads();
         spread_stage_packed<T, kVecQ>(n, s_pid, X, a2, b, NC, q0, REC, stage + OF);
         __syncthreads();
+        // a wave past the mesh's end lists nothing: on sides below 28 its bases
+        // would leave an entry's range
         unsigned* list = s_list + wave * cap;
-        const int cnt = spread_hits<T, P>(n, stage, REC, K, wave, lane, list);
+        const int cnt = org[0] + 4 * wave < K ? spread_hits<T, P>(n, stage, REC, K, wave, lane, list)
+                                              : 0;
         for (int k = 0; k < cnt; k++) {
             const unsigned entry = list[k];
             const T* rec = stage + (entry & 0xffffu);

@@ -58,6 +58,21 @@ def test_forms_identical_on_partial_blocks(sdt, K, prec):
         assert np.array_equal(out[0], out[form]), form
 
 
+@pytest.mark.parametrize("K,p", [(16, 4), (18, 4), (20, 5), (24, 6)])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_forms_identical_on_short_sides(sdt, K, p, prec):
+    # one x block of 16 to 24 points: waves of the comparison form lie past it
+    n, box = 700, 18.0
+    pos, rdi = uniform_system(n, box, 800 + K)
+    g = sdt.MobSpme(n, rdi, box, 0.9, 5.0, K, p, prec)
+    assert g.init(), g.init_error
+    g.update(pos)
+    f = np.random.default_rng(K).standard_normal((3 * n, 9))
+    ref = g.recip_mul_vector(f)
+    g.set_forms(0, 0, 1)
+    assert np.array_equal(ref, g.recip_mul_vector(f))
+
+
 @pytest.mark.parametrize("prec", [0, 1])
 def test_dense_blocks_overflow_the_stage(sdt, orc, prec):
     # 1500 particles in a box of 9 on 24^3: a block's candidates exceed every
