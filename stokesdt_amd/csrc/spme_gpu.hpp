@@ -34,6 +34,12 @@ struct SpmeTuning {
     }
 };
 
+// a spread block's candidates: ids[off .. off + n)
+struct SpreadSeg {
+    long long off;
+    int n;
+};
+
 template <typename T>
 struct SpmeGpu {
     int npos = 0, K = 0, porder = 0;
@@ -70,9 +76,10 @@ struct SpmeGpu {
     DevBuf<int> d_base;    // 3N B-spline base mesh indices (sorted order)
     DevBuf<double> d_a2;   // N radii squared (sorted order), poly only
     DevBuf<int> d_tile_start;  // ntile^3 + 1
-    // candidates of every 32 x 4 x 4 spread block: (offset, count) into d_ids
-    DevBuf<int2> d_blk;
-    DevBuf<int> d_ids, d_nids;
+    // candidates of every 32 x 4 x 4 spread block: its segment of d_ids
+    DevBuf<SpreadSeg> d_blk;
+    DevBuf<int> d_ids;
+    DevBuf<unsigned long long> d_nids;
     DevBuf<T> d_real;      // nmesh * K^3
     DevBuf<cplx<T>> d_spec;    // nmesh * K*K*Kh
 

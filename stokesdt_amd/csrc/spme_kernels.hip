@@ -98,7 +98,8 @@ __global__ void spme_gather_kernel(int npos, const int* __restrict__ perm,
                                    const double* __restrict__ frac_u, const int* __restrict__ base_u,
                                    const double* __restrict__ rdi, T* __restrict__ sten,
                                    double* __restrict__ frac, int* __restrict__ base,
-                                   double* __restrict__ a2, int* __restrict__ nids) {
+                                   double* __restrict__ a2,
+                                   unsigned long long* __restrict__ nids) {
     typedef Sten<T, P> St;
     const int is = blockIdx.x * blockDim.x + threadIdx.x;
     if (is == 0) *nids = 0;   // for spread_list_kernel, next on the stream
@@ -144,8 +145,9 @@ constexpr int kPtThreads = 512;
 // wave per block goes through the particles of the tiles its window touches
 // (the tiles of a row along x are one range of the sorted order, two where
 // they wrap) and keeps those whose stencil reaches the block, in that order.
-// blk[block] = (offset, count) into ids; the offsets come from an atomic
-// counter, so segments lie in any order, but each one's content is fixed.
+// blk[block] is its segment of ids; the offsets come from an atomic counter, so
+// segments lie in any order, but each one's content is fixed. They have 64
+// bits: a stencil reaches up to 18 blocks.
 // Finding the candidates inside every spread took a third of its 89 us for one
 // column at K = 128, N = 100 000 (62 us from the lists).
 constexpr int kListWaves = 16;
@@ -156,11 +158,12 @@ template <int P>
 __global__ void __launch_bounds__(64 * kListWaves)
 spread_list_kernel(int K, int ts, int ntile, int nsx, int nblocks,
                    const int* __restrict__ tile_start, const int* __restrict__ base,
-                   int* __restrict__ nids, int2* __restrict__ blk, int* __restrict__ ids) {
+                   unsigned long long* __restrict__ nids, SpreadSeg* __restrict__ blk,
+                   int* __restrict__ ids) {
     __shared__ int s_off_[kListWaves][kListRanges], s_beg_[kListWaves][kListRanges];
     __shared__ unsigned long long s_mask_[kListWaves][kListMasks];
     __shared__ int s_tot[kListWaves];
-    __shared__ int s_base;
+    __shared__ long long s_base;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     // waves past the last block repeat it and keep nothing
     const bool real = blockIdx.x * kListWaves + wave < nblocks;
@@ -253,12 +256,12 @@ spread_list_kernel(int K, int ts, int ntile, int nsx, int nblocks,
             s_tot[w] = sum;
             sum += t;
         }
-        s_base = sum > 0 ? atomicAdd(nids, sum) : 0;
+        s_base = sum > 0 ? (long long)atomicAdd(nids, (unsigned long long)sum) : 0;
     }
     __syncthreads();
     if (!real) return;
-    int off = s_base + s_tot[wave];
-    if (lane == 0) blk[bl] = make_int2(off, total);
+    long long off = s_base + s_tot[wave];
+    if (lane == 0) blk[bl] = SpreadSeg{off, total};
     for (int c0 = 0, g = 0; c0 < ncand; c0 += 64, g++) {
         const int ci = c0 + lane;
         const int is = particle(min(ci, ncand - 1));
@@ -480,7 +483,7 @@ __device__ __forceinline__ int sten_at(int x, unsigned entry, int d) {
 
 template <typename T, int P, int NQ, bool BLK>
 __global__ void __launch_bounds__(kPtThreads) __attribute__((amdgpu_waves_per_eu(BLK ? 4 : (sizeof(T) == 4 ? 6 : 5))))
-spread_mx_kernel(int K, int nsx, const int2* __restrict__ blk, const int* __restrict__ ids,
+spread_mx_kernel(int K, int nsx, const SpreadSeg* __restrict__ blk, const int* __restrict__ ids,
                  const T* __restrict__ sten, const double* __restrict__ a2,
                  const double* __restrict__ X, const T* __restrict__ Xb, int npos, int b,
                  int ncbw, int NC, int cap, T* __restrict__ mesh) {
@@ -500,9 +503,9 @@ spread_mx_kernel(int K, int nsx, const int2* __restrict__ blk, const int* __rest
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const unsigned lid = xcd_logical_id(blockIdx.x + blockIdx.y * gridDim.x, gridDim.x * gridDim.y);
     const int bxl = (int)(lid % gridDim.x), byl = (int)(lid / gridDim.x);
-    const int2 seg = blk[bxl];
-    const int ncand = seg.y;
-    const int* __restrict__ list_g = ids + seg.x;
+    const SpreadSeg seg = blk[bxl];
+    const int ncand = seg.n;
+    const int* __restrict__ list_g = ids + seg.off;
     const int K4 = (K + 3) >> 2;
     const int yz = bxl / nsx;
     const int org[3] = {(bxl % nsx) * 32, (yz % K4) * 4, (yz / K4) * 4};
@@ -633,7 +636,7 @@ constexpr int kVecQ = 16;
 
 template <typename T, int P>
 __global__ void __launch_bounds__(kPtThreads)
-spread_vec_kernel(int K, int nsx, const int2* __restrict__ blk, const int* __restrict__ ids,
+spread_vec_kernel(int K, int nsx, const SpreadSeg* __restrict__ blk, const int* __restrict__ ids,
                   const T* __restrict__ sten, const double* __restrict__ a2,
                   const double* __restrict__ X, int b, int NC, int cap, T* __restrict__ mesh) {
     typedef Sten<T, P> St;
@@ -644,7 +647,7 @@ spread_vec_kernel(int K, int nsx, const int2* __restrict__ blk, const int* __res
     unsigned* s_list = reinterpret_cast<unsigned*>(s_pid + cap);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int bxl = blockIdx.x, q0 = blockIdx.y * kVecQ;
-    const int2 seg = blk[bxl];
+    const SpreadSeg seg = blk[bxl];
     const int K4 = (K + 3) >> 2;
     const int yz = bxl / nsx;
     const int org[3] = {(bxl % nsx) * 32, (yz % K4) * 4, (yz / K4) * 4};
@@ -652,9 +655,9 @@ spread_vec_kernel(int K, int nsx, const int2* __restrict__ blk, const int* __res
     T acc[kVecQ];
 #pragma unroll
     for (int q = 0; q < kVecQ; q++) acc[q] = T(0);
-    for (int c0 = 0; c0 < seg.y; c0 += cap) {
-        const int n = min(cap, seg.y - c0);
-        spread_stage<T, P, 0>(n, ids + seg.x + c0, sten, nullptr, org, K, REC, stage, s_pid);
+    for (int c0 = 0; c0 < seg.n; c0 += cap) {
+        const int n = min(cap, seg.n - c0);
+        spread_stage<T, P, 0>(n, ids + seg.off + c0, sten, nullptr, org, K, REC, stage, s_pid);
         __syncthreads();
         spread_stage_packed<T, kVecQ>(n, s_pid, X, a2, b, NC, q0, REC, stage + OF);
         __syncthreads();
@@ -1396,7 +1399,6 @@ void SpmeGpu<T>::create(int npos_, double box_, double xi_, int K_, int porder_,
         return (long long)most;
     };
     const long long ids_cap = reach(32) * reach(4) * reach(4) * npos;
-    SDT_REQUIRE(ids_cap < (1LL << 31), SDT_EINVAL, "spread: too many particles");
     const size_t nblocks = (size_t)ceil_div(K, 32) * ceil_div(K, 4) * ceil_div(K, 4);
     d_nids.reserve(1);
     d_ids.reserve((size_t)ids_cap);
