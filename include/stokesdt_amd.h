@@ -313,7 +313,8 @@ int sdt_ensemble_destroy(sdt_ensemble_t e);
  * seed, arriving arrival_s seconds after sdt_serve_run starts.
  * sdt_serve_run admits arrived jobs first come first served while a slot
  * (max_active) is free and the job's predicted device footprint
- * (sdt_serve_footprint) fits what is left of capacity_bytes; a job whose
+ * (sdt_serve_footprint of unit radii; a submitted job's own radii count for
+ * its reservation) fits what is left of capacity_bytes; a job whose
  * footprint exceeds the whole capacity is refused (state 3). Every admitted
  * job steps on its own stream and host thread with its state resident on
  * the device, so jobs admitted while others run overlap with them; its

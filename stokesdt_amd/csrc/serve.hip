@@ -11,7 +11,14 @@
 
 namespace sdt {
 
-size_t serve_footprint(const ServeParams& p, int npos, int dim, double box, double rmax) {
+size_t serve_footprint(const ServeParams& p, int npos, int dim, double box, double rmax,
+                       const double* rdi) {
+    double amax = 1.0;
+    bool poly = false;
+    if (rdi) {
+        amax = *std::max_element(rdi, rdi + npos);
+        poly = amax != 1.0 || *std::min_element(rdi, rdi + npos) != 1.0;
+    }
     const double n3 = 3.0 * npos, K3 = (double)dim * dim * dim;
     const double spec = (double)dim * dim * (dim / 2 + 1) * 2.0;   // reals per half spectrum
     const int mi = p.mob_interval;
@@ -23,6 +30,11 @@ size_t serve_footprint(const ServeParams& p, int npos, int dim, double box, doub
     bytes += n3 * 8.0 * 8;              // positions, forces, step vectors, copies
     bytes += 2.0 * n3 * mi * 8.0;       // Gaussian block and displacements of an interval
     bytes += nnz * 4.0 * 2 + npos * 64.0;   // CSR and cell lists
+    // starts of the cells: pair list (half a cutoff wide, with the sort's
+    // counters), steric list (half a contact distance) and contact cells; a
+    // system of more cells than the lists take, or a bad length, fails at init
+    auto cells = [&](double w) { return w > 0 ? std::min(std::pow(box / w + 1, 3), 2e9) : 0.0; };
+    bytes += cells(rmax / 2) * 12.0 + cells(p.r0 * amax / 2) * 4.0 + cells(p.r0 * amax) * 12.0;
     if (p.kind == kServePlain) {
         const int p3 = p.porder * p.porder * p.porder, ldp = (p3 + 7) / 8 * 8;
         bytes += (double)npos * ldp * 12.0;             // weight and index tables
@@ -30,11 +42,26 @@ size_t serve_footprint(const ServeParams& p, int npos, int dim, double box, doub
         bytes += nnz * 72.0;                            // stored 3x3 blocks
         bytes += n3 * p.max_nrhs * 8.0 * (p.max_iters + 1 + 2);   // one group's basis
     } else {
-        const int e = p.kind == kServeFP32 ? 4 : 8;
+        const bool f32 = p.kind == kServeFP32;
+        const int e = f32 ? 4 : 8;
         const int cols = std::min(mi, BrwnLanczosGpu::kMaxBatchCols);
-        bytes += n3 * cols * 8.0 * (p.max_iters + 1 + 4);   // basis, Z, Y, active subsets
-        bytes += 3.0 * cols * (K3 + spec) * e;             // meshes of a batch
-        bytes += n3 * cols * e;                            // blocked input copy
+        const int bs = std::max(p.max_nrhs, 1), groups = (cols + bs - 1) / bs;
+        const int nc = poly ? 6 : 3;
+        auto up = [](int c, int w) { return (c + w - 1) / w * w; };
+        bytes += n3 * cols * 8.0 * (p.max_iters + 1 + 2);   // basis, active subsets
+        bytes += n3 * groups * bs * 8.0 * 2;                // Z, Y
+        bytes += (n3 / 2048 + 49) * groups * 2048.0;        // Gram partials
+        bytes += nc * (double)cols * (K3 + spec) * e;       // meshes of a batch
+        // column-blocked input copies: the real space's, and the spread's own
+        // where it cannot read that one (unequal radii; few columns)
+        if (cols >= 8) bytes += n3 * up(cols, f32 && cols >= 16 ? 16 : 8) * e;
+        if (nc * cols > 16) bytes += n3 * (poly ? up(2 * cols, f32 ? 16 : 8) : (f32 ? 16 : 8)) * e;
+        // sorted positions, radii, orders, sort buffer of the mobility; its
+        // packed columns; cell-ordered copies of the two pair lists; overlaps
+        bytes += npos * (84.0 + 48.0 + 100.0 + 16.0);
+        const int order = std::min(std::max(p.porder, 4), 8), K = std::min(dim, 1024);
+        bytes += f32 ? SpmeGpu<float>::system_bytes(npos, K, order)
+                     : SpmeGpu<double>::system_bytes(npos, K, order);
     }
     return (size_t)(bytes * 1.1) + ((size_t)64 << 20);
 }
@@ -70,7 +97,7 @@ int ServeGpu::submit(int npos, const double* pos, const double* rdi, double box,
     j->seed = seed;
     j->pos.assign(pos, pos + 3 * (size_t)npos);
     j->rdi.assign(rdi, rdi + npos);
-    j->bytes = serve_footprint(p_, npos, dim, box, rmax);
+    j->bytes = serve_footprint(p_, npos, dim, box, rmax, rdi);
     jobs_.push_back(std::move(j));
     return (int)jobs_.size() - 1;
 }

@@ -42,9 +42,12 @@ struct ServeJob {
 
 // Predicted device footprint (bytes) of one job: particle arrays, the
 // Gaussian and displacement blocks of an interval, the Lanczos basis of one
-// lockstep batch, its meshes and the real-space pair list (optimised path),
-// or the stored tables, blocks and one group's basis (plain path).
-size_t serve_footprint(const ServeParams& p, int npos, int dim, double box, double rmax);
+// lockstep batch, its meshes, stencil records and candidate lists, and the
+// real-space pair list (optimised path), or the stored tables, blocks and one
+// group's basis (plain path). rdi: the job's radii (null: unit radii); unequal
+// radii double the meshes.
+size_t serve_footprint(const ServeParams& p, int npos, int dim, double box, double rmax,
+                       const double* rdi = nullptr);
 
 class ServeGpu {
   public:

@@ -84,6 +84,8 @@ struct SpmeGpu {
     DevBuf<cplx<T>> d_spec;    // nmesh * K*K*Kh
 
     void create(int npos, double box, double xi, int K, int porder, bool poly);
+    // device bytes of a system beside its meshes and input copies
+    static double system_bytes(int npos, int K, int porder);
     void reserve_rhs(int b);
     // positions (original order, FP64 device) -> particle tiles; returns the
     // sort key of every particle in key_out (original order)

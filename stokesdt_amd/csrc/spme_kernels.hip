@@ -1356,6 +1356,41 @@ static FFTArgs fft_args(const FFTPlan& p) {
     return a;
 }
 
+// entries of the spread's candidate lists: the most blocks that one stencil can
+// reach, over its base points and per dimension (blocks of 32 or 4 points, the
+// last one partial), for every particle
+static long long spread_list_cap(int npos, int K, int porder) {
+    auto reach = [&](int len) {
+        int most = 0;
+        for (int b0 = 0; b0 < K; b0++) {
+            std::vector<int> got;
+            for (int q = 0; q < porder; q++) {
+                const int bl = ((b0 + q) % K) / len;
+                if (std::find(got.begin(), got.end(), bl) == got.end()) got.push_back(bl);
+            }
+            most = std::max(most, (int)got.size());
+        }
+        return (long long)most;
+    };
+    return reach(32) * reach(4) * reach(4) * npos;
+}
+
+// Sten<T, P>::N
+template <typename T>
+static int sten_values(int porder) {
+    const int sv = 16 / (int)sizeof(T);
+    return (sv + 3 * (porder + 3) + 3 + sv - 1) / sv * sv;
+}
+
+template <typename T>
+double SpmeGpu<T>::system_bytes(int npos, int K, int porder) {
+    // record, two offsets, two bases and a^2 of a particle; its list entries;
+    // block segments; starts and sort counters of tiles of 4^3 points or more
+    return npos * ((double)sten_values<T>(porder) * sizeof(T) + 2 * 24 + 2 * 12 + 8) +
+           4.0 * spread_list_cap(npos, K, porder) +
+           (double)K * K * K * (sizeof(SpreadSeg) / 512.0 + 12.0 / 64.0);
+}
+
 template <typename T>
 void SpmeGpu<T>::create(int npos_, double box_, double xi_, int K_, int porder_, bool poly_) {
     npos = npos_; box = box_; xi = xi_; K = K_; porder = porder_; poly = poly_;
@@ -1384,24 +1419,9 @@ void SpmeGpu<T>::create(int npos_, double box_, double xi_, int K_, int porder_,
     const int trow = std::min(ntile, (porder + 3 + ts - 1) / ts + 1);
     SDT_REQUIRE(2 * trow * trow <= kListRanges, SDT_EINVAL,
                 "spread: too many contributor tiles for this order and mesh");
-    // blocks that one stencil can reach: the most over its base points, per
-    // dimension (blocks of 32 or 4 points, the last one partial)
-    auto reach = [&](int len) {
-        int most = 0;
-        for (int b0 = 0; b0 < K; b0++) {
-            std::vector<int> got;
-            for (int q = 0; q < porder; q++) {
-                const int bl = ((b0 + q) % K) / len;
-                if (std::find(got.begin(), got.end(), bl) == got.end()) got.push_back(bl);
-            }
-            most = std::max(most, (int)got.size());
-        }
-        return (long long)most;
-    };
-    const long long ids_cap = reach(32) * reach(4) * reach(4) * npos;
     const size_t nblocks = (size_t)ceil_div(K, 32) * ceil_div(K, 4) * ceil_div(K, 4);
     d_nids.reserve(1);
-    d_ids.reserve((size_t)ids_cap);
+    d_ids.reserve((size_t)spread_list_cap(npos, K, porder));
     d_blk.reserve(nblocks);
     std::vector<double> tw(2 * K);
     for (int j = 0; j < K; j++) {
@@ -1419,9 +1439,7 @@ void SpmeGpu<T>::create(int npos_, double box_, double xi_, int K_, int porder_,
     }
     d_fac.reserve(K);
     SDT_HIP_CHECK(sync_memcpy(d_fac.get(), bs.data(), sizeof(double) * K, hipMemcpyHostToDevice));
-    // the stencil records: Sten<T, P>::N values
-    const int sv = 16 / (int)sizeof(T);
-    sten_n = (sv + 3 * (porder + 3) + 3 + sv - 1) / sv * sv;
+    sten_n = sten_values<T>(porder);
     d_sten.reserve((size_t)sten_n * npos);
     d_frac.reserve(3 * (size_t)npos);
     d_base.reserve(3 * (size_t)npos);
