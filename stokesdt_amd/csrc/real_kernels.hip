@@ -151,9 +151,22 @@ template <typename T, int RC, typename XT, bool BLK>
 static void launch_real(int npos, const int* d_rowptr, const int* d_colidx, const double* d_pos,
                         const double* d_rdi, double box, double xi, int b, double alpha,
                         const XT* X, double beta, double* Y, hipStream_t s) {
-    // lanes per row: 4 for the blocked gathers (measured at b = 100), 8 for
-    // the in-place ones (b < 8); 16 where 4 would leave fewer than 256
-    // workgroups (N = 700, 20 FP64 columns: 32 -> 16 us)
+    // lanes per row: 8 for the in-place gathers (b < 8); for the blocked ones 4
+    // where that makes 256 workgroups, one per CU, else 8, and 16 below 128. A
+    // row's gathers are a chain, which more lanes shorten; once the CUs are
+    // full they only add loads. us of the stage with 4, 8, 16 lanes, by
+    // workgroups at 4 lanes (volume fraction 0.2, cutoff 5):
+    //     32  N =   700, 20 FP64 columns  33.2  26.4  23.2
+    //    117  N =  1500, 40 FP64          32.5  25.8  25.3
+    //    125  N =  8000,  8 FP32          26.6  22.3  21.8
+    //    140  N =  3000, 20 FP64          34.1  30.4  35.8
+    //    171  N =  5500, 20 FP32          39.7  36.7  36.4
+    //    234  N =  3000, 40 FP64          33.3  30.1  39.4
+    //    250  N =  8000, 20 FP32          40.3  38.3  51.3
+    //    257  N =  5500, 20 FP64          39.8  42.7  47.2
+    //    601  N =  5500, 100 FP32         63.8  68.5  94.5
+    // (A row's sum takes another order with another number of lanes, so its
+    // last bits depend on the launch's size.)
     auto launch = [&](auto lanes) {
         constexpr int LPR = decltype(lanes)::value;
         dim3 grid(ceil_div((size_t)npos * LPR, 256), ceil_div(b, RC));
@@ -161,8 +174,11 @@ static void launch_real(int npos, const int* d_rowptr, const int* d_colidx, cons
                            d_rowptr, d_colidx, d_pos, d_rdi, box, xi, b, alpha, X, beta, Y);
     };
     if constexpr (BLK) {
-        if ((size_t)npos * 4 * ceil_div(b, RC) < 256 * 256)
+        const size_t wg4 = ceil_div((size_t)npos * 4, 256) * (size_t)ceil_div(b, RC);
+        if (wg4 < 128)
             launch(std::integral_constant<int, 16>());
+        else if (wg4 < 256)
+            launch(std::integral_constant<int, 8>());
         else
             launch(std::integral_constant<int, 4>());
     } else {
