@@ -36,9 +36,9 @@ int sdt_debug_spme_spread(sdt_mob_t mob, const double* f, double* mesh);
  * 163-198). */
 int sdt_debug_spme_interp(sdt_mob_t mob, const double* mesh, double alpha, double* v);
 /* Launch forms of a mobility's kernels, for tests and measurements:
- * interp_form, meshes per LDS pass of the interp kernel: 0 the built-in
- * choice (1), else 1, 2 or 4 (4: FP32 only; an error at apply time
- * otherwise); z_form, the most threads and pencils per workgroup of the z
+ * interp_form: 0 the built-in choice (blocks of tiles, or strips on large
+ * sparse meshes: sdt_debug_spme_interp_plan), 1, 2 or 4 strips with that many
+ * meshes per LDS pass (4: FP32 only; an error at apply time otherwise); z_form, the most threads and pencils per workgroup of the z
  * transform: 0 the built-in choice, 1 .. 5 = (256, 16), (128, 16), (256, 8),
  * (128, 8), (256, 4);
  * spread_form: the spread's sums: 0 on the matrix cores, 1 and 2 on the vector
@@ -48,6 +48,12 @@ int sdt_debug_spme_interp(sdt_mob_t mob, const double* mesh, double alpha, doubl
  * sums;
  * fft_form: 0 the fused x + y plane kernels where a plane fits LDS, 1 the
  * separate x and y passes. */
+int sdt_debug_spme_forms(sdt_mob_t mob, int interp_form, int z_form, int spread_form,
+                         int fft_form);
+/* The interpolation launch that an initialised mobility takes for b columns:
+ * plan[0] 1 strips, 0 blocks of tiles; of blocks plan[1..3] tiles per
+ * dimension, plan[4] columns a workgroup. */
+int sdt_debug_spme_interp_plan(sdt_mob_t mob, int b, int* plan);
 /* Right-hand sides per launch of an SPME mobility's mulvector (default 16;
  * [1, 1024]): a wider launch runs every column block of a product in one
  * spread and interpolation, as the block-Lanczos batches do. */
@@ -58,8 +64,6 @@ int sdt_debug_mob_launch_width(sdt_mob_t mob, int width);
  * spread candidate stage 16 .. 64 KB. */
 int sdt_debug_spme_tuning(sdt_mob_t mob, int fft_order, int interp_sxt, int interp_ch,
                           int spread_stage_kb);
-int sdt_debug_spme_forms(sdt_mob_t mob, int interp_form, int z_form, int spread_form,
-                         int fft_form);
 /* Mean device time (ms, HIP events on the handle's stream) of each stage of
  * one packed matvec with b right-hand sides over `reps` repetitions:
  * t[0] spread, t[1] forward x/y FFT, t[2] z FFT + influence + inverse z,

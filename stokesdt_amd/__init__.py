@@ -106,6 +106,7 @@ SIGNATURES = {
     "sdt_debug_spme_spread": (_I, [_P, _P, _P]),
     "sdt_debug_spme_interp": (_I, [_P, _P, _D, _P]),
     "sdt_debug_spme_forms": (_I, [_P, _I, _I, _I, _I]),
+    "sdt_debug_spme_interp_plan": (_I, [_P, _I, _P]),
     "sdt_debug_mob_launch_width": (_I, [_P, _I]),
     "sdt_debug_spme_tuning": (_I, [_P, _I, _I, _I, _I]),
     "sdt_bench_stage_times": (_I, [_P, _I, _I, _P]),
@@ -287,8 +288,8 @@ class MobSpme:
         return v
 
     def set_forms(self, interp=0, z=0, spread=0, fft=0):
-        """Launch forms (testing and measurement): interp meshes per LDS pass
-        (0 built-in, 1, 2 or 4 (FP32)); z transform shape (0 built-in,
+        """Launch forms (testing and measurement): interp (0 built-in, else
+        strips with 1, 2 or (FP32) 4 meshes per LDS pass); z transform shape (0 built-in,
         1 .. 5); spread form (0 built-in matrix-core sums, 1 or 2 vector-ALU
         sums, 3 one column block per workgroup); x / y transforms (0 fused planes where
         they fit, 1 separate passes)."""
@@ -296,6 +297,13 @@ class MobSpme:
 
     def set_interp_form(self, form):
         self.set_forms(interp=form)
+
+    def interp_plan(self, b):
+        """The interpolation launch for b columns: ("strips",) or ("blocks",
+        tiles per dimension, columns a workgroup)."""
+        p = np.zeros(5, dtype=np.int32)
+        _check(lib().sdt_debug_spme_interp_plan(self.h, int(b), _ptr(p)))
+        return ("strips",) if p[0] else ("blocks", tuple(int(x) for x in p[1:4]), int(p[4]))
 
     def set_launch_width(self, width):
         """Right-hand sides per launch of mul_vector (default 16)."""

@@ -808,6 +808,19 @@ int sdt_debug_spme_forms(sdt_mob_t mob, int interp_form, int z_form, int spread_
     });
 }
 
+int sdt_debug_spme_interp_plan(sdt_mob_t mob, int b, int* plan) {
+    SDT_CHECK_HANDLE(mob);
+    return guard([&] {
+        MobSpmeGpu* m = spme_of(mob);
+        SDT_REQUIRE(m->spme32() || m->spme64(), SDT_ESTATE, "interp plan asked before init");
+        SDT_REQUIRE(b >= 1 && plan, SDT_EINVAL, "bad arguments");
+        const InterpPlan p = m->spme32() ? m->spme32()->interp_plan(b) : m->spme64()->interp_plan(b);
+        plan[0] = p.strips ? 1 : 0;
+        for (int d = 0; d < 3; d++) plan[1 + d] = p.strips ? 0 : p.sd[d];
+        plan[4] = p.strips ? 0 : p.rb;
+    });
+}
+
 int sdt_debug_spme_tuning(sdt_mob_t mob, int fft_order, int interp_sxt, int interp_ch,
                           int spread_stage_kb) {
     SDT_CHECK_HANDLE(mob);

@@ -34,6 +34,15 @@ struct SpmeTuning {
     }
 };
 
+// An interpolation launch: strips of tiles, or blocks of sd tiles per dimension
+// with rb right-hand sides a workgroup, lds bytes and rreg region points a thread
+struct InterpPlan {
+    bool strips = false;
+    int sd[3] = {2, 2, 2};
+    int rb = 0, rreg = 0;
+    size_t lds = 0;
+};
+
 // a spread block's candidates: ids[off .. off + n)
 struct SpreadSeg {
     long long off;
@@ -54,8 +63,8 @@ struct SpmeGpu {
     SpmeTuning tune[2];
     FFTPlan plans[2];
     static int width_class(int b) { return b >= 8 ? 1 : 0; }
-    // interp meshes per LDS pass: 0 the built-in choice (1), else 1, 2 or
-    // (FP32) 4
+    // interpolation: 0 the built-in choice (interp_plan), else strips with 1, 2
+    // or (FP32) 4 meshes per LDS pass
     int interp_form = 0;
     // z transform launch shape: 0 the built-in choice, 1 .. 5 at most
     // (threads, pencils) = (256, 16), (128, 16), (256, 8), (128, 8), (256, 4)
@@ -108,6 +117,7 @@ struct SpmeGpu {
     void influence(int b, hipStream_t s);
     void fft_backward(int b, hipStream_t s);
     void interp(int b, double alpha, double beta, double* Y, hipStream_t s);
+    InterpPlan interp_plan(int b) const;   // the launch that interp takes for b
     int nmesh(int b) const { return (poly ? 6 : 3) * b; }
     StageTimer* timer = nullptr;
 

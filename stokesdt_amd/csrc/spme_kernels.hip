@@ -1750,12 +1750,11 @@ void SpmeGpu<T>::fft_backward(int b, hipStream_t s) {
 }
 
 template <typename T>
-void SpmeGpu<T>::interp(int b, double alpha, double beta, double* Y, hipStream_t s) {
-    const int NC = poly ? 6 : 3;
-    // alpha * K^3 / L^3 with the unnormalised inverse transform: alpha / L^3
-    const double a_eff = alpha / (box * box * box);
+InterpPlan SpmeGpu<T>::interp_plan(int b) const {
     const int RB = 4;
     const int R = porder - 1;
+    InterpPlan pl;
+    int* sd = pl.sd;
     // Cubes of tiles, unless the tuning or a form asks for strips. Sides by
     // tile side and order (measured over K = 36 .. 216, p = 4 .. 8, both
     // precisions): the larger the block the fewer its halo reads, up to 19
@@ -1769,7 +1768,6 @@ void SpmeGpu<T>::interp(int b, double alpha, double beta, double* Y, hipStream_t
     // 677 against 706 us).
     const SpmeTuning& tn = tune[width_class(b)];
     const double dens = (double)npos / ((double)K * K * K);
-    int sd[3] = {2, 2, 2};
     if (ts == 6) { sd[0] = 3; }
     else if (ts == 5) { sd[0] = 4; sd[1] = 3; }
     else if (ts == 4) { sd[0] = 4; sd[1] = 4; sd[2] = 3; }
@@ -1782,32 +1780,48 @@ void SpmeGpu<T>::interp(int b, double alpha, double beta, double* Y, hipStream_t
         return n;
     };
     auto particles = [&]() { return dens * sd[0] * sd[1] * sd[2] * ts * ts * ts; };
-    const bool strips = interp_form > 0 || tn.interp_sxt > 0 || tn.interp_ch > 0 ||
-                        (ts == 8 && particles() < 48 && blocks() * ceil_div(b, RB) > 2048);
-    if (!strips) {
-        const int CH = kIbThreads * kIbItems / porder;
-        auto reg_of = [&]() {
-            return (size_t)(sd[0] * ts + R) * (sd[1] * ts + R) * (sd[2] * ts + R);
-        };
-        auto lds_b = [&](int rb) {
-            return ((reg_of() + 3) / 4 * 4 + 2 * (size_t)CH * porder +
-                    (CH * (2 * porder + 1) + 3) / 4 * 4) * sizeof(T) +
-                   (size_t)CH * rb * 3 * (poly ? 8 : sizeof(T)) + CH * sizeof(int);
-        };
-        // smaller blocks where the particles exceed a chunk and on small
-        // meshes, where the grid would leave CUs idle
-        for (int d = 2; sd[0] > 1 || sd[1] > 1 || sd[2] > 1; d = (d + 2) % 3) {
-            if (reg_of() <= 19u * kIbThreads && lds_b(1) <= 150 * 1024 &&
-                particles() <= 0.9 * CH && blocks() * b >= 512)
-                break;
-            if (sd[d] > 1) sd[d]--;
-        }
-        int rbk = std::min(b, porder >= 7 && !poly ? 2 * RB : RB);
-        while (rbk > 1 && (lds_b(rbk) > (sizeof(T) == 4 ? 80 : 155) * 1024 ||
-                           blocks() * ceil_div(b, rbk) < 512))
-            rbk--;
-        const size_t lds = lds_b(rbk);
-        const int rreg = (int)ceil_div(reg_of(), kIbThreads);
+    pl.strips = interp_form > 0 || tn.interp_sxt > 0 || tn.interp_ch > 0 ||
+                (ts == 8 && particles() < 48 && blocks() * ceil_div(b, RB) > 2048);
+    if (pl.strips) return pl;
+    const int CH = kIbThreads * kIbItems / porder;
+    auto reg_of = [&]() {
+        return (size_t)(sd[0] * ts + R) * (sd[1] * ts + R) * (sd[2] * ts + R);
+    };
+    auto lds_b = [&](int rb) {
+        return ((reg_of() + 3) / 4 * 4 + 2 * (size_t)CH * porder +
+                (CH * (2 * porder + 1) + 3) / 4 * 4) * sizeof(T) +
+               (size_t)CH * rb * 3 * (poly ? 8 : sizeof(T)) + CH * sizeof(int);
+    };
+    // smaller blocks where the particles exceed a chunk and on small
+    // meshes, where the grid would leave CUs idle
+    for (int d = 2; sd[0] > 1 || sd[1] > 1 || sd[2] > 1; d = (d + 2) % 3) {
+        if (reg_of() <= 19u * kIbThreads && lds_b(1) <= 150 * 1024 &&
+            particles() <= 0.9 * CH && blocks() * b >= 512)
+            break;
+        if (sd[d] > 1) sd[d]--;
+    }
+    pl.rb = std::min(b, porder >= 7 && !poly ? 2 * RB : RB);
+    while (pl.rb > 1 && (lds_b(pl.rb) > (sizeof(T) == 4 ? 80 : 155) * 1024 ||
+                         blocks() * ceil_div(b, pl.rb) < 512))
+        pl.rb--;
+    pl.lds = lds_b(pl.rb);
+    pl.rreg = (int)ceil_div(reg_of(), kIbThreads);
+    return pl;
+}
+
+template <typename T>
+void SpmeGpu<T>::interp(int b, double alpha, double beta, double* Y, hipStream_t s) {
+    const int NC = poly ? 6 : 3;
+    // alpha * K^3 / L^3 with the unnormalised inverse transform: alpha / L^3
+    const double a_eff = alpha / (box * box * box);
+    const int RB = 4;
+    const int R = porder - 1;
+    const SpmeTuning& tn = tune[width_class(b)];
+    const InterpPlan pl = interp_plan(b);
+    if (!pl.strips) {
+        const int* sd = pl.sd;
+        const int rbk = pl.rb, rreg = pl.rreg;
+        const size_t lds = pl.lds;
         SDT_REQUIRE(rreg <= 19 && lds <= max_lds_bytes(), SDT_EINVAL, "interp: region too large");
         const int3 nb = make_int3(ceil_div(ntile, sd[0]), ceil_div(ntile, sd[1]), ceil_div(ntile, sd[2]));
         const dim3 grid(nb.x * nb.y * nb.z, ceil_div(b, rbk));

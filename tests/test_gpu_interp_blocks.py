@@ -51,14 +51,36 @@ def test_recip_matches_oracle(sdt, orc, n, box, K, p, poly):
 
 
 def test_sparse_large_mesh_takes_strips(sdt, orc):
-    # 8-point tiles, few particles per block, a grid above the line: the
-    # built-in choice and the strips are the same launch
+    # 8-point tiles, few particles per block, a grid above the line
     n, box, K = 400, 40.0, 192
     pos, rdi = uniform_system(n, box, 1400)
     g = sdt.MobSpme(n, rdi, box, 0.9, 5.0, K, 6, sdt.FP32)
     assert g.init()
+    assert g.interp_plan(3) == ("strips",)
     g.update(pos)
+    o = orc.MobSpme(n, rdi, box, 0.9, 5.0, K, 6)
+    assert o.init()
+    o.update(pos, rdi)
     f = np.random.default_rng(1).standard_normal((3 * n, 3))
-    out = g.recip_mul_vector(f)
+    assert orc.frob_rel_err(o.mul_vector(f, mode="recip"), g.recip_mul_vector(f)) < 2e-6
+
+
+@pytest.mark.parametrize("n,K,p,prec,b,plan", [
+    # FP32 blocks of 3 x 2 x 1 tiles: 768 on 128^3, 2304 on 192^3 (grid line 2048)
+    (400, 128, 6, 1, 8, ("blocks", (3, 2, 1), 4)),
+    (400, 128, 6, 1, 9, ("strips",)),
+    # 48 particles in a block of 3072 points of 192^3
+    (110591, 192, 6, 1, 1, ("strips",)),
+    (110593, 192, 6, 1, 1, ("blocks", (3, 2, 1), 1)),
+    # FP64 cubes of 2 tiles: 1728 on 192^3
+    (400, 192, 6, 0, 4, ("blocks", (2, 2, 2), 4)),
+    (400, 192, 6, 0, 5, ("strips",)),
+    # 6-point tiles stay with blocks
+    (400, 180, 6, 1, 16, ("blocks", (3, 2, 2), 4)),
+])
+def test_rule_between_strips_and_blocks(sdt, n, K, p, prec, b, plan):
+    g = sdt.MobSpme(n, np.ones(n), 0.5 * K, 0.9, 5.0, K, p, prec)
+    assert g.init(), g.init_error
+    assert g.interp_plan(b) == plan
     g.set_interp_form(1)
-    assert np.array_equal(out, g.recip_mul_vector(f))
+    assert g.interp_plan(b) == ("strips",)
