@@ -298,14 +298,15 @@ def test_interp_meshes_per_pass_refused(sdt):
 
 @pytest.mark.parametrize("prec", [0, 1])
 def test_z_transform_launch_shapes_agree(sdt, orc, prec):
-    # the z transform and influence run with 1024, 512 or 256 threads and
-    # 16, 8 or 4 pencils per workgroup; each pencil's arithmetic is the same
-    # in every shape, so the results are identical
+    # the z transform and influence run with 256 or 128 threads and 16, 8 or
+    # 4 pencils per workgroup (9 columns: the grid of 16 pencils, 9 x 132,
+    # exceeds the 1024 workgroups below which fewer are taken); each pencil's
+    # arithmetic is the same in every shape, so the results are identical
     n, box = 2000, 30.0
     g, o, _, _ = _pair(sdt, orc, n, box, 0.9, 5.0, 64, 6, False, 51, prec)
-    f = np.random.default_rng(52).standard_normal((3 * n, 5))
+    f = np.random.default_rng(52).standard_normal((3 * n, 9))
     ref = None
-    for z in (1, 2, 3, 4, 5):
+    for z in (0, 1, 2, 3, 4, 5):
         g.set_forms(0, z)
         out = g.recip_mul_vector(f)
         if ref is None:
@@ -338,23 +339,20 @@ def test_wide_full_product_overlapped_streams(sdt, orc, prec, tol):
 
 @pytest.mark.parametrize("prec,K,p", [(0, 48, 6), (1, 48, 6), (1, 100, 6), (1, 120, 8), (1, 64, 4)])
 def test_spread_forms_identical(sdt, orc, prec, K, p):
-    # the point-owner spread sums wide FP32 launches on the vector ALUs
-    # (forces from scalar loads or LDS) or on the matrix cores (one
-    # workgroup per column block, or per mesh block over all column blocks),
-    # wide FP64 launches on the vector ALUs per column block or over all of
-    # them (form 1 + 8, the built-in one), and stores its meshes per lane or
-    # as whole rows through LDS. The
-    # matrix cores take 4 candidates per step in list order with one
-    # rounding per product-add, so every form gives the same sums. The full
-    # product (b >= 8) spreads from the column-blocked copy, which the
-    # matrix-core forms need; each product is one launch (b = 20 and 40 are
-    # two and three column blocks, the last one partial); K = 48, 100 and
-    # 120 leave a 16-, a 4- (one active wave) and a 24-point partial x block,
-    # p = 4 and 8 the shortest and longest stencils.
+    # the spread sums on the matrix cores, a workgroup taking several column
+    # blocks in turn (0) or one (3), or on the vector ALUs (1, the comparison
+    # form). The matrix cores take 4 candidates per step in list order with one
+    # rounding per product-add, so every form gives the same sums. Each product
+    # is one launch (b = 20 and 40 are two and three FP32 column blocks, the
+    # last one partial); 0 and 3 differ where the mesh blocks alone fill the
+    # chip (FP32 from K = 64; FP64, with blocks of 8 columns, at 48 as well);
+    # K = 48, 100 and 120 leave a 16-, a 4- (one active wave) and a 24-point
+    # partial x block, p = 4 and 8 the shortest and longest stencils. 2 is
+    # taken as 1, and a bit of 4, or 8 beside 0 .. 2, changes nothing.
     n, box = 3000, 30.0
     g, o, _, _ = _pair(sdt, orc, n, box, 0.9, 5.0, K, p, False, 81, prec)
     g.set_launch_width(64)
-    forms = (0, 1, 2, 3, 4, 5, 6, 7, 9, 11, 15)
+    forms = (0, 1, 3)
     for b in (1, 20, 40):
         f = np.random.default_rng(82 + b).standard_normal((3 * n, b))
         out = {}
@@ -368,15 +366,18 @@ def test_spread_forms_identical(sdt, orc, prec, K, p):
         tol = 1e-10 if prec == 0 else 1e-5
         assert orc.frob_rel_err(o.mul_vector(f, mode="recip"), out[0][0]) < tol
         assert orc.frob_rel_err(o.mul_vector(f), out[0][1]) < tol
+    for form in range(16):
+        g.set_forms(0, 0, form)
     with pytest.raises(Exception):
         g.set_forms(0, 0, 16)
 
 
 def test_spread_stage_overflow_same_sums(sdt, orc):
-    # a 16 KB stage holds 50 candidates of the matrix-core spread, and a
+    # a 16 KB stage holds 44 candidates of the matrix-core spread (record, 48
+    # forces, lists: 372 bytes each), and a
     # 32 x 4 x 4 block here has about 80: the blocks overflow it, and the
     # workgroup then stages and sums each column block in chunks. The sums
-    # keep candidate order, so they equal the vector-ALU forms' (with their
+    # keep candidate order, so they equal the vector-ALU form's (with its
     # own chunking) to the bit, in one launch over three column blocks.
     n, box = 3000, 30.0
     g, o, _, _ = _pair(sdt, orc, n, box, 0.9, 5.0, 48, 6, False, 83, sdt.FP32)
@@ -384,10 +385,10 @@ def test_spread_stage_overflow_same_sums(sdt, orc):
     g.set_tuning(spread_stage_kb=16)
     f = np.random.default_rng(84).standard_normal((3 * n, 40))
     out = {}
-    for form in (0, 1, 2):
+    for form in (0, 1):
         g.set_forms(0, 0, form)
         out[form] = g.mul_vector(f)
-    assert np.array_equal(out[0], out[1]) and np.array_equal(out[0], out[2])
+    assert np.array_equal(out[0], out[1])
     assert orc.frob_rel_err(o.mul_vector(f), out[0]) < 1e-5
     with pytest.raises(Exception):
         g.set_tuning(spread_stage_kb=8)
@@ -397,9 +398,8 @@ def test_spread_stage_overflow_same_sums(sdt, orc):
 def test_fused_and_separate_xy_transforms_agree(sdt, orc, prec):
     # the x / y transforms run as one fused plane kernel where a plane fits
     # LDS and as separate x and y passes otherwise; forcing the separate
-    # passes on the same mesh checks one against the other (FP64: the same
-    # radix chain, identical; FP32 K = 128: the fused kernel's two-stage
-    # 16 x 8 transform against the generic chain, rounding only)
+    # passes on the same mesh checks one against the other (K = 128: the same
+    # two stages and operations, identical)
     n, box = 2000, 30.0
     g, o, _, _ = _pair(sdt, orc, n, box, 0.9, 5.0, 128, 6, False, 91, prec)
     f = np.random.default_rng(92).standard_normal((3 * n, 9))
@@ -407,8 +407,5 @@ def test_fused_and_separate_xy_transforms_agree(sdt, orc, prec):
     sep = g.recip_mul_vector(f)
     g.set_forms(0, 0, 0, 0)
     fused = g.recip_mul_vector(f)
-    if prec == 0:
-        assert np.array_equal(sep, fused)
-    else:
-        assert orc.frob_rel_err(fused, sep) < 1e-6
+    assert np.array_equal(sep, fused)
     assert orc.frob_rel_err(o.mul_vector(f, mode="recip"), sep) < (1e-10 if prec == 0 else 1e-5)

@@ -41,6 +41,7 @@ def test_recip_columns_match_oracle(sdt, orc, K, p, poly):
         assert orc.frob_rel_err(full, g.mul_vector(f[:, :9])) < tol
 
 
+# 50 (FP64) and 90: a workgroup takes several column blocks in turn in form 0
 @pytest.mark.parametrize("K", [30, 50, 90])
 @pytest.mark.parametrize("prec", [0, 1])
 def test_forms_identical_on_partial_blocks(sdt, K, prec):
@@ -52,7 +53,7 @@ def test_forms_identical_on_partial_blocks(sdt, K, prec):
     g.set_launch_width(64)
     f = np.random.default_rng(K).standard_normal((3 * n, 35))
     out = {}
-    for form in (0, 1, 2, 3, 4, 5, 7, 9, 11, 15):
+    for form in (0, 1, 3):
         g.set_forms(0, 0, form)
         out[form] = g.recip_mul_vector(f)
         assert np.array_equal(out[0], out[form]), form
