@@ -483,14 +483,18 @@ fft2_y_kernel(cplx<T>* __restrict__ spec, const double* __restrict__ tw_g, int l
 // memory. Where the registers of all components' butterflies would exceed
 // the budget (NC R2 complex values), the middle part is three steps through
 // LDS, spread over the components (K = 256 FP64 poly: 2.05 ms for 18 meshes
-// against 2.86 with one thread taking all components in turn).
+// against 2.86 with one thread taking all components in turn). The line lies
+// below 192 registers of values: FP64 with unequal radii and R2 = 8 reaches them
+// and then runs one or two waves per SIMD. Its us for 20 columns, in registers /
+// three steps: K = 64: 123 / 95, 72: 164 / 136, 80: 354 / 186, 96: 844 / 368,
+// 128: 940 / 868.
 // 256 threads where the middle is in registers: K = 128 FP32, 100 columns
 // 1.15 ms against 1.56 with 384 (two workgroups fit then, and more waves
 // wait at each barrier). Chunks in XCD order: 1.15 against 1.18 ms, FP64 2.20
 // against 2.45.
 template <typename T, int R2, int NC>
 struct ZShape {
-    static constexpr bool in_regs = NC * R2 * 2 * (int)sizeof(T) / 4 <= 192;
+    static constexpr bool in_regs = NC * R2 * 2 * (int)sizeof(T) / 4 < 192;
     static constexpr int NT = in_regs ? 256 : 512;
 };
 
