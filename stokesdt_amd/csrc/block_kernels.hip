@@ -22,7 +22,11 @@ constexpr int kGramThreads = 256;
 // rows per workgroup: up to 2048, fewer for short blocks so that about 48
 // chunks run side by side (a wave takes 32 rows a step: 16 serial steps in
 // 2048). By n alone: a group's sums do not depend on the batch it is in.
-// n = 2100, 20 columns: 17 -> 3.7 us.
+// More chunks lengthen the reduction. us of both kernels with chunks of 2048
+// rows, 24, 48, 96 and 192 chunks, 20 columns in groups of 8: n = 2100: 21.1
+// 6.4 6.2 7.0 6.9; 24 000: 21.9 14.3 11.3 13.7 20.5; 48 000: 22.0 21.9 15.2 16.0
+// 22.1; 90 000: 22.6 22.7 22.6 20.0 25.0; 100 columns, 24 000: 22.4 16.5 15.2
+// 17.9 26.1.
 static int gram_rows(long long n) {
     const long long r = (n / 48 + 127) / 128 * 128;
     return (int)std::min(2048LL, std::max(128LL, r));
@@ -134,7 +138,10 @@ void gram(long long n, int b, const double* A, const double* B, double* d_G, Dev
 // wave reads at once fall on distinct banks. C may alias A when nblk = 1
 // (in-place C = C S): a tile is in LDS before any of its rows is written.
 // kTsRows = 32, or 8 where 32 would leave fewer than 1024 workgroups (rows are
-// independent: the same result; n = 2100, 20 columns: 12.6 -> 5.5 us).
+// independent: the same result). us with 8 and 32 rows, 20 columns: n = 2100:
+// 5.2 11.4; 24 000: 10.9 14.1; 32 700: 13.7 15.4; 48 000: 18.8 20.0; 90 000: 31.0
+// 31.6; 300 000: 83.2 75.7; 100 columns, 24 000: 18.0 20.1; 32 700: 18.1 18.6;
+// 90 000: 40.2 43.8; 300 000: 121.1 118.7.
 constexpr int kTsCols = 128;   // widest packed block of the tile kernel
 
 template <int kTsRows>

@@ -78,13 +78,14 @@ __global__ void spme_prepare_kernel(int npos, const double* __restrict__ pos, do
 }
 
 // One particle's stencil record, made once per update and read by every
-// spread: the base index (3 ints in one 16-byte slot), then
+// spread and by the interpolation from blocks of tiles: the base index (3 ints
+// in one 16-byte slot), then
 // the 1D weights 0 0 0 wx[P] 0 0 0 wy[P] 0 0 0 wz[P] 0 0 0, padded to 16
 // bytes. The zeros are the weights of the points up to 3 outside a stencil, so
-// that 4 points of a mesh block read theirs without a range test. (The
+// that 4 points of a mesh block read theirs without a range test. (The strip
 // interpolation makes its weights from the offsets again: a record's bytes per
-// group of 4 columns cost it more, 3.56 against 3.19 ms for 100 FP64 columns
-// at K = 128.)
+// group of 4 columns cost that kernel more, 3.56 against 3.19 ms for 100 FP64
+// columns at K = 128.)
 template <typename T, int P>
 struct Sten {
     static constexpr int V = 16 / (int)sizeof(T);    // values per 16 bytes
@@ -1108,11 +1109,16 @@ interp_tile_kernel(int K, int ts, int ntile, int nsx, int sxt, int ch,
 // mesh's region is then (16 + P - 1)^3 points, 2.3 reads per mesh point (P =
 // 6) where the strips above read each 3.1 times. An item (particle, z line)
 // stays with its thread for all meshes, its x weights and stencil origin in
-// registers (y and z weights in LDS: with all in registers the 128 that two
-// workgroups per CU leave spilled, 1.95 against 1.78 ms); the particle sums of
-// a pass run beside the next region's stores, two barriers a pass.
+// registers, y and z weights in LDS; the particle sums of
+// a pass run beside the next region's stores, two barriers a pass. Two
+// workgroups per CU leave 128 registers: with all weights in registers 1.95
+// instead of 1.78 ms, and as it is the FP32 kernels of 16 and 19 region points
+// a thread still spill 12 to 116 bytes a lane (P = 6: 24 and 96; order 4 with
+// 16 points none, FP64 none).
 // Bound by the regions' loads, LDS reads with random bank conflicts and the
-// barriers between them. Interpolation of 100 FP32 columns, strips -> blocks:
+// barriers between them. HBM traffic of 100 FP32 columns, K = 128: 6.4 GB, of
+// which 5.5 GB fetched (the meshes 2.2 times, strips 2.0) and 0.6 GB spilled
+// values. Interpolation of 100 FP32 columns, strips -> blocks:
 // K = 128, N = 100 000: 1.95 -> 1.78 ms, K = 108, N = 50 000: 1.39 -> 1.06; 32
 // columns, K = 100, N = 50 000: 446 -> 302 us; 16 FP64 columns, K = 90,
 // N = 20 011: 302 -> 188 us.
@@ -1756,16 +1762,20 @@ InterpPlan SpmeGpu<T>::interp_plan(int b) const {
     InterpPlan pl;
     int* sd = pl.sd;
     // Cubes of tiles, unless the tuning or a form asks for strips. Sides by
-    // tile side and order (measured over K = 36 .. 216, p = 4 .. 8, both
-    // precisions): the larger the block the fewer its halo reads, up to 19
-    // region points in a thread's prefetch registers and to the particles of
-    // a chunk; sparse FP32 meshes of 8-point tiles (fewer than 2.2 particles
-    // per 4^3 points) take flatter blocks, whose passes are shorter (K = 216, 8
-    // columns: 550 against 640 us for cubes and 585 for strips). Strips stay
-    // faster on large sparse meshes, whose passes are all staging (three
-    // workgroups per CU against two): with 8-point tiles, below 48 particles a
-    // block on a grid above 2048 (K = 192, 16 columns, 26 particles a block:
-    // 677 against 706 us).
+    // tile side and order: the larger the block the fewer its halo reads, up to
+    // 19 region points in a thread's prefetch registers and to the particles of
+    // a chunk. The lines, us of the stage (p = 6; more in
+    // profiles/launch_rules.txt):
+    // - flat (3, 2, 1) blocks of 8-point tiles in FP32 below 2.2 particles per
+    //   4^3 points, whose passes are shorter: K = 128, 8 columns, flat / cube at
+    //   1.6: 138 / 141, 2.4: 152 / 152, 3: 168 / 163. (On K = 216 flat stays
+    //   ahead up to 4: 2.4: 632 / 724, 5: 1125 / 1091.)
+    // - strips on large sparse meshes of 8-point tiles, whose passes are all
+    //   staging (three workgroups per CU against two): below 48 particles a
+    //   block on a grid above 2048. K = 192, 16 FP32 columns, strips / blocks at
+    //   24 particles a block: 674 / 704, 48: 722 / 732, 75: 813 / 773. (Not so
+    //   in FP64, K = 192, 8 columns, 16: 665 / 591, nor on K = 216, 36: 1058 /
+    //   1005, which the line sends to strips too.)
     const SpmeTuning& tn = tune[width_class(b)];
     const double dens = (double)npos / ((double)K * K * K);
     if (ts == 6) { sd[0] = 3; }
@@ -1792,8 +1802,13 @@ InterpPlan SpmeGpu<T>::interp_plan(int b) const {
                 (CH * (2 * porder + 1) + 3) / 4 * 4) * sizeof(T) +
                (size_t)CH * rb * 3 * (poly ? 8 : sizeof(T)) + CH * sizeof(int);
     };
-    // smaller blocks where the particles exceed a chunk and on small
-    // meshes, where the grid would leave CUs idle
+    // smaller blocks where the particles exceed a chunk: K = 64, 8 FP32
+    // columns, cubes of 0.85 chunks 39 us; of 1.0 chunks 51, blocks of half 36.
+    // And on small meshes, where the grid would leave CUs idle: at least 512
+    // workgroups. K = 64, 8 FP32 columns, at least 128: 39, 256: 38, 512: 32,
+    // 1024: 38 us; K = 48, 20: 40, 31, 31, 39. FP64 (one or two workgroups per
+    // CU) and single columns do better with fewer, one full round of the CUs:
+    // K = 64, 4 FP64: 41, 21, 27, 31; K = 96, 1 FP32: 21, 21, 24, 27.
     for (int d = 2; sd[0] > 1 || sd[1] > 1 || sd[2] > 1; d = (d + 2) % 3) {
         if (reg_of() <= 19u * kIbThreads && lds_b(1) <= 150 * 1024 &&
             particles() <= 0.9 * CH && blocks() * b >= 512)
