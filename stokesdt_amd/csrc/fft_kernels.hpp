@@ -484,10 +484,12 @@ fft2_y_kernel(cplx<T>* __restrict__ spec, const double* __restrict__ tw_g, int l
 // the budget (NC R2 complex values), the middle part is three steps through
 // LDS, spread over the components (K = 256 FP64 poly: 2.05 ms for 18 meshes
 // against 2.86 with one thread taking all components in turn). The line lies
-// below 192 registers of values: FP64 with unequal radii and R2 = 8 reaches them
-// and then runs one or two waves per SIMD. Its us for 20 columns, in registers /
-// three steps: K = 64: 123 / 95, 72: 164 / 136, 80: 354 / 186, 96: 844 / 368,
-// 128: 940 / 868.
+// below 192 registers of values, where kernels run one or two waves per SIMD. us
+// in registers / three steps: unequal radii, FP64 with R2 = 8, 20 columns, K =
+// 64: 123 / 95, 72: 164 / 136, 80: 354 / 186, 96: 844 / 368, 128: 940 / 868; FP32
+// with R2 = 16, 8 columns, K = 256: 3286 / 2877, 288: 3549 / 2625; equal radii,
+// FP64 with R2 = 16, 8 columns, K = 256: 2275 / 2230, 288: 2290 / 2222, 320: 2971 /
+// 2965.
 // 256 threads where the middle is in registers: K = 128 FP32, 100 columns
 // 1.15 ms against 1.56 with 384 (two workgroups fit then, and more waves
 // wait at each barrier). Chunks in XCD order: 1.15 against 1.18 ms, FP64 2.20

@@ -2,7 +2,7 @@
 kernels differ: the smallest two-stage sides, odd radices, the largest fused
 planes, the separate x and y passes on both sides of that line (FP32 192 / 200,
 FP64 128 / 144), the components' three-step z pass (unequal radii in FP64 from a
-second radix of 8 up: 64, 72, 80, 90, ...; 54 and 60 below), and the general radix chain (250, 360).
+second radix of 8 up: 64, 72, 80, 90, ...; 54 and 60 below; 256 in FP64), and the general radix chain (250, 360).
 
 FP64 against the oracle's reciprocal product: the sums of a product of
 K^3 log K^3 operations in 64 bits, 1e-12 of the result (measured 2e-15); FP32
@@ -19,7 +19,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("K,p,poly", [
     (16, 4, False), (20, 4, True), (24, 6, False), (30, 6, True), (50, 6, False), (54, 6, True),
     (60, 6, True), (64, 6, True), (80, 6, True), (96, 6, True), (90, 6, True), (100, 6, False), (128, 6, True), (144, 6, False), (162, 6, True),
-    (180, 6, False), (192, 8, False), (200, 8, False), (240, 6, True), (250, 6, False),
+    (180, 6, False), (192, 8, False), (200, 8, False), (240, 6, True), (250, 6, False), (256, 8, False),
     (324, 6, False), (360, 6, False),
 ])
 def test_recip_matches_oracle_at_every_kind_of_side(sdt, orc, K, p, poly):
